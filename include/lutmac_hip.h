@@ -182,8 +182,8 @@ int lmx_extract_indices(const uint8_t *sign_plane, const uint8_t *zero_plane,
  * buffers: tiles in the lmx_tile_planes layout (16-byte aligned), scales in
  * the lmx_tile_scales layout; format, rows, cols, group, x, y, batch, flags
  * and stream mean what they mean for lmx_gemv, with the same kernel plan, so
- * y is bit-identical to lmx_gemv's (batches run one vector at a time).  It
- * allocates nothing: the split-K partials, ticket counters and the staging
+ * y is bit-identical to lmx_gemv's for up to 4 vectors (larger batches run in
+ * groups of 4).  It allocates nothing: the split-K partials, ticket counters and the staging
  * copy of x live in an 8 MiB device array that each GPU holds until the
  * process ends: a fixed 64 KiB of split-K ticket counters (one per 64-row
  * block), then the staging copy of x (Kp*4 B), then the split-K partials

@@ -25,6 +25,11 @@ DEVICE = ["-x", "hip", f"--offload-arch={ARCH}",
 
 SOURCES = [
     ("lmx_kernels.hip", True),
+    ("lmx_digit.hip", True),
+] + [
+    # the digit kernels, one translation unit per weight format
+    (f"lmx_digit_fmt.hip:LMX_DIGIT_FMT={f}", True) for f in range(1, 8)
+] + [
     ("lmx_probe.hip", True),
     ("lmx_noalloc.hip", True),
     ("lmx_decode.hip", True),
@@ -50,11 +55,12 @@ def build(verbose=True):
     os.makedirs(OUT_DIR, exist_ok=True)
     jobs = []
     for src, device in SOURCES:
-        path = os.path.join(CSRC, src)
+        name, _, define = src.partition(":")
+        path = os.path.join(CSRC, name)
         if not os.path.exists(path):
             continue
-        obj = os.path.join(OUT_DIR, src + ".o")
-        flags = COMMON + (DEVICE if device else ["-D__HIP_PLATFORM_AMD__"])
+        obj = os.path.join(OUT_DIR, src.replace(":", ".") + ".o")
+        flags = COMMON + (DEVICE if device else ["-D__HIP_PLATFORM_AMD__"]) + ([f"-D{define}"] if define else [])
         jobs.append(([HIPCC] + flags + ["-c", path, "-o", obj], obj))
     workers = max(1, min(len(jobs), int(os.environ.get("MAX_JOBS", "8"))))
     with ThreadPoolExecutor(workers) as pool:

@@ -166,18 +166,18 @@ void plan_weight(lmx_weight *w, int fmt, size_t rows, size_t cols, size_t group)
   w->fullk = choose_fullk(fmt, w->Npad, w->Kp, w->kfamily);
   w->staged = choose_staged();
   w->batched = env_int("LMX_BATCHED", 1) != 0;
+  // The digit kernels, unless a lookup-table plan was asked for.
+  w->digit = env_int("LMX_DIGIT", 1) != 0;
+  for (const char *name : {"LMX_FULLK", "LMX_KERNEL", "LMX_KSLICE", "LMX_REDUCE", "LMX_WAVES"})
+    if (std::getenv(name)) w->digit = false;
 }
 
 namespace {
 
 void free_weight(lmx_weight *w) {
   if (!w) return;
-  if (w->d_planes) (void)hipFree(w->d_planes);
-  if (w->d_scales) (void)hipFree(w->d_scales);
-  if (w->d_partials) (void)hipFree(w->d_partials);
-  if (w->d_counters) (void)hipFree(w->d_counters);
-  if (w->d_xrot) (void)hipFree(w->d_xrot);
-  if (w->d_bpartials) (void)hipFree(w->d_bpartials);
+  if (w->d_weight) (void)hipFree(w->d_weight);
+  if (w->d_scratch) (void)hipFree(w->d_scratch);
   if (w->d_nib) (void)hipFree(w->d_nib);
   delete w;
 }
@@ -211,28 +211,45 @@ int upload(int fmt, size_t rows, size_t cols, size_t group, const uint8_t *plane
       for (size_t g = 0; g < ng_src && g < w->n_groups; ++g)
         sc[(size_t(s) * w->n_groups + g) * w->Npad + r] = scales[(size_t(s) * rows + r) * ng_src + g];
 
-  const size_t row_blocks = w->Npad / kWave;  // enough counters for any waves-per-group choice
-  const size_t max_splits = w->Kp / kRotChunk;
+  // Two allocations a handle: the weight (planes, code copy, scales) and the
+  // scratch of its calls, allocated here so that no call allocates (graph
+  // capture stays possible).
+  const auto align = [](size_t n) { return round_up(n, 256); };
+  const size_t code_bytes = w->digit ? code_copy_bytes(fmt, w->Npad, w->Kp) : 0;
+  // enough counters for any waves-per-group choice and any sliced rows launch
+  const size_t counter_bytes = std::max<size_t>(w->Npad / kWave, kDigitTickets) * sizeof(unsigned);
+  // split-K partials of one vector; with batches those of the largest group
+  // (16; 128-wide k-slices, twice the splits, where 256-wide ones give the
+  // batched kernel less than a workgroup per CU), and the digits of 256
+  // vectors (512 of a long K, where two launches cost most), more where the
+  // matrix has the rows to make one launch of them worth it.  One call uses
+  // one of them at a time.
+  size_t work_bytes = w->Kp / kRotChunk * w->Npad * sizeof(float);
+  if (w->batched) {
+    const size_t vectors = std::min<size_t>(std::max<size_t>(w->Npad / 16, w->Kp > 4096 ? 512 : 256), 1024);
+    work_bytes = std::max(16 * batched_slice_splits(w->Npad, w->Kp) * w->Npad * sizeof(float),
+                          digit_bytes(w->Kp, vectors) + kDigitPartials);
+  }
+  char *base = nullptr;
   hipError_t e;
-  if ((e = hipMalloc(&w->d_planes, w->tile_bytes)) != hipSuccess ||
-      (e = hipMalloc(reinterpret_cast<void **>(&w->d_scales), w->scale_bytes)) != hipSuccess ||
-      (e = hipMalloc(reinterpret_cast<void **>(&w->d_partials), max_splits * w->Npad * sizeof(float))) != hipSuccess ||
-      (e = hipMalloc(reinterpret_cast<void **>(&w->d_counters), row_blocks * sizeof(unsigned))) != hipSuccess ||
-      (e = hipMalloc(reinterpret_cast<void **>(&w->d_xrot), w->Kp * sizeof(float))) != hipSuccess) {
+  if ((e = hipMalloc(&w->d_weight, align(w->tile_bytes) + align(code_bytes) + w->scale_bytes)) != hipSuccess ||
+      (e = hipMalloc(&w->d_scratch, align(counter_bytes) + align(w->Kp * sizeof(float)) + work_bytes)) != hipSuccess) {
     free_weight(w);
     return hip_fail(e, "hipMalloc (weight)");
   }
-  // Batched partials for the largest vector group (16), allocated with the
-  // handle so that no GEMV call allocates (graph capture stays possible).
+  base = static_cast<char *>(w->d_weight);
+  w->d_planes = base;
+  if (code_bytes) w->d_codes = base + align(w->tile_bytes);
+  w->d_scales = reinterpret_cast<float *>(base + align(w->tile_bytes) + align(code_bytes));
+  base = static_cast<char *>(w->d_scratch);
+  w->d_counters = reinterpret_cast<unsigned *>(base);
+  w->d_xrot = reinterpret_cast<float *>(base + align(counter_bytes));
+  w->d_partials = reinterpret_cast<float *>(base + align(counter_bytes) + align(w->Kp * sizeof(float)));
   if (w->batched) {
-    // 128-wide k-slices (twice the splits) where 256-wide ones give the
-    // batched kernel less than a workgroup per CU (batched_slice_splits)
-    const size_t n = 16 * batched_slice_splits(w->Npad, w->Kp) * w->Npad;
-    if ((e = hipMalloc(reinterpret_cast<void **>(&w->d_bpartials), n * sizeof(float))) != hipSuccess) {
-      free_weight(w);
-      return hip_fail(e, "hipMalloc (batched partials)");
-    }
-    w->bpartials_cap = n;
+    w->d_bpartials = w->d_partials;
+    w->bpartials_cap = work_bytes / sizeof(float);
+    w->d_digits = w->d_partials;
+    w->digit_cap = work_bytes;
     // 4-bit: the codes once more in the matrix-core kernel's layout (groups
     // of 4, 8 and 16 vectors; the same 4 bits per weight as the planes)
     if (fmt == LMX_FMT_INT4 && mfma_batched()) {
@@ -251,9 +268,16 @@ int upload(int fmt, size_t rows, size_t cols, size_t group, const uint8_t *plane
       }
     }
   }
-  if ((e = hipMemcpy(w->d_planes, tiles.data(), w->tile_bytes, hipMemcpyHostToDevice)) != hipSuccess ||
-      (e = hipMemcpy(w->d_scales, sc.data(), w->scale_bytes, hipMemcpyHostToDevice)) != hipSuccess ||
-      (e = hipMemset(w->d_counters, 0, row_blocks * sizeof(unsigned))) != hipSuccess ||
+  if ((e = hipMemcpy(w->d_planes, tiles.data(), w->tile_bytes, hipMemcpyHostToDevice)) != hipSuccess) {
+    free_weight(w);
+    return hip_fail(e, "upload (weight)");
+  }
+  if (code_bytes && (st = launch_code_copy(fmt, w->d_planes, w->Npad, w->Kp, w->d_codes, nullptr))) {
+    free_weight(w);
+    return st;
+  }
+  if ((e = hipMemcpy(w->d_scales, sc.data(), w->scale_bytes, hipMemcpyHostToDevice)) != hipSuccess ||
+      (e = hipMemset(w->d_counters, 0, counter_bytes)) != hipSuccess ||
       (e = hipDeviceSynchronize()) != hipSuccess) {
     free_weight(w);
     return hip_fail(e, "upload (weight)");
@@ -331,6 +355,43 @@ int gemv_batched(const lmx_weight *w, GemvArgs a, const float *x, float *y, size
   return LMX_OK;
 }
 
+// y = W x of `batch` vectors on the digit kernels: up to 4 in one launch,
+// more through digits split into the handle's scratch.  One vector of a 1-3
+// bit format stays on the lookup tables, whose planes are half to an eighth of
+// the bytes while the digits cost the same (8192 x 8192, us: ternary 6.5
+// against 8.2, RRQ-2 7.1 / 9.5, binary 5.3 / 7.1; 4-bit 9.7 / 8.0, 8-bit
+// 17.9 / 15.7).  *done = the vectors covered.
+int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done) {
+  const float *resid = a.resid;
+  const bool copies = code_copy_bytes(w->format, 1, kRotChunk) != 0;
+  // (the split kernels read the code copy where the format has one)
+  const size_t cap = w->d_digits && (!copies || w->d_codes) ? digit_capacity(w->Kp, w->digit_cap) : 0;
+  a.cols = int(w->cols);
+  for (*done = 0; *done < batch;) {
+    const size_t left = batch - *done;
+    a.x = x + *done * w->cols;
+    a.y = y + *done * w->rows;
+    a.resid = resid ? resid + *done * w->rows : nullptr;
+    size_t n = std::min<size_t>(left, 4);
+    int st;
+    // One launch for up to 4 vectors makes their digits once per row block:
+    // past 16 256-chunks that costs more than a launch of its own, unless the
+    // codes themselves are most of the work (2048 x 8192, 4 vectors, us:
+    // ternary 11.4 against 9.4 split, 4-bit 8.0 / 9.1).
+    if (cap && (left > 4 || (left > 1 && !copies && w->Kp > 4096))) {
+      n = std::min(left, cap);
+      const DigitVectors d = digit_vectors(w, w->d_digits, n);
+      if ((st = launch_digit_split(w->format, a, d, stream)) || (st = launch_digit_gemm(w->format, a, d, stream)))
+        return st;
+    } else {
+      if (!copies && (left == 1 || w->Kp > 4096)) return LMX_OK;   // one by one on the lookup tables
+      if ((st = launch_digit_gemv(w->format, a, int(n), stream))) return st;
+    }
+    *done += n;
+  }
+  return LMX_OK;
+}
+
 bool batched_epilogue_ok(const lmx_weight *w, int epi, size_t batch) {
   if (!w->batched || batch < 4 || batch % 4 || w->cols % 4) return false;   // every vector in a group of 16/8/4
   if (epi == kEpiSiluPair) return w->rows % 8 == 0;
@@ -342,6 +403,7 @@ bool batched_epilogue_ok(const lmx_weight *w, int epi, size_t batch) {
 GemvArgs weight_args(const lmx_weight *w) {
   GemvArgs a{};
   a.planes = w->d_planes;
+  a.codes = w->d_codes;
   a.scales = w->d_scales;
   a.partials = w->d_partials;
   a.counters = w->d_counters;
@@ -589,7 +651,8 @@ int gemv_impl(const lmx_weight *w, const float *x, float *y, size_t batch, unsig
   size_t b0 = 0;
   if (flags != LMX_ROTATE_FWHT_FULL) {
     a.rotate = flags == LMX_ROTATE_FWHT256 ? LMX_ROTATE_FWHT256 : LMX_ROTATE_NONE;
-    if ((st = gemv_batched(w, a, x, y, batch, stream, &b0))) return st;
+    if ((st = w->digit ? digit_linear(w, a, x, y, batch, stream, &b0) : gemv_batched(w, a, x, y, batch, stream, &b0)))
+      return st;
   }
   for (size_t b = b0; b < batch; ++b) {
     a.x = x + b * w->cols;
@@ -624,7 +687,8 @@ int lmx_linear(const lmx_weight *w, const float *bias, const float *x, float *y,
   a.bias = bias;
   a.rotate = rotate ? LMX_ROTATE_FWHT256 : LMX_ROTATE_NONE;
   size_t b0 = 0;
-  if ((st = gemv_batched(w, a, x, y, batch, stream, &b0))) return st;
+  if ((st = w->digit ? digit_linear(w, a, x, y, batch, stream, &b0) : gemv_batched(w, a, x, y, batch, stream, &b0)))
+    return st;
   for (size_t b = b0; b < batch; ++b) {
     a.x = x + b * w->cols;
     a.y = y + b * w->rows;

@@ -1,0 +1,255 @@
+// lmx_digit.hip -- activations split into digits once for many vectors, and
+// the dispatch of the digit kernels over the weight formats.
+#include "lmx_digit_kernels.hpp"
+
+namespace lmx {
+
+// lmx_digit_fmt.hip, one translation unit per format
+template <int FMT> int digit_gemv_fmt(const GemvArgs &a, int nv, void *stream);
+template <int FMT> int digit_gemm_fmt(const GemvArgs &a, const DigitVectors &d, void *stream);
+template <int FMT> int code_copy_fmt(const void *planes, size_t Npad, size_t Kp, void *codes, void *stream);
+
+namespace {
+
+// ---------------------------------------------------------------------------
+// Digits of many vectors relative to each vector, one workgroup per vector (tile form): dig[quad][chunk][step][lane][16 B].
+template <bool ROT, int XM>
+__global__ __launch_bounds__(512) void digit_split_kernel(const float *__restrict__ x, int cols, int Kp,
+                                                          const float *__restrict__ xw, float eps, float factor,
+                                                          char *__restrict__ dig, float *__restrict__ vfac,
+                                                          int *__restrict__ vexp) {
+  constexpr int NW = 8;
+  __shared__ uint32_t mx[NW];
+  __shared__ float ssw[NW];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int v = blockIdx.x;
+  const DigitLane dl(lane);
+  const int pairs = Kp / kRotChunk;
+  x += size_t(v) * cols;
+  float ss = 0.0f;
+  const auto values = [&](int c2, float (&o)[4]) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int k = c2 * kRotChunk + dl.k(b), kc = min(k, cols - 1);
+      float t = x[kc];
+      if constexpr (XM == kXModeRmsNorm) {
+        t = k < cols ? t : 0.0f;
+        ss = fmaf(t, t, ss);
+        t *= xw[kc];
+      }
+      o[b] = k < cols ? t : 0.0f;
+    }
+    if constexpr (ROT) fwht256_regs_x16(o[0], o[1], o[2], o[3], lane);
+  };
+  constexpr int KEEP = 4;   // 256-chunks of a wave kept between the passes (K <= 8192)
+  float keep[KEEP][4];
+  uint32_t m = 0;
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j) {
+    if (wave + j * NW < pairs) {
+      values(wave + j * NW, keep[j]);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) m = max(m, __float_as_uint(keep[j][b]) & 0x7FFFFFFFu);
+    }
+  }
+  for (int c2 = wave + KEEP * NW; c2 < pairs; c2 += NW) {
+    float o[4];
+    values(c2, o);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) m = max(m, __float_as_uint(o[b]) & 0x7FFFFFFFu);
+  }
+  m = row_max(m);
+  m = max(m, lane_xor_u32<16>(m, lane));
+  m = max(m, lane_xor_u32<32>(m, lane));
+  if constexpr (XM == kXModeRmsNorm) ss = lane_sum<32>(ss, lane);
+  if (lane == 0) {
+    mx[wave] = m;
+    ssw[wave] = ss;
+  }
+  __syncthreads();
+  float sum = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    m = max(m, mx[i]);
+    sum += ssw[i];
+  }
+  const int e = split_exponent(m);
+  if (threadIdx.x == 0) {
+    float f = factor;
+    if constexpr (XM == kXModeRmsNorm) f *= 1.0f / sqrtf(sum / float(cols) + eps);
+    vfac[v] = m >= kNotFinite ? __builtin_nanf("") : f;
+    vexp[v] = e - 156;
+  }
+  const int t = 7 - dl.kl;
+  char *base = dig + size_t(v >> 2) * (size_t(Kp / kChunk) * kQuadChunk) + (t >> 2) * 1024 +
+               (dl.kq * 16 + (v & 3) * 4) * 16 + (t & 3) * 4;
+  const auto emit = [&](int c2, const float (&o)[4]) {
+    uint32_t dg[4];
+    digits4(o, e, dg);
+    char *dst = base + size_t(2 * c2 + dl.c) * kQuadChunk;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t *>(dst + q * 16) = dg[q];
+  };
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j)
+    if (wave + j * NW < pairs) emit(wave + j * NW, keep[j]);
+  for (int c2 = wave + KEEP * NW; c2 < pairs; c2 += NW) {
+    float o[4];
+    values(c2, o);
+    emit(c2, o);
+  }
+}
+
+// Digits relative to each 128-chunk (rows form): one wave per vector and
+// 256-chunk, so that a few long vectors spread over the chip.  RMSNorm: every
+// workgroup of a vector sums its squares over the whole row.
+template <int XM>
+__global__ __launch_bounds__(256) void digit_split_chunks_kernel(const float *__restrict__ x, int cols, int Kp,
+                                                                 const float *__restrict__ xw, float eps, float factor,
+                                                                 unsigned rotate, DigitVectors d) {
+  constexpr int NW = 4;
+  __shared__ float ssw[NW];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+  const int v = int(blockIdx.y), c2 = int(blockIdx.x) * NW + wave;
+  const DigitLane dl(lane);
+  x += size_t(v) * cols;
+  float o[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int k = c2 * kRotChunk + dl.k(b);
+    const uint32_t kc = uint32_t(min(k, cols - 1));
+    float t = x[kc];
+    if constexpr (XM == kXModeRmsNorm) t *= xw[kc];
+    o[b] = k < cols ? t : 0.0f;
+  }
+  if (blockIdx.x == 0) {   // the vector's factor
+    float f = factor;
+    if constexpr (XM == kXModeRmsNorm) {
+      float ss = 0.0f;
+      for (int k = threadIdx.x; k < cols; k += 256) ss = fmaf(x[k], x[k], ss);
+      ss = lane_sum<32>(ss, lane);
+      if (lane == 0) ssw[wave] = ss;
+      __syncthreads();
+      f *= 1.0f / sqrtf(((ssw[0] + ssw[1]) + (ssw[2] + ssw[3])) / float(cols) + eps);
+    }
+    if (threadIdx.x == 0) d.fac[v] = f;
+  }
+  if (c2 * kRotChunk >= Kp) return;   // wave-uniform; no barrier follows
+  if (rotate == LMX_ROTATE_FWHT256) fwht256_regs_x16(o[0], o[1], o[2], o[3], lane);
+  const uint32_t mb = chunk_max_bits(o);
+  const int e = split_exponent(mb);
+  uint32_t dg[4];
+  digits4(o, e, dg);
+  const int t = 7 - dl.kl;
+  const size_t qc = size_t(v >> 2) * size_t(Kp / kChunk) + size_t(2 * c2 + dl.c);
+  char *dst = d.digits + qc * kQuadChunk + (t >> 2) * 1024 + (dl.kq * 16 + (v & 3) * 4) * 16 + (t & 3) * 4;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t *>(dst + q * 16) = dg[q];
+  if ((lane & 31) == 0)
+    d.mult[qc * 4 + (v & 3)] = mb >= kNotFinite ? __builtin_nanf("") : __builtin_amdgcn_ldexpf(1.0f, e - 156);
+}
+
+}  // namespace
+
+// Two row tiles per workgroup once that leaves a workgroup per CU: each makes
+// the digits of the whole K (4-bit, us, one tile against two: 2048 x 2048
+// 3.18 / 3.44, 3072 x 2048 3.35 / 3.56, 17920 x 1536 5.54 / 5.27, 8192 x 8192
+// 12.0 / 8.0).
+int digit_gemv_tiles(const GemvArgs &a) { return a.epi == kEpiSiluPair || a.Npad / kTile >= 512 ? 2 : 1; }
+
+int launch_digit_gemv(int fmt, const GemvArgs &a, int nv, void *stream) {
+  switch (fmt) {
+  case LMX_FMT_TERNARY: return digit_gemv_fmt<LMX_FMT_TERNARY>(a, nv, stream);
+  case LMX_FMT_BINARY: return digit_gemv_fmt<LMX_FMT_BINARY>(a, nv, stream);
+  case LMX_FMT_RRQ2: return digit_gemv_fmt<LMX_FMT_RRQ2>(a, nv, stream);
+  case LMX_FMT_RRQ3: return digit_gemv_fmt<LMX_FMT_RRQ3>(a, nv, stream);
+  case LMX_FMT_INT3: return digit_gemv_fmt<LMX_FMT_INT3>(a, nv, stream);
+  case LMX_FMT_INT4: return digit_gemv_fmt<LMX_FMT_INT4>(a, nv, stream);
+  case LMX_FMT_INT8: return digit_gemv_fmt<LMX_FMT_INT8>(a, nv, stream);
+  }
+  return fail(LMX_ERR_UNSUPPORTED_FORMAT, "unknown format %d", fmt);
+}
+
+static float code_factor(int fmt, unsigned rotate) {
+  int sh = 6;
+  if (fmt == LMX_FMT_INT4) sh = 4;
+  if (fmt == LMX_FMT_INT3) sh = 5;
+  if (fmt == LMX_FMT_INT8) sh = 0;
+  return (rotate == LMX_ROTATE_FWHT256 ? 0.0625f : 1.0f) / float(1 << sh);
+}
+
+// digits, mult (rows form), fac and exp of `vectors` vectors
+size_t digit_bytes(size_t Kp, size_t vectors) {
+  const size_t quads = (vectors + 3) / 4;
+  return quads * (Kp / kChunk) * (kQuadChunk + 16) + quads * 32;
+}
+
+size_t digit_capacity(size_t Kp, size_t bytes) {
+  return bytes > kDigitPartials ? (bytes - kDigitPartials) / digit_bytes(Kp, 4) * 4 : 0;
+}
+
+DigitVectors digit_vectors(const lmx_weight *w, void *scratch, size_t count) {
+  DigitVectors d{};
+  const size_t quads = (count + 3) / 4, chunks = w->Kp / kChunk;
+  d.digits = static_cast<char *>(scratch);
+  d.mult = reinterpret_cast<float *>(d.digits + quads * chunks * kQuadChunk);
+  d.fac = d.mult + quads * chunks * 4;
+  d.exp = reinterpret_cast<int *>(d.fac + quads * 4);
+  d.partials = reinterpret_cast<float *>(d.exp + quads * 4);
+  d.count = int(count);
+  // The tile kernel where it has most of a workgroup per CU (2048 columns,
+  // us: 192 workgroups 21 against 25, 128 workgroups 20 / 18).
+  d.tile = (w->Npad / kTile + 7) / 8 * ((quads + 7) / 8) >= 192;
+  return d;
+}
+
+int launch_digit_split(int fmt, const GemvArgs &a, const DigitVectors &d, void *stream) {
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const float f = code_factor(fmt, a.rotate);
+  const bool rot = a.rotate == LMX_ROTATE_FWHT256;
+  if (!d.tile) {
+    const dim3 grid{unsigned((a.Kp / kRotChunk + 3) / 4), unsigned(d.count)};
+    if (a.xmode == kXModeRmsNorm)
+      digit_split_chunks_kernel<kXModeRmsNorm><<<grid, dim3(256), 0, st>>>(a.x, a.cols, a.Kp, a.xw, a.eps, f, a.rotate, d);
+    else
+      digit_split_chunks_kernel<kXModeNone><<<grid, dim3(256), 0, st>>>(a.x, a.cols, a.Kp, a.xw, a.eps, f, a.rotate, d);
+    return launched("digit_split_chunks");
+  }
+#define LMX_SP(R, XM) \
+  digit_split_kernel<R, XM><<<dim3(unsigned(d.count)), dim3(512), 0, st>>>(a.x, a.cols, a.Kp, a.xw, a.eps, f, d.digits, d.fac, d.exp)
+  if (a.xmode == kXModeRmsNorm) {
+    if (rot) LMX_SP(true, kXModeRmsNorm); else LMX_SP(false, kXModeRmsNorm);
+  } else {
+    if (rot) LMX_SP(true, kXModeNone); else LMX_SP(false, kXModeNone);
+  }
+#undef LMX_SP
+  return launched("digit_split");
+}
+
+int launch_digit_gemm(int fmt, const GemvArgs &a, const DigitVectors &d, void *stream) {
+  if (code_copy_bytes(fmt, 1, kRotChunk) && !a.codes)
+    return fail(LMX_ERR_INVALID_ARGUMENT, "the split digit kernels need the code copy of format %d", fmt);
+  switch (fmt) {
+  case LMX_FMT_TERNARY: return digit_gemm_fmt<LMX_FMT_TERNARY>(a, d, stream);
+  case LMX_FMT_BINARY: return digit_gemm_fmt<LMX_FMT_BINARY>(a, d, stream);
+  case LMX_FMT_RRQ2: return digit_gemm_fmt<LMX_FMT_RRQ2>(a, d, stream);
+  case LMX_FMT_RRQ3: return digit_gemm_fmt<LMX_FMT_RRQ3>(a, d, stream);
+  case LMX_FMT_INT3: return digit_gemm_fmt<LMX_FMT_INT3>(a, d, stream);
+  case LMX_FMT_INT4: return digit_gemm_fmt<LMX_FMT_INT4>(a, d, stream);
+  case LMX_FMT_INT8: return digit_gemm_fmt<LMX_FMT_INT8>(a, d, stream);
+  }
+  return fail(LMX_ERR_UNSUPPORTED_FORMAT, "unknown format %d", fmt);
+}
+
+size_t code_copy_bytes(int fmt, size_t Npad, size_t Kp) {
+  return fmt == LMX_FMT_INT4 ? Npad * Kp / 2 : fmt == LMX_FMT_INT8 ? Npad * Kp : 0;
+}
+
+int launch_code_copy(int fmt, const void *planes, size_t Npad, size_t Kp, void *codes, void *stream) {
+  if (fmt == LMX_FMT_INT4) return code_copy_fmt<LMX_FMT_INT4>(planes, Npad, Kp, codes, stream);
+  if (fmt == LMX_FMT_INT8) return code_copy_fmt<LMX_FMT_INT8>(planes, Npad, Kp, codes, stream);
+  return LMX_OK;
+}
+
+}  // namespace lmx

@@ -1,0 +1,686 @@
+// lmx_digit_kernels.hpp -- GEMV and GEMM kernels on the 8-bit matrix cores
+// with exact products (lmx_digit.hpp: the digit split, layouts, identities),
+// included by the .hip sources only.
+//
+//   digit_gemv_kernel   1..4 vectors in one launch: every wave makes the
+//                       digits of its own 256-chunks in LDS and multiplies
+//                       them with its rows
+//   digit_rows_kernel   few split vectors or few rows: k over the waves of a
+//                       workgroup, fragments straight from the caches
+//   digit_tile_kernel   many split vectors and rows: fragments staged in LDS
+#ifndef LMX_DIGIT_KERNELS_HPP
+#define LMX_DIGIT_KERNELS_HPP
+
+#include <hip/hip_runtime.h>
+
+#include <cstdlib>
+
+#include "lmx_digit.hpp"
+
+namespace lmx {
+namespace {
+
+constexpr int kTile = 16;          // weight rows per matrix-core tile
+constexpr uint32_t kQuadChunk = 2048;   // digit bytes of a quad's 128-chunk
+
+__device__ __forceinline__ int scale_group(const GemvArgs &a, int ch) {
+  return a.gshift >= 0 ? ch >> a.gshift : ch / a.group_chunks;
+}
+
+// ---------------------------------------------------------------------------
+// 1..4 vectors, one launch: RT row tiles per workgroup, the whole K over its
+// waves (wave w takes the 256-chunks w, w + W, ... , PPW of them a round).
+// NV = 1: the fragment rows of the other three vectors of a quad hold other
+// 128-chunks' digits instead (chunk q of a group of four in rows 4 q .. 4 q +
+// 3, zeros elsewhere), so four chunks' digit sums land in four lane groups of
+// one accumulator and are joined and scaled once.
+// NV = 4: one accumulator per chunk, its four lane groups the four vectors.
+template <int FMT, bool COPY, int NV, int RT, int PPW, int XM, int EPI>
+__global__ __launch_bounds__(1024) void digit_gemv_kernel(GemvArgs a, int nv) {
+  constexpr int CW = Source<FMT, COPY>::CW, S = Fmt<FMT>::S;
+  constexpr int ROWS = 4 * NV;                     // fragment rows kept
+  // a fragment, 16 bytes longer: the digit writes of the steps and chunks of
+  // a 256-chunk (4 lanes each of 16 bytes in 64) start in different banks
+  constexpr uint32_t FRAG = 4 * ROWS * 16 + (NV == 1 ? 16 : 0);
+  constexpr bool PAIR = EPI == kEpiSiluPair;
+  constexpr bool NORM = XM == kXModeRmsNorm;
+  constexpr int CH = 2 * PPW;                      // 128-chunks of a wave's round
+  constexpr int G = NV == 1 ? 4 : 1;               // chunks per accumulator
+  constexpr int NG = (CH + G - 1) / G;
+  constexpr int OUT = PAIR ? RT / 2 * kTile : RT * kTile;   // outputs per vector
+  __shared__ __attribute__((aligned(16))) char frags[16][CH][2][FRAG];   // [wave][chunk][step]
+  __shared__ __attribute__((aligned(16))) uint32_t zeros[4];
+  __shared__ float mults[16][CH][NV];
+  __shared__ float red[16][RT * kTile * NV];
+  __shared__ float ssq[16][NV];
+
+  const int lane = threadIdx.x & (kWave - 1), W = blockDim.x / kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+  const int li = lane & 15, kq = lane >> 4;
+  const int pairs = a.Kp / kRotChunk;
+  const bool rot = a.rotate == LMX_ROTATE_FWHT256;
+  const DigitLane dl(lane);
+
+  // first row of each tile; PAIR: RT/2 tiles of gate rows, then the matching up rows
+  uint32_t row0[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    if constexpr (PAIR)
+      row0[t] = uint32_t((t < RT / 2 ? 0 : a.rows / 2) + (int(blockIdx.x) * (RT / 2) + t % (RT / 2)) * kTile);
+    else
+      row0[t] = uint32_t((int(blockIdx.x) * RT + t) * kTile);
+  }
+  if (NV == 1 && threadIdx.x < 4) zeros[threadIdx.x] = 0u;
+
+  float acc[RT], ss[NV];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) acc[t] = 0.0f;
+#pragma unroll
+  for (int n = 0; n < NV; ++n) ss[n] = 0.0f;
+  float eb0 = 0.0f, eb1 = 0.0f;   // the epilogue thread's bias and residual terms, requested early
+  const int on = int(threadIdx.x) / OUT, orow = int(blockIdx.x) * OUT + int(threadIdx.x) % OUT;
+  const bool stores = on < nv && on < NV && orow < (PAIR ? a.rows / 2 : a.rows);
+
+  for (int p0 = wave; p0 < pairs; p0 += PPW * W) {
+    // ---- the round's activations, then its weights and scales (indices clamped, masked below) ----
+    float xr[PPW][NV][4], xw[PPW][4];
+#pragma unroll
+    for (int p = 0; p < PPW; ++p) {
+      const int c2 = min(p0 + p * W, pairs - 1);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const uint32_t k = uint32_t(min(c2 * kRotChunk + dl.k(b), a.cols - 1));
+#pragma unroll
+        for (int n = 0; n < NV; ++n) xr[p][n][b] = (a.x + size_t(min(n, nv - 1)) * a.cols)[k];
+        if constexpr (NORM) xw[p][b] = a.xw[k];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // every wave's activation requests ahead of the weight stream (and the
+    // zeros written): the barrier waits for no load
+    if (p0 == wave) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+      __builtin_amdgcn_s_barrier();
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t w[PPW][2][RT][CW];
+    float sc[G == 4 ? NG : CH][RT][S];
+    const auto load_w = [&](int p) {
+      const int c2 = min(p0 + p * W, pairs - 1);
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+          load_codes<FMT, COPY, true>(a, uint32_t(2 * c2 + c), row0[t], uint32_t(li), uint32_t(kq), w[p][c][t]);
+    };
+    const auto load_s = [&](int i) {
+      // G = 4: lane group kq takes chunk 4 i + kq of the round; else chunk i
+      const int q = G == 4 ? 4 * i + kq : i;
+      const int c2 = min(p0 + (q >> 1) * W, pairs - 1);
+      const uint32_t g = uint32_t(scale_group(a, 2 * c2 + (q & 1)));
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int s = 0; s < S; ++s) sc[i][t][s] = (a.scales + row0[t])[uint32_t(s * a.n_groups + g) * uint32_t(a.Npad) + uint32_t(li)];
+    };
+#pragma unroll
+    for (int p = 0; p < PPW; ++p) {
+      load_w(p);
+      if constexpr (G == 4) {
+        if (p % 2 == 0) load_s(p / 2);
+      } else {
+        load_s(2 * p);
+        load_s(2 * p + 1);
+      }
+    }
+    if (p0 == wave && stores) {
+      if (a.bias) {
+        eb0 = a.bias[orow];
+        if constexpr (PAIR) eb1 = a.bias[a.rows / 2 + orow];
+      }
+      if constexpr (!PAIR)
+        if (a.resid) eb1 = a.resid[size_t(on) * a.rows + orow];   // read before this thread stores y (resid may be y)
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- digits of the wave's 256-chunks ----
+#pragma unroll
+    for (int p = 0; p < PPW; ++p) {
+      const int c2 = p0 + p * W;
+      const bool live = c2 < pairs;   // else zeros: the chunk adds nothing
+      const bool full = c2 * kRotChunk + kRotChunk <= a.cols;
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        float x[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          x[b] = xr[p][n][b];
+          if (!full) x[b] = live && c2 * kRotChunk + dl.k(b) < a.cols ? x[b] : 0.0f;   // wave-uniform branch
+          if constexpr (NORM) {
+            ss[n] = fmaf(x[b], x[b], ss[n]);
+            x[b] *= xw[p][b];
+          }
+        }
+        if (rot) fwht256_regs_x16(x[0], x[1], x[2], x[3], lane);
+        const uint32_t mb = chunk_max_bits(x);
+        const int e = split_exponent(mb);
+        uint32_t dg[4];
+        digits4(x, e, dg);
+        const int t = 7 - dl.kl;
+        char *dst = frags[wave][2 * p + dl.c][t >> 2] + (dl.kq * ROWS + 4 * n) * 16 + (t & 3) * 4;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t *>(dst + q * 16) = dg[q];
+        if ((lane & 31) == 0)
+          mults[wave][2 * p + dl.c][n] = mb >= kNotFinite ? __builtin_nanf("") : __builtin_amdgcn_ldexpf(1.0f, e - 156);
+      }
+    }
+    // a wave reads only the digits it wrote; its LDS operations complete in order
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+
+    // ---- products ----
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+      v4i sum[RT][S];
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int s = 0; s < S; ++s) sum[t][s] = v4i{0, 0, 0, 0};
+#pragma unroll
+      for (int q = 0; q < G; ++q) {
+        const int ch = G * i + q;
+        if (ch >= CH) break;
+        v4i f[2];
+        if constexpr (G == 4) {
+          const char *src = frags[wave][ch][0] + (kq * ROWS + (li & 3)) * 16;
+          const bool mine = (li >> 2) == q;
+#pragma unroll
+          for (int m = 0; m < 2; ++m)
+            f[m] = *reinterpret_cast<const v4i *>(mine ? src + m * FRAG : reinterpret_cast<const char *>(zeros));
+        } else {
+#pragma unroll
+          for (int m = 0; m < 2; ++m)
+            f[m] = *reinterpret_cast<const v4i *>(frags[wave][ch][m] + (kq * ROWS + li) * 16);
+        }
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+          for (int s = 0; s < S; ++s) {
+            uint32_t wb[8];
+            source_bytes<FMT, COPY>(w[ch >> 1][ch & 1][t], s, wb);
+            sum[t][s] = chunk_product(wb, f[0], f[1], sum[t][s]);
+          }
+      }
+      // lane group kq: chunk 4 i + kq (G = 4) or vector kq of chunk i; a chunk past the round's adds 0
+      const float mult = G == 4 ? (4 * i + kq < CH ? mults[wave][min(4 * i + kq, CH - 1)][0] : 0.0f) : mults[wave][i][kq & (NV - 1)];
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int s = 0; s < S; ++s) acc[t] = fmaf(join_digits(sum[t][s]) * sc[i][t][s], mult, acc[t]);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+
+  // ---- the lane groups of a wave (NV = 1), then the waves in order ----
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const float v = NV == 1 ? strided_sum<kTile>(acc[t], lane) : acc[t];
+    if (kq < NV) red[wave][kq * RT * kTile + t * kTile + li] = v;
+  }
+  if constexpr (NORM) {
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      const float s = lane_sum<32>(ss[n], lane);
+      if (lane == 0) ssq[wave][n] = s;
+    }
+  }
+  __syncthreads();
+  float v = 0.0f;
+  if (stores) {
+    const int r = int(threadIdx.x) % OUT;
+    float scale = (rot ? 0.0625f : 1.0f) / float(1 << Code<FMT>::SH);
+    if constexpr (NORM) {
+      float s = 0.0f;
+      for (int k = 0; k < W; ++k) s += ssq[k][on];
+      scale *= 1.0f / sqrtf(s / float(a.cols) + a.eps);
+    }
+    const float *rd = red[0] + on * RT * kTile + r;
+    if constexpr (PAIR) {
+      float u = 0.0f;
+      for (int k = 0; k < W; ++k) {
+        v += rd[k * RT * kTile * NV];
+        u += rd[k * RT * kTile * NV + OUT];
+      }
+      a.y[size_t(on) * (a.rows / 2) + orow] = silu(fmaf(v, scale, eb0)) * fmaf(u, scale, eb1);
+    } else {
+      for (int k = 0; k < W; ++k) v += rd[k * RT * kTile * NV];
+      v *= scale;
+      if (a.bias) v += eb0;
+      if (a.resid) v += eb1;
+      a.y[size_t(on) * a.rows + orow] = v;
+    }
+  }
+  if constexpr (!PAIR) {
+    if (a.amax && threadIdx.x < kWave)   // one vector, at most 64 rows per workgroup
+      wave_argmax(a.amax, blockIdx.x, argmax_value(a, v, orow, stores), orow, stores);
+  }
+}
+
+// y = sum (times the vector's factor and exponent) (+ bias) (+ resid), or the
+// SiLU pair's product, of one output.
+__device__ __forceinline__ float vector_scale(float sum, float fac, int ex) {
+  return __builtin_amdgcn_ldexpf(sum * fac, ex);
+}
+
+// ---------------------------------------------------------------------------
+// NQ quads of vectors against RT row tiles: a workgroup takes one of gridDim.z
+// slices of the chunks, spread over its waves, fragments straight from memory
+// (each vector's digits are relative to its chunk: d.mult).  With more than
+// one slice the workgroups of a row block leave their sums in d.partials and
+// the last one to finish (a ticket) adds them in slice order: agent-scope
+// relaxed stores and loads, which need no write-back of the XCDs' L2s.
+template <int FMT, bool COPY, int NQ, int RT, int EPI>
+__global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVectors d) {
+  constexpr int CW = Source<FMT, COPY>::CW, S = Fmt<FMT>::S;
+  constexpr bool PAIR = EPI == kEpiSiluPair;
+  constexpr int SUMS = RT * NQ * kWave;
+  __shared__ float red[16][SUMS];
+  __shared__ unsigned ticket;
+  const int lane = threadIdx.x & (kWave - 1), W = blockDim.x / kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+  const int li = lane & 15, kq = lane >> 4;
+  const int Kc = a.Kp / kChunk;
+  const uint32_t Npad = uint32_t(a.Npad);
+  const int quads = (d.count + 3) / 4, q0 = int(blockIdx.y) * NQ;
+  const int slices = int(gridDim.z), slice = int(blockIdx.z);
+  const int ch0 = Kc * slice / slices, ch1 = Kc * (slice + 1) / slices;
+  uint32_t row0[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    if constexpr (PAIR)
+      row0[t] = uint32_t((t < RT / 2 ? 0 : a.rows / 2) + (int(blockIdx.x) * (RT / 2) + t % (RT / 2)) * kTile);
+    else
+      row0[t] = uint32_t((int(blockIdx.x) * RT + t) * kTile);
+  }
+  const size_t qbytes = size_t(Kc) * kQuadChunk;
+  uint32_t w[2][RT][CW];
+  float sc[2][RT][S], mu[2][NQ];
+  v4i f[2][NQ][2];
+  const auto load = [&](int b, int ch) {
+    const uint32_t g = uint32_t(scale_group(a, ch));
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      load_codes<FMT, COPY, false>(a, uint32_t(ch), row0[t], uint32_t(li), uint32_t(kq), w[b][t]);
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+        sc[b][t][s] = (a.scales + size_t(s * a.n_groups + g) * Npad + row0[t])[uint32_t(li)];
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int qq = min(q0 + q, quads - 1);
+      mu[b][q] = (d.mult + (size_t(qq) * Kc + ch) * 4)[uint32_t(kq)];
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+        f[b][q][m] = reinterpret_cast<const v4i *>(d.digits + size_t(qq) * qbytes + size_t(ch) * kQuadChunk + m * 1024)[lane];
+    }
+  };
+  float acc[RT][NQ];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) acc[t][q] = 0.0f;
+  const auto work = [&](int b) {
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        uint32_t wb[8];
+        source_bytes<FMT, COPY>(w[b][t], s, wb);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+          acc[t][q] = fmaf(join_digits(chunk_product(wb, f[b][q][0], f[b][q][1])) * sc[b][t][s], mu[b][q], acc[t][q]);
+      }
+  };
+  if (ch0 + wave < ch1) load(0, ch0 + wave);
+  for (int ch = ch0 + wave; ch < ch1; ch += 2 * W) {
+    if (ch + W < ch1) load(1, ch + W);
+    work(0);
+    if (ch + W >= ch1) break;
+    if (ch + 2 * W < ch1) load(0, ch + 2 * W);
+    work(1);
+  }
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) red[wave][(t * NQ + q) * kWave + lane] = acc[t][q];
+  __syncthreads();
+  const auto wg_sum = [&](int o) {
+    float v = 0.0f;
+    for (int k = 0; k < W; ++k) v += red[k][o];
+    return v;
+  };
+  const size_t blocks = size_t(gridDim.x) * gridDim.y, block = size_t(blockIdx.y) * gridDim.x + blockIdx.x;
+  if (slices > 1) {
+    float *part = d.partials + (size_t(slice) * blocks + block) * SUMS;
+    for (int o = threadIdx.x; o < SUMS; o += blockDim.x)
+      __hip_atomic_store(part + o, wg_sum(o), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (threadIdx.x == 0)
+      ticket = __hip_atomic_fetch_add(a.counters + block, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (ticket != unsigned(slices - 1)) return;   // uniform over the workgroup
+    if (threadIdx.x == 0) __hip_atomic_store(a.counters + block, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  const auto total = [&](int o) {
+    if (slices == 1) return wg_sum(o);
+    float v = 0.0f;
+    const float *part = d.partials + block * SUMS + o;
+    for (int s0 = 0; s0 < slices; s0 += 8) {   // 8 loads in flight, summed in order
+      float t[8];
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        t[s] = s0 + s < slices ? __hip_atomic_load(part + size_t(s0 + s) * blocks * SUMS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0f;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) v += t[s];
+    }
+    return v;
+  };
+  // output o: (tile, quad, lane) -> row tile * 16 + lane % 16, vector 4 quad + lane / 16
+  constexpr int OUT = (PAIR ? RT / 2 : RT) * NQ * kWave;
+  for (int o = threadIdx.x; o < OUT; o += blockDim.x) {
+    const int l = o & (kWave - 1), q = (o / kWave) % NQ, t = o / (kWave * NQ);
+    const int vec = 4 * (q0 + q) + (l >> 4);
+    if (vec >= d.count) continue;
+    const float fac = d.fac[vec];
+    float v = total(o) * fac;
+    if constexpr (PAIR) {
+      const int h = a.rows / 2, row = (int(blockIdx.x) * (RT / 2) + t) * kTile + (l & 15);
+      float u = total(OUT + o) * fac;
+      if (a.bias) v += a.bias[row], u += a.bias[h + row];
+      a.y[size_t(vec) * h + row] = silu(v) * u;
+    } else {
+      const int row = (int(blockIdx.x) * RT + t) * kTile + (l & 15);
+      if (row < a.rows) {
+        if (a.bias) v += a.bias[row];
+        if (a.resid) v += a.resid[size_t(vec) * a.rows + row];
+        a.y[size_t(vec) * a.rows + row] = v;
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Many vectors: 4 waves of RT row tiles x the same NQ quads, the quads'
+// fragments of a chunk staged in LDS (two chunks deep).
+template <int FMT, bool COPY, int NQ, int RT, int EPI>
+__global__ __launch_bounds__(256, 3) void digit_tile_kernel(GemvArgs a, DigitVectors d) {
+  constexpr int CW = Source<FMT, COPY>::CW, S = Fmt<FMT>::S;
+  constexpr bool PAIR = EPI == kEpiSiluPair;
+  constexpr int WAVES = 4;
+  __shared__ __attribute__((aligned(16))) char frags[2][NQ * kQuadChunk];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+  const int li = lane & 15, kq = lane >> 4;
+  const int Kc = a.Kp / kChunk;
+  const uint32_t Npad = uint32_t(a.Npad);
+  const int quads = (d.count + 3) / 4, q0 = int(blockIdx.y) * NQ;
+  const int wg = int(blockIdx.x) * WAVES + wave;   // the wave's group of RT tiles
+  const int half_rows = a.rows / 2;
+  uint32_t row0[RT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    if constexpr (PAIR)   // groups past the last redo it and are not stored
+      row0[t] = uint32_t((t < RT / 2 ? 0 : half_rows) +
+                         min((wg * (RT / 2) + t % (RT / 2)) * kTile, half_rows - kTile));
+    else
+      row0[t] = uint32_t(min((wg * RT + t) * kTile, a.Npad - kTile));
+  }
+  const size_t qbytes = size_t(Kc) * kQuadChunk;
+  constexpr int LD = NQ * int(kQuadChunk) / (256 * 16);   // 16-byte pieces per thread and chunk
+  static_assert(LD * 256 * 16 == NQ * int(kQuadChunk), "whole pieces");
+  // A chunk's codes and fragments are requested two chunks ahead (they come
+  // from the MALL where another XCD wrote or read them first); past the last
+  // chunk the last one is requested again.
+  uint32_t w[2][RT][CW];
+  float sc[2][RT][S];
+  v4i st[2][LD];
+  const char *fsrc[LD];
+#pragma unroll
+  for (int i = 0; i < LD; ++i) {
+    const int p = int(threadIdx.x) + 256 * i, q = p / 128, o = p % 128;
+    fsrc[i] = d.digits + size_t(min(q0 + q, quads - 1)) * qbytes + o * 16;
+  }
+  const auto load_f = [&](int b, int ch) {
+#pragma unroll
+    for (int i = 0; i < LD; ++i) st[b][i] = *reinterpret_cast<const v4i *>(fsrc[i] + size_t(min(ch, Kc - 1)) * kQuadChunk);
+  };
+  const auto store_f = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < LD; ++i) *reinterpret_cast<v4i *>(frags[b] + (int(threadIdx.x) + 256 * i) * 16) = st[b][i];
+  };
+  const auto load_w = [&](int b, int ch) {
+    ch = min(ch, Kc - 1);
+    const uint32_t g = uint32_t(scale_group(a, ch));
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      load_codes<FMT, COPY, false>(a, uint32_t(ch), row0[t], uint32_t(li), uint32_t(kq), w[b][t]);
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+        sc[b][t][s] = (a.scales + size_t(s * a.n_groups + g) * Npad + row0[t])[uint32_t(li)];
+    }
+  };
+  float acc[RT][NQ];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) acc[t][q] = 0.0f;
+  const auto chunk = [&](int ch, const int b) {   // b = ch % 2
+    load_f(b, ch + 2);
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      uint32_t wb[RT][8];
+      float cs[RT];
+#pragma unroll
+      for (int t = 0; t < RT; ++t) {
+        source_bytes<FMT, COPY>(w[b][t], s, wb[t]);
+        cs[t] = sc[b][t][s];
+      }
+      if (s == S - 1) load_w(b, ch + 2);   // the words are bytes now
+      // The products of quad q run while quad q - 1's sums are joined and quad
+      // q + 1's fragments arrive; the barriers keep the compiler from issuing
+      // every quad's reads and products first (registers).
+      v4i f[2][2], sum[2][RT];
+      const auto read = [&](int q) {
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          f[q & 1][m] = *reinterpret_cast<const v4i *>(frags[b] + q * kQuadChunk + m * 1024 + lane * 16);
+      };
+      read(0);
+#pragma unroll
+      for (int q = 0; q <= NQ; ++q) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (q + 1 < NQ) read(q + 1);
+        if (q < NQ) {
+#pragma unroll
+          for (int t = 0; t < RT; ++t) sum[q & 1][t] = chunk_product(wb[t], f[q & 1][0], f[q & 1][1]);
+        }
+        if (q > 0) {
+#pragma unroll
+          for (int t = 0; t < RT; ++t) {
+            acc[t][q - 1] = fmaf(join_digits(sum[(q - 1) & 1][t]), cs[t], acc[t][q - 1]);
+            asm volatile("" : "+v"(acc[t][q - 1]));   // else every join sinks to the chunk's end
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    store_f(b ^ 1);
+    __syncthreads();
+  };
+  load_f(0, 0);
+  load_w(0, 0);
+  load_f(1, 1);
+  load_w(1, 1);
+  store_f(0);
+  __syncthreads();
+#pragma unroll 1
+  for (int ch = 0; ch < Kc; ch += 2) {   // Kc is even
+    chunk(ch, 0);
+    chunk(ch + 1, 1);
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int vec = 4 * (q0 + q) + kq;
+    if (vec >= d.count) continue;
+    const float fac = d.fac[vec];
+    const int ex = d.exp[vec];
+#pragma unroll
+    for (int t = 0; t < (PAIR ? RT / 2 : RT); ++t) {
+      float v = vector_scale(acc[t][q], fac, ex);
+      if constexpr (PAIR) {
+        const int row = (wg * (RT / 2) + t) * kTile + li;
+        if (row >= half_rows) continue;
+        float u = vector_scale(acc[RT / 2 + t][q], fac, ex);
+        if (a.bias) v += a.bias[row], u += a.bias[half_rows + row];
+        a.y[size_t(vec) * half_rows + row] = silu(v) * u;
+      } else {
+        const int row = (wg * RT + t) * kTile + li;
+        if (row >= a.rows) continue;
+        if (a.bias) v += a.bias[row];
+        if (a.resid) v += a.resid[size_t(vec) * a.rows + row];
+        a.y[size_t(vec) * a.rows + row] = v;
+      }
+    }
+  }
+}
+
+int launched(const char *what) {
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? LMX_OK : fail(LMX_ERR_LAUNCH_FAILED, "%s launch: %s", what, hipGetErrorString(e));
+}
+
+// Batches come with a handle, so with its code copy where the format has one.
+template <int FMT, int NQ, int RT>
+int launch_rows(const GemvArgs &a, const DigitVectors &d, hipStream_t st) {
+  constexpr bool COPY = has_copy<FMT>();
+  const bool pair = a.epi == kEpiSiluPair;
+  const int Kc = a.Kp / kChunk, W = Kc >= 16 ? 16 : Kc;
+  const unsigned gx = pair ? a.rows / 2 / (RT / 2 > 0 ? RT / 2 : 1) / kTile : a.Npad / RT / kTile;
+  const unsigned gy = ((d.count + 3) / 4 + NQ - 1) / NQ;
+  // slices of the chunks where the row blocks alone leave most CUs idle, each
+  // wave keeping at least a chunk
+  // (at most 256 workgroups then: their tickets and sums fit the scratch)
+  int slices = 1;
+  while (gx * gy * (slices + 1) <= 256 && Kc / (slices + 1) >= W) ++slices;
+  const dim3 grid{gx, gy, unsigned(slices)}, block{unsigned(W * kWave)};
+  if (pair) {
+    if constexpr (RT >= 2) digit_rows_kernel<FMT, COPY, NQ, RT, kEpiSiluPair><<<grid, block, 0, st>>>(a, d);
+  } else {
+    digit_rows_kernel<FMT, COPY, NQ, RT, kEpiStore><<<grid, block, 0, st>>>(a, d);
+  }
+  return launched("digit_rows");
+}
+
+template <int FMT, int NQ, int RT>
+int launch_tile(const GemvArgs &a, const DigitVectors &d, hipStream_t st) {
+  constexpr bool COPY = has_copy<FMT>();
+  const int quads = (d.count + 3) / 4;
+  const int groups = a.epi == kEpiSiluPair ? (a.rows / 2 / kTile + RT / 2 - 1) / (RT / 2) : (a.Npad / kTile + RT - 1) / RT;
+  const dim3 grid{unsigned((groups + 3) / 4), unsigned((quads + NQ - 1) / NQ)};
+  if (a.epi == kEpiSiluPair) digit_tile_kernel<FMT, COPY, NQ, RT, kEpiSiluPair><<<grid, dim3(256), 0, st>>>(a, d);
+  else digit_tile_kernel<FMT, COPY, NQ, RT, kEpiStore><<<grid, dim3(256), 0, st>>>(a, d);
+  return launched("digit_tile");
+}
+
+template <int FMT>
+int launch_gemm_fmt(const GemvArgs &a, const DigitVectors &d, hipStream_t st) {
+  if (d.tile) return launch_tile<FMT, 8, 2>(a, d, st);
+  const int quads = (d.count + 3) / 4;
+  if (quads <= 2) return launch_rows<FMT, 2, 2>(a, d, st);
+  return launch_rows<FMT, 4, 2>(a, d, st);
+}
+
+template <int FMT, bool COPY, int NV, int RT, int PPW>
+int launch_digit_gemv_cfg(const GemvArgs &a, int nv, int W, hipStream_t st) {
+  const dim3 block{unsigned(W * kWave)};
+  const bool pair = a.epi == kEpiSiluPair;
+  const dim3 grid{unsigned(pair ? a.rows / 2 / (kTile * RT / 2) : a.Npad / (kTile * RT))};
+  if (pair) {
+    if constexpr (RT >= 2)
+      digit_gemv_kernel<FMT, COPY, NV, RT, PPW, kXModeRmsNorm, kEpiSiluPair><<<grid, block, 0, st>>>(a, nv);
+  } else if (a.xmode == kXModeRmsNorm) {
+    digit_gemv_kernel<FMT, COPY, NV, RT, PPW, kXModeRmsNorm, kEpiStore><<<grid, block, 0, st>>>(a, nv);
+  } else {
+    digit_gemv_kernel<FMT, COPY, NV, RT, PPW, kXModeNone, kEpiStore><<<grid, block, 0, st>>>(a, nv);
+  }
+  return launched("digit_gemv");
+}
+
+template <int FMT, bool COPY, int NV, int RT>
+int launch_digit_gemv_rt(const GemvArgs &a, int nv, hipStream_t st) {
+  // as few rounds of 256-chunks per wave as 16 waves allow, spread evenly
+  const int pairs = a.Kp / kRotChunk;
+  const int per = (pairs + 15) / 16;
+  const int W = (pairs + per - 1) / per;
+  if constexpr (NV == 1) {
+    if (per >= 2) return launch_digit_gemv_cfg<FMT, COPY, NV, RT, 2>(a, nv, W, st);
+  }
+  return launch_digit_gemv_cfg<FMT, COPY, NV, RT, 1>(a, nv, W, st);
+}
+
+template <int FMT, bool COPY>
+int launch_digit_gemv_src(const GemvArgs &a, int nv, hipStream_t st) {
+  const bool two = digit_gemv_tiles(a) == 2;
+  if (nv == 1) return two ? launch_digit_gemv_rt<FMT, COPY, 1, 2>(a, nv, st) : launch_digit_gemv_rt<FMT, COPY, 1, 1>(a, nv, st);
+  return two ? launch_digit_gemv_rt<FMT, COPY, 4, 2>(a, nv, st) : launch_digit_gemv_rt<FMT, COPY, 4, 1>(a, nv, st);
+}
+
+template <int FMT>
+int launch_digit_gemv_fmt(const GemvArgs &a, int nv, hipStream_t st) {
+  if constexpr (has_copy<FMT>()) {
+    if (a.codes) return launch_digit_gemv_src<FMT, true>(a, nv, st);
+  }
+  return launch_digit_gemv_src<FMT, false>(a, nv, st);
+}
+
+// The code copy of 4- and 8-bit planes: one thread per plane word of a row.
+template <int FMT>
+__global__ __launch_bounds__(256) void code_copy_kernel(const uint32_t *__restrict__ planes, uint32_t Npad, size_t n,
+                                                        uint32_t *__restrict__ codes) {
+  constexpr int P = Fmt<FMT>::P;
+  const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;   // (chunk * Npad + row) * 4 + kq
+  if (i >= n) return;
+  const size_t rk = i % (size_t(Npad) * 4), ch = i / (size_t(Npad) * 4);
+  uint32_t w[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) w[p] = planes[(ch * P + p) * Npad * 4 + rk];
+  if constexpr (FMT == LMX_FMT_INT4) {
+    uint32_t nib[4];
+    nibbles(w[0], w[1], w[2], ~w[3], nib);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) codes[i * 4 + j] = nib[j];
+  } else {
+    uint32_t out[8];
+    code_bytes<FMT>(w, 0, out);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) codes[i * 8 + j] = out[j];
+  }
+}
+
+template <int FMT>
+int launch_code_copy_fmt(const void *planes, size_t Npad, size_t Kp, void *codes, hipStream_t st) {
+  if constexpr (has_copy<FMT>()) {
+    const size_t n = Kp / kChunk * Npad * 4;
+    code_copy_kernel<FMT><<<dim3(unsigned((n + 255) / 256)), dim3(256), 0, st>>>(
+        static_cast<const uint32_t *>(planes), uint32_t(Npad), n, static_cast<uint32_t *>(codes));
+    return launched("code_copy");
+  }
+  return LMX_OK;
+}
+
+}  // namespace
+}  // namespace lmx
+
+#endif  // LMX_DIGIT_KERNELS_HPP

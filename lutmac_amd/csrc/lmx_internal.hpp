@@ -8,6 +8,8 @@
 
 #include "lutmac_hip.h"
 
+struct lmx_weight;
+
 namespace lmx {
 
 constexpr int kChunk = 128;        // k per chunk: one uint4 per plane per row
@@ -51,6 +53,7 @@ void nibble_tiles(const uint8_t *planes, size_t rows, size_t row_bytes, size_t N
 struct GemvArgs {
   const void *planes;      // tiled planes
   const void *nib;         // int4 codes in the matrix-core layout (nibble_tiles), or null
+  const void *codes;       // digit kernels: 4- and 8-bit code copy (code_copy_bytes), or null
   const float *scales;     // [S][n_groups][Npad]
   const float *x;          // [cols]
   float *y;                // [rows]
@@ -210,6 +213,37 @@ int batched_launch_splits(size_t Npad, size_t Kp);
 // one round of workgroups; quad_serves tells beforehand).
 int launch_gemv_quad(int fmt, const GemvArgs &a, void *stream);
 bool quad_serves(const GemvArgs &a);
+// ---- digit kernels (lmx_digit.hip): exact products on the 8-bit matrix cores ----
+// Vectors split into signed-byte digits by launch_digit_split.
+struct DigitVectors {
+  char *digits;       // [quads of 4 vectors][Kp/128][2 KiB]
+  float *fac;         // [count] factor of a vector's sums (norm, rotation, code scale; NaN: not finite)
+  int *exp;           // tile form: [count] the power of two of a vector's digits
+  float *mult;        // rows form: [quads][Kp/128][4] that of each vector's chunk
+  float *partials;    // rows form: sums of k-slices (kDigitPartials bytes)
+  int count;
+  int tile;           // for the tile kernel (many vectors and rows), else the rows kernel
+};
+constexpr unsigned kDigitTickets = 256;   // row blocks of a sliced rows launch, at most
+// Bytes of slice sums: up to 256 workgroups of 2 row tiles x 4 quads x 64 sums.
+constexpr size_t kDigitPartials = 256 * 512 * sizeof(float);
+size_t digit_bytes(size_t Kp, size_t vectors);
+size_t digit_capacity(size_t Kp, size_t bytes);   // vectors (a multiple of 4) that fit in bytes
+DigitVectors digit_vectors(const lmx_weight *w, void *scratch, size_t count);
+// a.x [count][cols], transform a.xmode (a.xw, a.eps), a.rotate -> d
+int launch_digit_split(int fmt, const GemvArgs &a, const DigitVectors &d, void *stream);
+// y = W x of the split vectors (+ a.bias per row) (+ a.resid per vector row), or the SiLU pair (a.epi)
+int launch_digit_gemm(int fmt, const GemvArgs &a, const DigitVectors &d, void *stream);
+// 1..4 vectors in one launch, with transform a.xmode and epilogue a.epi
+// (argmax keys, one slot per workgroup, for one vector)
+int launch_digit_gemv(int fmt, const GemvArgs &a, int nv, void *stream);
+int digit_gemv_tiles(const GemvArgs &a);   // 16-row tiles per workgroup of that launch
+// 4- and 8-bit codes laid out for the matrix-core operands, made from the
+// plane tiles on the device: [Kp/128][Npad][4 plane words][4 or 8 words];
+// 0 bytes for the other formats, which the kernels read from the planes.
+size_t code_copy_bytes(int fmt, size_t Npad, size_t Kp);
+int launch_code_copy(int fmt, const void *planes, size_t Npad, size_t Kp, void *codes, void *stream);
+
 // Number of argmax key slots a launch with these arguments writes.
 size_t gemv_argmax_slots(const GemvArgs &a);
 int launch_fwht256(float *x, size_t n, void *stream);
@@ -238,15 +272,21 @@ struct lmx_weight {
   int fullk = 0;           // full-K kernel configuration (kFullK_*), 0 = split-K
   int kfamily = 0;         // full-K kernel family for plain activations (kKernel*)
   int staged = 1;          // full-K: later chunks' weight loads after the prologue
+  void *d_weight = nullptr;      // allocation of the planes, codes and scales
+  void *d_scratch = nullptr;     // allocation of the counters, staging and partials
   void *d_planes = nullptr;
   float *d_scales = nullptr;
   float *d_partials = nullptr;
   unsigned *d_counters = nullptr;
   float *d_xrot = nullptr;  // staging for LMX_ROTATE_FWHT_FULL (cols floats)
+  bool digit = true;             // digit kernels (LMX_DIGIT=0, or a lookup-table plan asked for: not)
   bool batched = true;           // batch >= 2 through the batched kernel (LMX_BATCHED=0: one GEMV per vector)
-  float *d_bpartials = nullptr;  // batched partials [16][Kp/256][Npad], allocated with the handle
+  float *d_bpartials = nullptr;  // batched partials [16][Kp/256][Npad] (the memory of d_partials)
+  void *d_codes = nullptr;       // digit kernels: 4- and 8-bit code copy
   void *d_nib = nullptr;         // int4 with the matrix-core kernel: codes in nibble_tiles layout
   size_t bpartials_cap = 0;      // floats
+  void *d_digits = nullptr;      // scratch of the digit kernels: d_bpartials, or the caller's
+  size_t digit_cap = 0;          // its bytes
 };
 
 namespace lmx {
@@ -263,6 +303,9 @@ GemvArgs weight_args(const lmx_weight *w);
 // below 4).
 int gemv_batched(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream,
                  size_t *done);
+// y = W x of `batch` vectors on the digit kernels (a.bias, a.resid, a.rotate; x of any alignment);
+// *done = the vectors covered, the rest (one by one on the lookup tables) left to the caller
+int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done);
 // Whether gemv_batched serves epilogue epi (kEpi*) for `batch` vectors of w
 // with no vector left to the single-vector path (x 16-byte aligned assumed).
 bool batched_epilogue_ok(const lmx_weight *w, int epi, size_t batch);

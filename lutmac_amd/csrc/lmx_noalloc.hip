@@ -13,7 +13,8 @@
 //                 fixed region, so no other call's staging or partials ever
 //                 land on a counter (up to 16384 row blocks, Npad <= 1 Mi rows)
 //   [64 KiB, +X)  staging copy of x (unaligned x, length-K FWHT)   X = Kp * 4
-//   [.., ...)     split-K partials [Kp/kslice][Npad] fp32 (split-K plans only)
+//   [.., ...)     split-K partials [Kp/kslice][Npad] fp32 (split-K plans), or
+//                 the digits of up to 4 vectors and their slice sums
 // The counters must read zero when a call starts: the first call on a
 // device zeroes the whole array with a fill kernel and waits for it before
 // any call may use the array, and every split-K launch leaves each counter
@@ -88,7 +89,7 @@ extern "C" int lmx_gemv_tiles_noalloc(int format, const void *tiles, const float
     return fail(LMX_ERR_INVALID_ARGUMENT, "tiles must be 16-byte and scales 4-byte aligned");
   lmx_weight w;   // the plan lmx_weight_create would choose, over the caller's buffers
   plan_weight(&w, format, rows, cols, group);
-  w.batched = false;   // one vector at a time: the batched kernel's partials would not fit
+  w.batched = false;   // the batched lookup kernel's partials would not fit
   const size_t row_blocks = w.Npad / kWave;
   const size_t staging = round_up(w.Kp * sizeof(float), 256);
   // split-K plans, and the layered full-K plan (which runs the split-K
@@ -113,5 +114,9 @@ extern "C" int lmx_gemv_tiles_noalloc(int format, const void *tiles, const float
   w.d_counters = reinterpret_cast<unsigned *>(base);
   w.d_xrot = reinterpret_cast<float *>(base + kCounterBytes);
   w.d_partials = reinterpret_cast<float *>(base + kCounterBytes + staging);
+  if (kCounterBytes + staging + digit_bytes(w.Kp, 4) + kDigitPartials <= kScratchBytes) {
+    w.d_digits = base + kCounterBytes + staging;   // one group of up to 4 vectors at a time
+    w.digit_cap = digit_bytes(w.Kp, 4) + kDigitPartials;
+  }
   return gemv_impl(&w, x, y, batch, flags, stream);
 }

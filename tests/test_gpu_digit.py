@@ -1,0 +1,151 @@
+"""The digit kernels (exact products on the 8-bit matrix cores) at the edges of
+their tiles, slices and groups, against 64-bit sums.
+
+An output sums K products whose activations are fixed point below 2^-30 of
+their chunk's (or vector's) largest magnitude, and ceil(K / 128) chunk sums
+rounded to fp32: the bound is that rounding over the sum of the chunks'
+magnitudes, plus the FWHT's 10 roundings where the call rotates."""
+import numpy as np
+import pytest
+import torch
+
+import lutmac_amd as L
+from lutmac_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.0 ** -24
+
+
+def fwht64(x):
+    y = x.reshape(-1, 256).astype(np.float64).copy()
+    h = 1
+    while h < 256:
+        y = y.reshape(-1, 256 // (2 * h), 2, h)
+        y = np.stack([y[:, :, 0] + y[:, :, 1], y[:, :, 0] - y[:, :, 1]], axis=2).reshape(-1, 256)
+        h *= 2
+    return y.reshape(x.shape) / 16
+
+
+def check(fmt, planes, scales, rows, cols, group, x, y, rotate, bias=None):
+    """y [batch, rows] of x [batch, cols] within the derived bound (cols a multiple of 256 when rotating)."""
+    W = synth.dequant_f64(fmt, planes, scales, rows, cols, group)
+    xr = fwht64(x) if rotate else x.astype(np.float64)
+    ref = xr @ W.T
+    mag = np.abs(xr) @ np.abs(W).T
+    big = np.abs(xr).max(axis=1, keepdims=True) * np.abs(W).sum(axis=1)[None, :]
+    chunks = -(-cols // 128) + 18 * L.STAGES[fmt]     # the running sum, the wave and slice sums, scales and joins
+    bound = (chunks + (20 if rotate else 0)) * EPS * mag + 2.0 ** -29 * big
+    if rotate:
+        bound = bound + 10 * EPS * np.abs(x).sum(axis=1, keepdims=True) * np.abs(W).max()
+    if bias is not None:
+        ref = ref + bias
+        bound = bound + EPS * np.abs(ref)
+    err = np.abs(y - ref)
+    worst = float((err - bound).max())
+    assert worst <= 0, (L.FORMAT_NAMES[fmt], rows, cols, x.shape[0], worst, float(err.max()))
+
+
+def make(fmt, rows, cols, seed, group=128):
+    planes, scales, g = synth.make_weights(fmt, rows, cols, seed=seed, group=group)
+    return planes, scales, g, L.Weight.from_planes(fmt, planes, scales, rows, cols, g)
+
+
+def vectors(batch, cols, seed):
+    return np.stack([synth.make_activations(cols, seed=seed + i, outliers=True) for i in range(batch)])
+
+
+# 1..4 vectors take one launch (the 1-3 bit formats from 2), more the split
+# vectors: quads and groups of quads partly filled, rows past the last tile,
+# a K of one 256-chunk, of more waves than chunks, and of several rounds.
+@pytest.mark.parametrize("fmt", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("rows,cols", [(1, 256), (65, 768), (300, 2048), (130, 8960)])
+@pytest.mark.parametrize("batch", [1, 2, 4, 5, 9, 17])
+def test_digit_linear(cuda, fmt, rows, cols, batch):
+    planes, scales, g, w = make(fmt, rows, cols, seed=rows + cols + fmt)
+    x = vectors(batch, cols, seed=batch)
+    bias = np.random.default_rng(3).standard_normal(rows).astype(np.float32)
+    xd = torch.from_numpy(x).cuda()
+    y = w.linear(xd, bias=torch.from_numpy(bias).cuda()).cpu().numpy().reshape(batch, rows)
+    check(fmt, planes, scales, rows, cols, g, x, y, rotate=fmt in (1, 2, 3, 4), bias=bias)
+    w.close()
+
+
+# The tile kernel takes over at 192 workgroups (8 row tiles x 32 vectors
+# each): a shape on either side, a last row group and vector group partly
+# filled, and a group scale of three chunks.
+@pytest.mark.parametrize("fmt", [1, 3, 4, 6, 7])
+@pytest.mark.parametrize("rows,cols,batch,group", [(2040, 512, 353, 128), (2040, 512, 383, 128), (6100, 768, 129, 384)])
+def test_digit_tiles(cuda, fmt, rows, cols, batch, group):
+    planes, scales, g, w = make(fmt, rows, cols, seed=7 + fmt, group=group)
+    x = vectors(batch, cols, seed=50)
+    y = w.gemv(torch.from_numpy(x).cuda()).cpu().numpy().reshape(batch, rows)
+    check(fmt, planes, scales, rows, cols, g, x, y, rotate=False)
+    w.close()
+
+
+# A handful of rows over a long K: the k-slices of a row block are summed by
+# its last workgroup, whose ticket is back at zero for the next call.
+def test_digit_slices_repeat(cuda):
+    planes, scales, g, w = make(L.FMT_INT4, 200, 8192, seed=1)
+    x = vectors(6, 8192, seed=2)
+    xd = torch.from_numpy(x).cuda()
+    first = w.gemv(xd).cpu().numpy()
+    check(L.FMT_INT4, planes, scales, 200, 8192, g, x, first.reshape(6, 200), rotate=False)
+    for _ in range(3):
+        assert np.array_equal(w.gemv(xd).cpu().numpy().view(np.uint32), first.view(np.uint32))
+    w.close()
+
+
+# Activations far from 1 (the fixed point follows the exponent), all zero, and
+# not finite: such a vector gives NaN in every row, the others are untouched.
+@pytest.mark.parametrize("batch", [1, 3, 6])
+def test_digit_ranges(cuda, batch):
+    rows, cols = 96, 512
+    planes, scales, g, w = make(L.FMT_INT4, rows, cols, seed=5)
+    base = vectors(batch, cols, seed=9)
+    for factor in (2.0 ** 100, 2.0 ** -90):
+        x = (base * np.float32(factor)).astype(np.float32)
+        y = w.gemv(torch.from_numpy(x).cuda()).cpu().numpy().reshape(batch, rows)
+        check(L.FMT_INT4, planes, scales, rows, cols, g, x, y, rotate=False)
+    assert not w.gemv(torch.zeros(batch * cols, device="cuda")).any()
+    for bad in (float("inf"), float("nan")):
+        x = base.copy()
+        x[0, 77] = bad
+        y = w.gemv(torch.from_numpy(x).cuda()).cpu().numpy().reshape(batch, rows)
+        assert np.isnan(y[0]).all()
+        if batch > 1:
+            check(L.FMT_INT4, planes, scales, rows, cols, g, x[1:], y[1:], rotate=False)
+    w.close()
+
+
+# x of any 4-byte alignment and a column count that is no multiple of 4
+def test_digit_unaligned(cuda):
+    rows, cols, batch = 70, 1000, 7
+    planes, scales, g, w = make(L.FMT_INT8, rows, cols, seed=6)
+    x = vectors(batch, cols, seed=3)
+    buf = torch.empty(batch * cols + 1, device="cuda")
+    buf[1:] = torch.from_numpy(x.ravel()).cuda()
+    y = w.gemv(buf[1:]).cpu().numpy().reshape(batch, rows)
+    check(L.FMT_INT8, planes, scales, rows, cols, g, x, y, rotate=False)
+    w.close()
+
+
+# Captured and replayed with eager calls between, one shape of each kernel
+@pytest.mark.parametrize("rows,cols,batch", [(512, 2048, 1), (512, 2048, 4), (512, 8192, 16), (2048, 512, 400)])
+def test_digit_graph(cuda, rows, cols, batch):
+    planes, scales, g, w = make(L.FMT_INT4, rows, cols, seed=8)
+    x = torch.randn(batch * cols, device="cuda")
+    eager = w.gemv(x).clone()
+    out = torch.empty_like(eager)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        w.gemv(x, out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        w.gemv(x)
+        torch.cuda.synchronize()
+    w.close()
