@@ -174,14 +174,30 @@ def _dev_ptr(t):
         raise ValueError("expected a device tensor")
     if not t.is_contiguous():
         raise ValueError("expected a contiguous tensor")
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
+
+
+_CURRENT_STREAM = None
+
+
+def _current_stream():
+    """Handle of torch's current stream on the current device.  The raw lookup
+    takes 0.2 us where building a torch Stream object takes 2.7 us, a third of
+    a small GEMV's call."""
+    global _CURRENT_STREAM
+    if _CURRENT_STREAM is None:
+        import torch
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        device = getattr(torch._C, "_cuda_getDevice", None)
+        if raw is None or device is None or not torch.cuda.is_available():
+            return torch.cuda.current_stream().cuda_stream
+        torch.cuda.init()
+        _CURRENT_STREAM = lambda: raw(device())   # noqa: E731
+    return _CURRENT_STREAM()
 
 
 def _stream_ptr(stream):
-    if stream is None:
-        import torch
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    return _current_stream() if stream is None else stream.cuda_stream
 
 
 # ---- host-only helpers -----------------------------------------------------
@@ -354,17 +370,17 @@ class Weight:
         return out
 
     def gemv(self, x, y=None, flags=ROTATE_NONE, stream=None):
-        import torch
         batch = x.numel() // self.cols
         if y is None:
+            import torch
             y = torch.empty(batch * self.rows, dtype=torch.float32, device=x.device)
         check(lib().lmx_gemv(self._h, _dev_ptr(x), _dev_ptr(y), batch, flags, _stream_ptr(stream)))
         return y
 
     def linear(self, x, bias=None, y=None, stream=None):
-        import torch
         batch = x.numel() // self.cols
         if y is None:
+            import torch
             y = torch.empty(batch * self.rows, dtype=torch.float32, device=x.device)
         check(lib().lmx_linear(self._h, _dev_ptr(bias), _dev_ptr(x), _dev_ptr(y), batch,
                                _stream_ptr(stream)))
