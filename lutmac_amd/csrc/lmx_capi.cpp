@@ -207,8 +207,8 @@ int upload(int fmt, size_t rows, size_t cols, size_t group, const uint8_t *plane
   }
   tile_planes(fmt, planes, rows, row_bytes, w->Npad, w->Kp, tiles.data());
   for (int s = 0; s < fi.stages; ++s)
-    for (size_t r = 0; r < rows; ++r)
-      for (size_t g = 0; g < ng_src && g < w->n_groups; ++g)
+    for (size_t g = 0; g < ng_src && g < w->n_groups; ++g)
+      for (size_t r = 0; r < rows; ++r)
         sc[(size_t(s) * w->n_groups + g) * w->Npad + r] = scales[(size_t(s) * rows + r) * ng_src + g];
 
   // Two allocations a handle: the weight (planes, code copy, scales) and the
@@ -360,9 +360,12 @@ int gemv_batched(const lmx_weight *w, GemvArgs a, const float *x, float *y, size
 // bit format stays on the lookup tables, whose planes are half to an eighth of
 // the bytes while the digits cost the same (8192 x 8192, us: ternary 6.5
 // against 8.2, RRQ-2 7.1 / 9.5, binary 5.3 / 7.1; 4-bit 9.7 / 8.0, 8-bit
-// 17.9 / 15.7).  *done = the vectors covered.
-int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done) {
+// 17.9 / 15.7).  *done = the vectors covered; `all`: every one, the single
+// vectors of those formats too (a.xmode and a.epi have no other form there).
+int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done,
+                 bool all) {
   const float *resid = a.resid;
+  const size_t out_rows = a.epi == kEpiSiluPair ? w->rows / 2 : w->rows;
   const bool copies = code_copy_bytes(w->format, 1, kRotChunk) != 0;
   // (the split kernels read the code copy where the format has one)
   const size_t cap = w->d_digits && (!copies || w->d_codes) ? digit_capacity(w->Kp, w->digit_cap) : 0;
@@ -370,21 +373,21 @@ int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size
   for (*done = 0; *done < batch;) {
     const size_t left = batch - *done;
     a.x = x + *done * w->cols;
-    a.y = y + *done * w->rows;
-    a.resid = resid ? resid + *done * w->rows : nullptr;
+    a.y = y + *done * out_rows;
+    a.resid = resid ? resid + *done * out_rows : nullptr;
     size_t n = std::min<size_t>(left, 4);
     int st;
     // One launch for up to 4 vectors makes their digits once per row block:
     // past 16 256-chunks that costs more than a launch of its own, unless the
     // codes themselves are most of the work (2048 x 8192, 4 vectors, us:
     // ternary 11.4 against 9.4 split, 4-bit 8.0 / 9.1).
-    if (cap && (left > 4 || (left > 1 && !copies && w->Kp > 4096))) {
+    if (cap && (left > 4 || (!copies && w->Kp > 4096 && (left > 1 || all)))) {
       n = std::min(left, cap);
       const DigitVectors d = digit_vectors(w, w->d_digits, n);
       if ((st = launch_digit_split(w->format, a, d, stream)) || (st = launch_digit_gemm(w->format, a, d, stream)))
         return st;
     } else {
-      if (!copies && (left == 1 || w->Kp > 4096)) return LMX_OK;   // one by one on the lookup tables
+      if (!copies && !all && (left == 1 || w->Kp > 4096)) return LMX_OK;   // one by one on the lookup tables
       if ((st = launch_digit_gemv(w->format, a, int(n), stream))) return st;
     }
     *done += n;
@@ -651,7 +654,7 @@ int gemv_impl(const lmx_weight *w, const float *x, float *y, size_t batch, unsig
   size_t b0 = 0;
   if (flags != LMX_ROTATE_FWHT_FULL) {
     a.rotate = flags == LMX_ROTATE_FWHT256 ? LMX_ROTATE_FWHT256 : LMX_ROTATE_NONE;
-    if ((st = w->digit ? digit_linear(w, a, x, y, batch, stream, &b0) : gemv_batched(w, a, x, y, batch, stream, &b0)))
+    if ((st = w->digit ? digit_linear(w, a, x, y, batch, stream, &b0, false) : gemv_batched(w, a, x, y, batch, stream, &b0)))
       return st;
   }
   for (size_t b = b0; b < batch; ++b) {
@@ -687,7 +690,7 @@ int lmx_linear(const lmx_weight *w, const float *bias, const float *x, float *y,
   a.bias = bias;
   a.rotate = rotate ? LMX_ROTATE_FWHT256 : LMX_ROTATE_NONE;
   size_t b0 = 0;
-  if ((st = w->digit ? digit_linear(w, a, x, y, batch, stream, &b0) : gemv_batched(w, a, x, y, batch, stream, &b0)))
+  if ((st = w->digit ? digit_linear(w, a, x, y, batch, stream, &b0, false) : gemv_batched(w, a, x, y, batch, stream, &b0)))
     return st;
   for (size_t b = b0; b < batch; ++b) {
     a.x = x + b * w->cols;

@@ -41,6 +41,7 @@
 #include "lmx_device.hpp"
 #include "lmx_internal.hpp"
 #include "lmx_lanes.hpp"
+#include "lmx_prefill.hpp"
 #include "lutmac_decode.h"
 
 namespace lmx {
@@ -86,13 +87,15 @@ template <int FMT>
 __global__ __launch_bounds__(256) void embed_kernel(const uint8_t *__restrict__ planes, const float *__restrict__ scales,
                                                     int Npad, int rows, int n_groups, int group_chunks, int cols,
                                                     const int *__restrict__ tokens, const int *__restrict__ pos,
-                                                    float *__restrict__ out, int tstride) {
+                                                    float *__restrict__ out, int tstride, int T, int p0) {
   constexpr int P = EmbFmt<FMT>::P, S = EmbFmt<FMT>::S;
   const int k = blockIdx.x * 256 + threadIdx.x;
   if (k >= cols) return;
-  // sequence blockIdx.y: its tokens at tokens[y * tstride], its row at out[y * cols]
+  // row y = b * T + t: sequence b (its tokens at tokens[b * tstride]), position
+  // t of the T from *pos, or from p0 where pos is null; its row at out[y * cols]
   out += size_t(blockIdx.y) * cols;
-  const int t = min(max(tokens[size_t(blockIdx.y) * tstride + *pos], 0), rows - 1);
+  const int at = (pos ? *pos : p0) + int(blockIdx.y) % T;
+  const int t = min(max(tokens[size_t(int(blockIdx.y) / T) * tstride + at], 0), rows - 1);
   const int c = k / kChunk, byte = (k % kChunk) / 8, bit = 7 - k % 8;
   int b[P];
 #pragma unroll
@@ -853,6 +856,10 @@ struct lmx_decoder {
   unsigned *penalty_counts() const { return penalty != 1.0f ? pcount : nullptr; }
   int n_forced = 0;
   size_t host_pos = 0;
+  // Rows of a prompt pass (prefill_rows of them), allocated by the first prompt long enough
+  float *p_hidden = nullptr, *p_qkv = nullptr, *p_attn = nullptr, *p_gate_up = nullptr, *p_act = nullptr;
+  int prompt_pos = 0;        // where the steps start after the prompt passes
+  bool warm = false;         // an eager step has set up every kernel
   float pos_div = 1.0f;
   // Attention chunks that load their K/V rows before the position is known
   // (LMX_ATTN_SPEC overrides; later chunks wait for the position and load
@@ -862,6 +869,12 @@ struct lmx_decoder {
   std::vector<void *> allocs;
   hipStream_t stream = nullptr;   // capture/replay stream of lmx_decoder_generate
 
+  int alloc_rows(float **p, size_t n) {   // uninitialised
+    const hipError_t e = hipMalloc(reinterpret_cast<void **>(p), n * sizeof(float));
+    if (e != hipSuccess) return hip_err(e, "hipMalloc (decoder)");
+    allocs.push_back(*p);
+    return LMX_OK;
+  }
   int alloc(void **p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) return hip_err(e, "hipMalloc (decoder)");
@@ -885,11 +898,29 @@ GemvArgs decode_args(const lmx_weight *w, int xmode, int epi) {
   return a;
 }
 
+// Whether one vector of this weight runs on the digit kernels (4 and 8 bits,
+// digit_linear's rule).
+bool one_on_digits(const lmx_weight *w) { return w->digit && w->d_codes; }
+
+// Whether every linear of the decoder can run on the digit kernels for any
+// number of rows.
+bool on_digits(const lmx_decoder *d) {
+  const auto ok = [](const lmx_weight *w) { return w->digit && w->d_digits; };
+  for (const lmx_decoder::Layer &L : d->layers)
+    if (!ok(L.qkv) || !ok(L.o) || !ok(L.gate_up) || !ok(L.down)) return false;
+  return ok(d->head);
+}
+
+// Whether the digit kernels form SiLU(gate)*up in the gate|up epilogue (whole
+// row tiles in each half).
+bool digit_pairs(const lmx_weight *gate_up) { return gate_up->rows % 32 == 0; }
+
 // The gate|up launch writes SiLU(gate)*up itself (kEpiSiluPair) where its
 // kernel plan serves that epilogue; else (or with LMX_SILU_PAIR=0) the down
 // projection forms it in its table prologue.
 bool gate_up_pairs(const lmx_weight *gate_up) {
   const char *e = std::getenv("LMX_SILU_PAIR");
+  if ((!e || std::atoi(e) != 0) && one_on_digits(gate_up) && digit_pairs(gate_up)) return true;
   return (!e || std::atoi(e) != 0) && silu_pair_rows(gate_up->format, decode_args(gate_up, kXModeRmsNorm, kEpiSiluPair)) > 0;
 }
 
@@ -908,29 +939,31 @@ int gemv(const lmx_weight *w, const float *x, float *y, const float *bias, int x
   a.xmode = xmode;
   a.xw = xw;
   a.eps = eps;
+  if (one_on_digits(w) && xmode != kXModeSiluMul) return launch_digit_gemv(w->format, a, 1, st);
   return launch_gemv(w->format, a, st);
 }
 
 
 template <int FMT>
 void launch_embed(const lmx_weight *w, const int *tokens, const int *pos, float *out, size_t batch, int tstride,
-                  hipStream_t st) {
-  embed_kernel<FMT><<<dim3(unsigned((w->cols + 255) / 256), unsigned(batch)), dim3(256), 0, st>>>(
+                  int T, int p0, hipStream_t st) {
+  embed_kernel<FMT><<<dim3(unsigned((w->cols + 255) / 256), unsigned(batch * size_t(T))), dim3(256), 0, st>>>(
       static_cast<const uint8_t *>(w->d_planes), w->d_scales, int(w->Npad), int(w->rows), int(w->n_groups),
-      int(w->group / kChunk), int(w->cols), tokens, pos, out, tstride);
+      int(w->group / kChunk), int(w->cols), tokens, pos, out, tstride, T, p0);
 }
 
-// Embedding rows of `batch` sequences (tokens of sequence b at tokens[b * tstride]).
-int embed(const lmx_weight *w, const int *tokens, const int *pos, float *out, size_t batch, int tstride,
+// Embedding rows of `batch` sequences (tokens of sequence b at tokens[b *
+// tstride]), T positions each from *pos, or from p0 where pos is null.
+int embed(const lmx_weight *w, const int *tokens, const int *pos, float *out, size_t batch, int tstride, int T, int p0,
           hipStream_t st) {
   switch (w->format) {
-  case LMX_FMT_TERNARY: launch_embed<LMX_FMT_TERNARY>(w, tokens, pos, out, batch, tstride, st); break;
-  case LMX_FMT_BINARY: launch_embed<LMX_FMT_BINARY>(w, tokens, pos, out, batch, tstride, st); break;
-  case LMX_FMT_RRQ2: launch_embed<LMX_FMT_RRQ2>(w, tokens, pos, out, batch, tstride, st); break;
-  case LMX_FMT_RRQ3: launch_embed<LMX_FMT_RRQ3>(w, tokens, pos, out, batch, tstride, st); break;
-  case LMX_FMT_INT3: launch_embed<LMX_FMT_INT3>(w, tokens, pos, out, batch, tstride, st); break;
-  case LMX_FMT_INT4: launch_embed<LMX_FMT_INT4>(w, tokens, pos, out, batch, tstride, st); break;
-  case LMX_FMT_INT8: launch_embed<LMX_FMT_INT8>(w, tokens, pos, out, batch, tstride, st); break;
+  case LMX_FMT_TERNARY: launch_embed<LMX_FMT_TERNARY>(w, tokens, pos, out, batch, tstride, T, p0, st); break;
+  case LMX_FMT_BINARY: launch_embed<LMX_FMT_BINARY>(w, tokens, pos, out, batch, tstride, T, p0, st); break;
+  case LMX_FMT_RRQ2: launch_embed<LMX_FMT_RRQ2>(w, tokens, pos, out, batch, tstride, T, p0, st); break;
+  case LMX_FMT_RRQ3: launch_embed<LMX_FMT_RRQ3>(w, tokens, pos, out, batch, tstride, T, p0, st); break;
+  case LMX_FMT_INT3: launch_embed<LMX_FMT_INT3>(w, tokens, pos, out, batch, tstride, T, p0, st); break;
+  case LMX_FMT_INT4: launch_embed<LMX_FMT_INT4>(w, tokens, pos, out, batch, tstride, T, p0, st); break;
+  case LMX_FMT_INT8: launch_embed<LMX_FMT_INT8>(w, tokens, pos, out, batch, tstride, T, p0, st); break;
   default: return fail(LMX_ERR_UNSUPPORTED_FORMAT, "embedding format %d", w->format);
   }
   return launch_err("embed");
@@ -1102,6 +1135,119 @@ int rmsnorm_rows(const lmx_decoder *d, const float *x, const float *wt, float *y
 
 int step_batched_rows(lmx_decoder *d, hipStream_t st);
 
+// y = W x' (+ bias) (+ resid) of `rows` rows on the digit kernels, x' the
+// RMSNorm of x with weight xw where given; epi kEpiSiluPair: SiLU(gate)*up.
+int digit_rows(const lmx_decoder *d, const lmx_weight *w, const float *x, float *y, size_t rows, const float *bias,
+               const float *resid, const float *xw, int epi, hipStream_t st) {
+  GemvArgs a = decode_args(w, xw ? kXModeRmsNorm : kXModeNone, epi);
+  a.bias = bias;
+  a.resid = resid;
+  a.xw = xw;
+  a.eps = d->cfg.rms_eps;
+  size_t done = 0;
+  const int r = digit_linear(w, a, x, y, rows, st, &done, true);
+  if (r) return r;
+  return done == rows ? LMX_OK : fail(LMX_ERR_INVALID_ARGUMENT, "digit rows covered %zu of %zu", done, rows);
+}
+
+// The MLP of `rows` rows in place: hidden += down(SiLU(gate) * up).
+int digit_mlp(const lmx_decoder *d, const lmx_decoder::Layer &L, float *hidden, float *gate_up, float *act, size_t rows,
+              hipStream_t st) {
+  const int ffn = int(d->cfg.ffn);
+  int r;
+  if (digit_pairs(L.gate_up)) {
+    if ((r = digit_rows(d, L.gate_up, hidden, act, rows, nullptr, nullptr, L.post_norm, kEpiSiluPair, st))) return r;
+  } else {
+    if ((r = digit_rows(d, L.gate_up, hidden, gate_up, rows, nullptr, nullptr, L.post_norm, kEpiStore, st))) return r;
+    silu_mul_rows_kernel<<<dim3(unsigned((ffn + 255) / 256), unsigned(rows)), dim3(256), 0, st>>>(gate_up, ffn, act);
+    if ((r = launch_err("silu_mul_rows"))) return r;
+  }
+  return digit_rows(d, L.down, act, hidden, rows, nullptr, hidden, nullptr, kEpiStore, st);
+}
+
+// Rows of one prompt pass: as many positions of every sequence as fill about
+// 512 rows, past which the linears' time grows with the rows.
+size_t prefill_rows(const lmx_decoder *d) {
+  return d->batch * std::min<size_t>(std::max<size_t>(512 / d->batch, 1), d->cfg.max_seq);
+}
+
+// Positions p0 .. p0 + T - 1 of every sequence into the KV cache, all linears
+// on T * batch rows at once.  The last layer stops at its cache: nothing
+// reads its output at these positions.
+int prefill_pass(lmx_decoder *d, int p0, int T, hipStream_t st) {
+  const lmx_decoder_config &c = d->cfg;
+  const size_t M = d->batch * size_t(T);
+  const int group = int(c.n_heads / c.n_kv_heads), hd = int(c.head_dim);
+  const size_t per_layer = attn_chunks(c) * kAttnChunk * c.n_kv_heads * c.head_dim;
+  const float scale = 1.0f / std::sqrt(float(c.head_dim));
+  int r = embed(d->embed, d->tokens, nullptr, d->p_hidden, d->batch, int(c.max_seq + 1), T, p0, st);
+  if (r) return r;
+  const dim3 rope_grid(unsigned(((c.n_heads + 2 * c.n_kv_heads) * (c.head_dim / 2) + 255) / 256), unsigned(M));
+  const dim3 attn_grid(unsigned((T * group + 15) / 16), unsigned(c.n_kv_heads), unsigned(d->batch));
+  for (size_t l = 0; l < c.n_layers; ++l) {
+    const lmx_decoder::Layer &L = d->layers[l];
+    float *kc = d->kcache + l * per_layer, *vc = d->vcache + l * per_layer;
+    if ((r = digit_rows(d, L.qkv, d->p_hidden, d->p_qkv, M, L.qkv_bias, nullptr, L.in_norm, kEpiStore, st))) return r;
+    if (hd == 64)
+      prefill_rope_kernel<64><<<rope_grid, dim3(256), 0, st>>>(d->p_qkv, d->rope, kc, vc, int(c.n_heads),
+                                                              int(c.n_kv_heads), T, p0, d->kv_seq);
+    else
+      prefill_rope_kernel<128><<<rope_grid, dim3(256), 0, st>>>(d->p_qkv, d->rope, kc, vc, int(c.n_heads),
+                                                               int(c.n_kv_heads), T, p0, d->kv_seq);
+    if ((r = launch_err("prefill_rope"))) return r;
+    if (l + 1 == c.n_layers) break;
+    if (hd == 64)
+      prefill_attention_kernel<64><<<attn_grid, dim3(256), 0, st>>>(d->p_qkv, kc, vc, int(c.n_heads),
+                                                                   int(c.n_kv_heads), T, p0, scale, d->kv_seq, d->p_attn);
+    else
+      prefill_attention_kernel<128><<<attn_grid, dim3(256), 0, st>>>(
+          d->p_qkv, kc, vc, int(c.n_heads), int(c.n_kv_heads), T, p0, scale, d->kv_seq, d->p_attn);
+    if ((r = launch_err("prefill_attention")) ||
+        (r = digit_rows(d, L.o, d->p_attn, d->p_hidden, M, nullptr, d->p_hidden, nullptr, kEpiStore, st)) ||
+        (r = digit_mlp(d, L, d->p_hidden, d->p_gate_up, d->p_act, M, st)))
+      return r;
+  }
+  return LMX_OK;
+}
+
+// The prompt's first n positions in passes, then the position and (one
+// sequence) its embedding set for the steps from position n on.
+int prefill(lmx_decoder *d, size_t n, hipStream_t st) {
+  const lmx_decoder_config &c = d->cfg;
+  const size_t rows = prefill_rows(d), T = rows / d->batch;
+  int r;
+  if (!d->p_hidden) {
+    bool pairs = true;
+    for (const lmx_decoder::Layer &L : d->layers) pairs = pairs && digit_pairs(L.gate_up);
+    if ((r = d->alloc_rows(&d->p_qkv, rows * (c.n_heads + 2 * c.n_kv_heads) * c.head_dim)) ||
+        (r = d->alloc_rows(&d->p_attn, rows * c.n_heads * c.head_dim)) ||
+        (!pairs && (r = d->alloc_rows(&d->p_gate_up, rows * 2 * c.ffn))) ||
+        (r = d->alloc_rows(&d->p_act, rows * c.ffn)) || (r = d->alloc_rows(&d->p_hidden, rows * c.hidden)))
+      return r;
+  }
+  for (size_t p = 0; p < n; p += T)
+    if ((r = prefill_pass(d, int(p), int(std::min(T, n - p)), st))) return r;
+  d->prompt_pos = int(n);
+  const hipError_t e = hipMemcpyAsync(d->pos, &d->prompt_pos, sizeof(int), hipMemcpyHostToDevice, st);
+  if (e != hipSuccess) return hip_err(e, "decoder position");
+  return d->batch == 1 ? embed(d->embed, d->tokens, d->pos, d->hidden, 1, int(c.max_seq + 1), 1, 0, st) : LMX_OK;
+}
+
+// The layers of a batched step on the digit kernels, and the logits.
+int step_batched_digits(lmx_decoder *d, float *lg, hipStream_t st) {
+  const lmx_decoder_config &c = d->cfg;
+  int r;
+  for (size_t l = 0; l < c.n_layers; ++l) {
+    const lmx_decoder::Layer &L = d->layers[l];
+    if ((r = digit_rows(d, L.qkv, d->hidden, d->qkv, d->batch, L.qkv_bias, nullptr, L.in_norm, kEpiStore, st)) ||
+        (r = attention(d, l, st)) ||
+        (r = digit_rows(d, L.o, d->attn_out, d->hidden, d->batch, nullptr, d->hidden, nullptr, kEpiStore, st)) ||
+        (r = digit_mlp(d, L, d->hidden, d->gate_up, d->act, d->batch, st)))
+      return r;
+  }
+  return digit_rows(d, d->head, d->hidden, lg, d->batch, nullptr, nullptr, d->final_norm, kEpiStore, st);
+}
+
 // Four rows of one linear in one group (the four-vector kernel where the
 // plan has it, else the batched kernel): y = W x' (+ bias) (+ resid), x' the
 // RMSNorm of x with weight xw when xmode asks.
@@ -1142,11 +1288,13 @@ bool quad_step(const lmx_decoder *d) {
 int step_batched(lmx_decoder *d, float *logits_out, hipStream_t st) {
   const lmx_decoder_config &c = d->cfg;
   const size_t B = d->batch;
-  int r = embed(d->embed, d->tokens, d->pos, d->hidden, B, int(c.max_seq + 1), st);
+  int r = embed(d->embed, d->tokens, d->pos, d->hidden, B, int(c.max_seq + 1), 1, 0, st);
   if (r) return r;
   float *lg = logits_out ? logits_out : d->logits;
-  const bool quad = quad_step(d);
-  if (quad) {
+  const bool digits = on_digits(d), quad = !digits && quad_step(d);
+  if (digits) {
+    if ((r = step_batched_digits(d, lg, st))) return r;
+  } else if (quad) {
     // qkv: RMSNorm in the table build; o: + hidden in the epilogue; gate|up:
     // RMSNorm in the batched table build, SiLU(gate)*up in its reduction;
     // down: + hidden in its reduction; the head normalises its own input.
@@ -1188,7 +1336,7 @@ int step_batched(lmx_decoder *d, float *logits_out, hipStream_t st) {
     if ((r = step_batched_rows(d, st))) return r;
     if ((r = rmsnorm_rows(d, d->hidden, d->final_norm, d->normed, st))) return r;
   }
-  if (!quad && (r = gemv_rows(d, d->head, d->normed, lg, nullptr, nullptr, st))) return r;
+  if (!quad && !digits && (r = gemv_rows(d, d->head, d->normed, lg, nullptr, nullptr, st))) return r;
   // parts per row: about 256 workgroups in all (LMX_ARGMAX_PARTS overrides)
   const char *ap = std::getenv("LMX_ARGMAX_PARTS");
   const int parts = std::max(1, std::min(kArgmaxParts, ap ? std::atoi(ap) : int(256 / B)));
@@ -1271,7 +1419,7 @@ int set_position(lmx_decoder *d, const int32_t *tokens, size_t n, hipStream_t st
   if (e == hipSuccess) e = hipMemcpyAsync(d->pos, &zero, sizeof(int), hipMemcpyHostToDevice, st);
   if (e != hipSuccess) return hip_err(e, "decoder reset");
   if (d->batch == 1) {   // a batch-1 step starts from the embedding of the token at its position
-    const int r = embed(d->embed, d->tokens, d->pos, d->hidden, 1, int(d->cfg.max_seq + 1), st);
+    const int r = embed(d->embed, d->tokens, d->pos, d->hidden, 1, int(d->cfg.max_seq + 1), 1, 0, st);
     if (r) return r;
   }
   std::vector<unsigned> hist;   // the penalty's history starts as the whole prompt (inference.cpp:264-268)
@@ -1421,7 +1569,7 @@ int lmx_decoder_set_head(lmx_decoder *d, const lmx_weight *embed, const lmx_weig
   if (embed->device != d->device || head->device != d->device)
     return fail(LMX_ERR_INVALID_ARGUMENT, "weight on another device");
   if ((st = upload(d, &d->final_norm, final_norm, d->cfg.hidden))) return st;
-  const size_t slots = gemv_argmax_slots(weight_args(head));
+  const size_t slots = one_on_digits(head) ? digit_argmax_slots(weight_args(head)) : gemv_argmax_slots(weight_args(head));
   if ((st = d->alloc(reinterpret_cast<void **>(&d->amax), slots * sizeof(unsigned long long)))) return st;
   d->amax_slots = slots;
   d->embed = embed;
@@ -1489,10 +1637,17 @@ int lmx_decoder_generate(lmx_decoder *d, const int32_t *prompt, size_t n_prompt,
     if (dep) (void)hipEventDestroy(dep);
     if (e0 != hipSuccess) return hip_err(e0, "decoder stream ordering");
   }
-  // One eager step (first-launch set-up of every kernel), then capture.
-  if ((st = set_position(d, prompt, n_prompt, s)) || (st = step(d, nullptr, s))) return st;
-  hipError_t e = hipStreamSynchronize(s);
-  if (e != hipSuccess) return hip_err(e, "decoder warm-up step");
+  // The decoder's first generation runs one eager step (first-launch set-up
+  // of every kernel) before it captures.
+  hipError_t e = hipSuccess;
+  if ((st = set_position(d, prompt, n_prompt, s))) return st;
+  if (!d->warm) {
+    if ((st = step(d, nullptr, s))) return st;
+    e = hipStreamSynchronize(s);
+    if (e != hipSuccess) return hip_err(e, "decoder warm-up step");
+    if ((st = set_position(d, prompt, n_prompt, s))) return st;
+    d->warm = true;
+  }
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
@@ -1510,9 +1665,15 @@ int lmx_decoder_generate(lmx_decoder *d, const int32_t *prompt, size_t n_prompt,
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
   for (auto &x : ev)
     if (e == hipSuccess) e = hipEventCreate(&x);
-  if (e == hipSuccess && (st = set_position(d, prompt, n_prompt, s)) != LMX_OK) e = hipErrorUnknown;
   if (e == hipSuccess) e = hipEventRecord(ev[0], s);
-  for (size_t i = 0; i < n_prompt && e == hipSuccess; ++i) e = hipGraphLaunch(exec, s);
+  // All but the prompt's last position in passes of many rows; a pass costs
+  // about as much as three steps, so a shorter prompt takes steps.
+  size_t passed = 0;
+  if (e == hipSuccess && n_prompt > 4 && on_digits(d)) {
+    passed = n_prompt - 1;
+    if ((st = prefill(d, passed, s)) != LMX_OK) e = hipErrorUnknown;
+  }
+  for (size_t i = passed; i < n_prompt && e == hipSuccess; ++i) e = hipGraphLaunch(exec, s);
   if (e == hipSuccess) e = hipEventRecord(ev[1], s);
   for (size_t i = 1; i < n_new && e == hipSuccess; ++i) e = hipGraphLaunch(exec, s);
   if (e == hipSuccess) e = hipEventRecord(ev[2], s);

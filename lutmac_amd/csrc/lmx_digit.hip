@@ -158,6 +158,8 @@ __global__ __launch_bounds__(256) void digit_split_chunks_kernel(const float *__
 // 12.0 / 8.0).
 int digit_gemv_tiles(const GemvArgs &a) { return a.epi == kEpiSiluPair || a.Npad / kTile >= 512 ? 2 : 1; }
 
+size_t digit_argmax_slots(const GemvArgs &a) { return size_t(a.Npad) / (kTile * digit_gemv_tiles(a)); }
+
 int launch_digit_gemv(int fmt, const GemvArgs &a, int nv, void *stream) {
   switch (fmt) {
   case LMX_FMT_TERNARY: return digit_gemv_fmt<LMX_FMT_TERNARY>(a, nv, stream);

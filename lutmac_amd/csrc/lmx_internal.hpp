@@ -237,6 +237,7 @@ int launch_digit_gemm(int fmt, const GemvArgs &a, const DigitVectors &d, void *s
 // 1..4 vectors in one launch, with transform a.xmode and epilogue a.epi
 // (argmax keys, one slot per workgroup, for one vector)
 int launch_digit_gemv(int fmt, const GemvArgs &a, int nv, void *stream);
+size_t digit_argmax_slots(const GemvArgs &a);   // argmax key slots of that launch
 int digit_gemv_tiles(const GemvArgs &a);   // 16-row tiles per workgroup of that launch
 // 4- and 8-bit codes laid out for the matrix-core operands, made from the
 // plane tiles on the device: [Kp/128][Npad][4 plane words][4 or 8 words];
@@ -303,9 +304,11 @@ GemvArgs weight_args(const lmx_weight *w);
 // below 4).
 int gemv_batched(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream,
                  size_t *done);
-// y = W x of `batch` vectors on the digit kernels (a.bias, a.resid, a.rotate; x of any alignment);
-// *done = the vectors covered, the rest (one by one on the lookup tables) left to the caller
-int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done);
+// y = W x of `batch` vectors on the digit kernels (a.bias, a.resid, a.rotate, a.xmode none or RMSNorm,
+// a.epi store or SiLU pair; x of any alignment); *done = the vectors covered, the rest (one by one on
+// the lookup tables) left to the caller unless `all`
+int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done,
+                 bool all);
 // Whether gemv_batched serves epilogue epi (kEpi*) for `batch` vectors of w
 // with no vector left to the single-vector path (x 16-byte aligned assumed).
 bool batched_epilogue_ok(const lmx_weight *w, int epi, size_t batch);

@@ -1,0 +1,58 @@
+"""Prompt passes (many positions at once) against the same prompt taken one
+position a step: the logits of the position after the prompt, from a cache
+that the passes filled and from one that the steps filled."""
+import numpy as np
+import pytest
+import torch
+
+import lutmac_amd as L
+from conftest import rel_max_err
+from lutmac_amd import decode as D
+
+pytestmark = pytest.mark.gpu
+
+# Both forms are fp32 sums of the same terms in other orders; the bound is the
+# decoder tests' own against the oracle.
+DECODE_TOL = 1e-5
+
+
+def both(model, batch, prompt):
+    """Logits [batch, vocab] after the prompt: passes, then steps."""
+    n = prompt.shape[1]
+    dec = D.Decoder(model, batch=batch)
+    p = prompt if batch > 1 else prompt[0]
+    out, _, _ = dec.generate(p, 2)
+    vocab = model.cfg.vocab
+    a, b = (torch.empty(batch * vocab, device="cuda") for _ in range(2))
+    dec.step(a)
+    toks = np.asarray(out).reshape(batch, n + 2)
+    dec.reset(toks if batch > 1 else toks[0])
+    for _ in range(n + 2):
+        dec.step(b)
+    torch.cuda.synchronize()
+    dec.close()
+    return a.cpu().numpy().reshape(batch, vocab), b.cpu().numpy().reshape(batch, vocab)
+
+
+# Prompt lengths: the shortest that takes a pass, one and more 16-row query
+# tiles (16 / group positions each), past a 64-position cache chunk, and, with
+# 512 rows a pass, several passes; heads with 1, 4 and 6 queries per key head;
+# ffn 264 (no whole row tiles per half) leaves SiLU(gate)*up to a kernel of its
+# own, there with every family of formats among the linears.
+@pytest.mark.parametrize("batch,n", [(1, 5), (1, 17), (1, 130), (3, 65), (16, 70), (1, 700)])
+@pytest.mark.parametrize("heads,kv,hd,ffn", [(8, 2, 64, 512), (6, 1, 128, 264), (4, 4, 64, 512)])
+def test_prompt_passes(cuda, batch, n, heads, kv, hd, ffn):
+    cfg = D.small_config(n_heads=heads, n_kv_heads=kv, head_dim=hd, ffn=ffn, max_seq=n + 4, vocab=515,
+                         qkv_bias=kv == 4)
+    model = quantized(cfg) if ffn == 264 else D.SyntheticModel(cfg, seed=n + heads, group=128, random_norms=True)
+    prompt = np.random.default_rng(n).integers(0, cfg.vocab, (batch, n)).astype(np.int32)
+    passes, steps = both(model, batch, prompt)
+    for b in range(batch):
+        assert rel_max_err(passes[b], steps[b]) < DECODE_TOL, b
+
+
+def quantized(cfg):
+    return D.QuantizedModel(cfg, {"q": (L.FMT_TERNARY, 128, 0), "k": (L.FMT_TERNARY, 128, 0),
+                                  "v": (L.FMT_TERNARY, 128, 0), "o": (L.FMT_RRQ2, 128, L.QUANT_RESIDUAL),
+                                  "gate": (L.FMT_INT8, 256, 0), "up": (L.FMT_INT8, 256, 0),
+                                  "down": (L.FMT_BINARY, 128, 0), "embed": (L.FMT_INT4, 128, 0)}, seed=4)
