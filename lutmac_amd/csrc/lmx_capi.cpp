@@ -142,7 +142,6 @@ int choose_reduce() {
 }  // namespace
 
 int plane_split_level() { return env_int("LMX_PS", 1); }
-int mfma_batched() { return env_int("LMX_MFMA", 1); }
 
 void plan_weight(lmx_weight *w, int fmt, size_t rows, size_t cols, size_t group) {
   FormatInfo fi;
@@ -165,8 +164,8 @@ void plan_weight(lmx_weight *w, int fmt, size_t rows, size_t cols, size_t group)
   }
   w->fullk = choose_fullk(fmt, w->Npad, w->Kp, w->kfamily);
   w->staged = choose_staged();
-  w->batched = env_int("LMX_BATCHED", 1) != 0;
-  // The digit kernels, unless a lookup-table plan was asked for.
+  // One vector of 4 or 8 bits on the digit kernels, unless a lookup-table plan
+  // was asked for.
   w->digit = env_int("LMX_DIGIT", 1) != 0;
   for (const char *name : {"LMX_FULLK", "LMX_KERNEL", "LMX_KSLICE", "LMX_REDUCE", "LMX_WAVES"})
     if (std::getenv(name)) w->digit = false;
@@ -178,7 +177,6 @@ void free_weight(lmx_weight *w) {
   if (!w) return;
   if (w->d_weight) (void)hipFree(w->d_weight);
   if (w->d_scratch) (void)hipFree(w->d_scratch);
-  if (w->d_nib) (void)hipFree(w->d_nib);
   delete w;
 }
 
@@ -215,21 +213,15 @@ int upload(int fmt, size_t rows, size_t cols, size_t group, const uint8_t *plane
   // scratch of its calls, allocated here so that no call allocates (graph
   // capture stays possible).
   const auto align = [](size_t n) { return round_up(n, 256); };
-  const size_t code_bytes = w->digit ? code_copy_bytes(fmt, w->Npad, w->Kp) : 0;
+  const size_t code_bytes = code_copy_bytes(fmt, w->Npad, w->Kp);
   // enough counters for any waves-per-group choice and any sliced rows launch
   const size_t counter_bytes = std::max<size_t>(w->Npad / kWave, kDigitTickets) * sizeof(unsigned);
-  // split-K partials of one vector; with batches those of the largest group
-  // (16; 128-wide k-slices, twice the splits, where 256-wide ones give the
-  // batched kernel less than a workgroup per CU), and the digits of 256
-  // vectors (512 of a long K, where two launches cost most), more where the
-  // matrix has the rows to make one launch of them worth it.  One call uses
-  // one of them at a time.
-  size_t work_bytes = w->Kp / kRotChunk * w->Npad * sizeof(float);
-  if (w->batched) {
-    const size_t vectors = std::min<size_t>(std::max<size_t>(w->Npad / 16, w->Kp > 4096 ? 512 : 256), 1024);
-    work_bytes = std::max(16 * batched_slice_splits(w->Npad, w->Kp) * w->Npad * sizeof(float),
-                          digit_bytes(w->Kp, vectors) + kDigitPartials);
-  }
+  // the split-K partials of one vector, or the digits of 256 vectors (512 of a
+  // long K, where two launches cost most), more where the matrix has the rows
+  // to make one launch of them worth it: one call uses one of them at a time
+  const size_t vectors = std::min<size_t>(std::max<size_t>(w->Npad / 16, w->Kp > 4096 ? 512 : 256), 1024);
+  const size_t work_bytes = std::max(w->Kp / kRotChunk * w->Npad * sizeof(float),
+                                     digit_bytes(w->Kp, vectors) + kDigitPartials);
   char *base = nullptr;
   hipError_t e;
   if ((e = hipMalloc(&w->d_weight, align(w->tile_bytes) + align(code_bytes) + w->scale_bytes)) != hipSuccess ||
@@ -245,29 +237,8 @@ int upload(int fmt, size_t rows, size_t cols, size_t group, const uint8_t *plane
   w->d_counters = reinterpret_cast<unsigned *>(base);
   w->d_xrot = reinterpret_cast<float *>(base + align(counter_bytes));
   w->d_partials = reinterpret_cast<float *>(base + align(counter_bytes) + align(w->Kp * sizeof(float)));
-  if (w->batched) {
-    w->d_bpartials = w->d_partials;
-    w->bpartials_cap = work_bytes / sizeof(float);
-    w->d_digits = w->d_partials;
-    w->digit_cap = work_bytes;
-    // 4-bit: the codes once more in the matrix-core kernel's layout (groups
-    // of 4, 8 and 16 vectors; the same 4 bits per weight as the planes)
-    if (fmt == LMX_FMT_INT4 && mfma_batched()) {
-      std::vector<uint8_t> nib;
-      try {
-        nib.resize(w->Kp * w->Npad / 2);
-      } catch (const std::bad_alloc &) {
-        free_weight(w);
-        return fail(LMX_ERR_OUT_OF_MEMORY, "host staging allocation failed");
-      }
-      nibble_tiles(planes, rows, row_bytes, w->Npad, w->Kp, nib.data());
-      if ((e = hipMalloc(&w->d_nib, nib.size())) != hipSuccess ||
-          (e = hipMemcpy(w->d_nib, nib.data(), nib.size(), hipMemcpyHostToDevice)) != hipSuccess) {
-        free_weight(w);
-        return hip_fail(e, "hipMalloc (matrix-core codes)");
-      }
-    }
-  }
+  w->d_digits = w->d_partials;
+  w->digit_cap = work_bytes;
   if ((e = hipMemcpy(w->d_planes, tiles.data(), w->tile_bytes, hipMemcpyHostToDevice)) != hipSuccess) {
     free_weight(w);
     return hip_fail(e, "upload (weight)");
@@ -312,49 +283,6 @@ int stage_if_needed(const lmx_weight *w, GemvArgs &a, void *stream) {
 
 }  // namespace
 
-// Batched vectors in groups of 16/8/4 through the batched kernel (weights
-// read once per group; below 4 vectors one GEMV per vector is faster), a
-// group of 4 through the four-vector full-K kernel where the handle's plan
-// has one; returns the number of vectors done.  Needs x
-// 16-byte aligned with cols % 4 == 0 (every vector then is).  Uses the
-// handle's batched partials, allocated with the handle.
-int gemv_batched(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream,
-                 size_t *done) {
-  *done = 0;
-  if (a.epi != kEpiStore && !batched_epilogue_ok(w, a.epi, batch))
-    return fail(LMX_ERR_INVALID_ARGUMENT, "batched epilogue %d does not cover %zu vectors of a %zu x %zu weight", a.epi,
-                batch, w->rows, w->cols);
-  if (!w->batched || batch < 4 || reinterpret_cast<size_t>(x) % 16 || w->cols % 4) return LMX_OK;
-  const float *resid = a.resid;  // [batch][rows] residual rows, offset with the vectors
-  float *y2 = a.y2;               // kEpiNormOut: [batch][rows]
-  const size_t out_rows = a.epi == kEpiSiluPair ? w->rows / 2 : w->rows;
-  while (batch - *done >= 4) {
-    const size_t left = batch - *done;
-    const int nb = left >= 16 ? 16 : left >= 8 ? 8 : 4;
-    if (size_t(nb) * batched_slice_splits(w->Npad, w->Kp) * w->Npad > w->bpartials_cap)
-      return fail(LMX_ERR_INVALID_ARGUMENT, "batched partials of %zu floats hold no group of %d", w->bpartials_cap, nb);
-    a.x = x + *done * w->cols;
-    a.y = y + *done * out_rows;
-    a.y2 = y2 ? y2 + *done * w->rows : nullptr;
-    a.resid = resid ? resid + *done * w->rows : nullptr;
-    a.cols = int(w->cols);
-    a.partials = w->d_bpartials;
-    a.nib = w->d_nib;
-    if (nb == 4 && a.epi != kEpiNormOut && a.epi != kEpiPartials) {   // one full-K launch where the plan allows
-      const int q = launch_gemv_quad(w->format, a, stream);
-      if (q != 1) {
-        if (q) return q;
-        *done += 4;
-        continue;
-      }
-    }
-    int st = launch_gemv_batch(w->format, a, nb, stream);   // RMSNorm in groups of 4 only
-    if (st) return st;
-    *done += size_t(nb);
-  }
-  return LMX_OK;
-}
-
 // y = W x of `batch` vectors on the digit kernels: up to 4 in one launch,
 // more through digits split into the handle's scratch.  One vector of a 1-3
 // bit format stays on the lookup tables, whose planes are half to an eighth of
@@ -387,20 +315,13 @@ int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size
       if ((st = launch_digit_split(w->format, a, d, stream)) || (st = launch_digit_gemm(w->format, a, d, stream)))
         return st;
     } else {
-      if (!copies && !all && (left == 1 || w->Kp > 4096)) return LMX_OK;   // one by one on the lookup tables
+      // one by one on the lookup tables
+      if (!all && (left == 1 ? !copies || !w->digit : !copies && w->Kp > 4096)) return LMX_OK;
       if ((st = launch_digit_gemv(w->format, a, int(n), stream))) return st;
     }
     *done += n;
   }
   return LMX_OK;
-}
-
-bool batched_epilogue_ok(const lmx_weight *w, int epi, size_t batch) {
-  if (!w->batched || batch < 4 || batch % 4 || w->cols % 4) return false;   // every vector in a group of 16/8/4
-  if (epi == kEpiSiluPair) return w->rows % 8 == 0;
-  if (epi == kEpiNormOut) return w->rows <= size_t(kNormOutMaxRows);
-  if (epi == kEpiPartials) return batch == 4 || batch == 8 || batch == 16;   // one group: one set of partials
-  return epi == kEpiStore;
 }
 
 GemvArgs weight_args(const lmx_weight *w) {
@@ -654,8 +575,7 @@ int gemv_impl(const lmx_weight *w, const float *x, float *y, size_t batch, unsig
   size_t b0 = 0;
   if (flags != LMX_ROTATE_FWHT_FULL) {
     a.rotate = flags == LMX_ROTATE_FWHT256 ? LMX_ROTATE_FWHT256 : LMX_ROTATE_NONE;
-    if ((st = w->digit ? digit_linear(w, a, x, y, batch, stream, &b0, false) : gemv_batched(w, a, x, y, batch, stream, &b0)))
-      return st;
+    if ((st = digit_linear(w, a, x, y, batch, stream, &b0, false))) return st;
   }
   for (size_t b = b0; b < batch; ++b) {
     a.x = x + b * w->cols;
@@ -690,8 +610,7 @@ int lmx_linear(const lmx_weight *w, const float *bias, const float *x, float *y,
   a.bias = bias;
   a.rotate = rotate ? LMX_ROTATE_FWHT256 : LMX_ROTATE_NONE;
   size_t b0 = 0;
-  if ((st = w->digit ? digit_linear(w, a, x, y, batch, stream, &b0, false) : gemv_batched(w, a, x, y, batch, stream, &b0)))
-    return st;
+  if ((st = digit_linear(w, a, x, y, batch, stream, &b0, false))) return st;
   for (size_t b = b0; b < batch; ++b) {
     a.x = x + b * w->cols;
     a.y = y + b * w->rows;

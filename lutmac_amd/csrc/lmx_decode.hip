@@ -26,8 +26,8 @@
 //   finish_embed_kernel    maximum of the keys -> next token, position + 1,
 //                          and the next token's embedding into the hidden state
 // (Batches of sequences start each step with embed_kernel and finish with
-// argmax_rows_kernel; their linears run the batched GEMV, whose reductions
-// also write the normed rows and SiLU(gate)*up, see step_batched.)
+// argmax_rows_kernel; their linears run on the digit kernels, as do those of
+// the passes that take many positions of a prompt at once, lmx_prefill.hpp.)
 // The position and the token sequence live in device memory, so the same
 // captured step replays for every position.
 #include <hip/hip_runtime.h>
@@ -107,23 +107,6 @@ __global__ __launch_bounds__(256) void embed_kernel(const uint8_t *__restrict__ 
   out[k] = weight_value<FMT>(b, s);
 }
 
-// Batched decode helpers (one workgroup per sequence row).
-// y[b] = x[b] * inv_rms(x[b]) * w, inv_rms = 1/sqrt(sum x^2 / n + eps)
-// (norm.cpp:18-34).
-__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                                           int n, float eps, float *__restrict__ y) {
-  __shared__ float red[4];
-  x += size_t(blockIdx.x) * n;
-  y += size_t(blockIdx.x) * n;
-  float s = 0.0f;
-  for (int k = threadIdx.x; k < n; k += 256) s += x[k] * x[k];
-  s = lane_sum<32>(s, threadIdx.x & (kWave - 1));
-  if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = s;
-  __syncthreads();
-  const float inv = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / float(n) + eps);
-  for (int k = threadIdx.x; k < n; k += 256) y[k] = x[k] * inv * w[k];
-}
-
 // act[b][k] = silu(gu[b][k]) * gu[b][ffn + k] (model.cpp:36, 413-416).
 __global__ __launch_bounds__(256) void silu_mul_rows_kernel(const float *__restrict__ gu, int ffn,
                                                             float *__restrict__ act) {
@@ -137,7 +120,6 @@ __global__ __launch_bounds__(256) void silu_mul_rows_kernel(const float *__restr
 constexpr int kArgmaxParts = 32;   // most workgroups per logits row
 constexpr int kAttnMaxSplit = 8;   // most workgroups sharing one KV head's query heads
 constexpr int kTicketPad = 32;     // unsigneds per ticket (attention, greedy pick): one 128-byte line each
-constexpr int kAttnMaxParts = 16;  // most q|k|v split partials attention sums itself
 
 // Greedy token of every sequence: the first maximum of its logits row
 // (model.cpp:480-490); written unless the next position is forced.  Each
@@ -517,12 +499,7 @@ __device__ __forceinline__ void chunk_attend(const float (*ks)[HD + 4], const fl
 // speculatively, before the position is known; later units read the
 // position first and, when it lies before them, load nothing and take no
 // ticket (the merge reads units up to the position only).
-// PARTS: the q|k|v rows arrive as the batched GEMV's split partials
-// qparts [batch][qsplits][qnpad] (no reduction launch before attention); the
-// workgroup sums the rows it needs in split order (+ qbias), exactly as the
-// batched reduction would, into LDS, loading them in the same round trip as
-// the unit's K and V rows.
-template <int HD, int CPW, bool PARTS>
+template <int HD, int CPW>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void attn_kernel(const float *__restrict__ qkv, float *__restrict__ kc,
                                                    float *__restrict__ vc, const int *__restrict__ pos_p,
                                                    const float2 *__restrict__ rope, int n_heads,
@@ -530,8 +507,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void a
                                                    float *__restrict__ part, int n_chunks,
                                                    unsigned *__restrict__ tickets, float *__restrict__ out,
                                                    size_t qkv_stride, size_t kv_stride, int spec_units,
-                                                   int hsplit, const float *__restrict__ qparts, int qsplits,
-                                                   int qnpad, const float *__restrict__ qbias) {
+                                                   int hsplit) {
   constexpr int VD = HD / kWave;          // value columns per lane
   constexpr int NT = 512;
   constexpr int KV4 = kAttnChunk * HD / 4 / NT;   // float4 of K (and of V) per thread and chunk
@@ -542,7 +518,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void a
   __shared__ float qs[8][HD];
   __shared__ float pw[8][kAttnChunk];
   __shared__ float knew[HD];
-  __shared__ float qkvb[PARTS ? (8 + 2) * HD : 1];   // PARTS: the summed q (up to 8 heads), k and v rows
   __shared__ unsigned ticket;
   // Every argument in SGPRs before the first wait: their loads then take one
   // round trip (left to the compiler they came in three batches, each waited
@@ -550,14 +525,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void a
   asm volatile("" ::"s"(qkv), "s"(kc), "s"(vc), "s"(pos_p), "s"(rope), "s"(part), "s"(tickets), "s"(out));
   asm volatile("" ::"s"(n_heads), "s"(n_kv), "s"(group), "s"(max_seq), "s"(scale), "s"(n_chunks), "s"(qkv_stride),
                "s"(kv_stride), "s"(spec_units), "s"(hsplit));
-  if constexpr (PARTS) asm volatile("" ::"s"(qparts), "s"(qsplits), "s"(qnpad), "s"(qbias));
   __builtin_amdgcn_sched_barrier(0);
   {
     // sequence blockIdx.y of a batch: its q|k|v row, KV cache, partials,
     // tickets and output (the position is shared)
     const size_t b = blockIdx.y;
     qkv += b * qkv_stride;
-    if constexpr (PARTS) qparts += b * size_t(qsplits) * size_t(qnpad);
     kc += b * kv_stride;
     vc += b * kv_stride;
     part += b * size_t(n_heads) * n_chunks * (HD + 4);
@@ -620,36 +593,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void a
   const float *qin = qkv + size_t(h0 + (wave < hpw ? wave : 0)) * HD;
   float qa[RP], qb[RP], ka[RP], kb[RP], vn[VD];
   float2 rt[RP];   // (cos, sin) of the position's rotation angles
-  // PARTS: value i < nval of the workgroup's q (hpw heads), k, v rows; thread
-  // t sums values t, t + NT, ... (VPT of them) over the splits
-  constexpr int VPT = PARTS ? ((8 + 2) * HD + NT - 1) / NT : 1;
-  constexpr int NP = PARTS ? kAttnMaxParts : 1;
-  const int nq = hpw * HD, nval = nq + 2 * HD;
-  const auto qkv_row = [&](int i) {   // value i -> its row of the fused q|k|v output
-    return i < nq ? h0 * HD + i : i < nq + HD ? (n_heads + kvh) * HD + (i - nq) : (n_heads + n_kv + kvh) * HD + (i - nq - HD);
-  };
-  float pv[VPT][NP], pb[VPT];
-  if constexpr (PARTS) {
 #pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-      const int r = qkv_row(min(int(threadIdx.x) + j * NT, nval - 1));
-#pragma unroll
-      for (int t = 0; t < NP; ++t) pv[j][t] = t < qsplits ? qparts[size_t(t) * qnpad + r] : 0.0f;
-      pb[j] = qbias ? qbias[r] : 0.0f;
-    }
+  for (int i = 0; i < RP; ++i) {
+    const int d = min(lane + i * kWave, HALF - 1);
+    qa[i] = qin[d];
+    qb[i] = qin[d + HALF];
+    ka[i] = kin[d];
+    kb[i] = kin[d + HALF];
   }
-  if constexpr (!PARTS) {
 #pragma unroll
-    for (int i = 0; i < RP; ++i) {
-      const int d = min(lane + i * kWave, HALF - 1);
-      qa[i] = qin[d];
-      qb[i] = qin[d + HALF];
-      ka[i] = kin[d];
-      kb[i] = kin[d + HALF];
-    }
-#pragma unroll
-    for (int u = 0; u < VD; ++u) vn[u] = vin[u * kWave + lane];
-  }
+  for (int u = 0; u < VD; ++u) vn[u] = vin[u * kWave + lane];
   __builtin_amdgcn_sched_barrier(0);
   pos = min(__builtin_amdgcn_readfirstlane(praw), max_seq - 1);
 #pragma unroll
@@ -660,48 +613,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void a
   for (int i = 0; i < KV4; ++i)
     asm volatile("" ::"v"(kr[i].x), "v"(kr[i].y), "v"(kr[i].z), "v"(kr[i].w), "v"(vr[i].x), "v"(vr[i].y),
                  "v"(vr[i].z), "v"(vr[i].w));
-  if constexpr (PARTS) {
 #pragma unroll
-    for (int i = 0; i < RP; ++i) asm volatile("" ::"v"(rt[i].x), "v"(rt[i].y));
+  for (int i = 0; i < RP; ++i)
+    asm volatile("" ::"v"(rt[i].x), "v"(rt[i].y), "v"(qa[i]), "v"(qb[i]), "v"(ka[i]), "v"(kb[i]));
 #pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-#pragma unroll
-      for (int t = 0; t < NP; ++t) asm volatile("" ::"v"(pv[j][t]));
-      asm volatile("" ::"v"(pb[j]));
-    }
-    // split-order sums (+ bias), the batched reduction's expression: one
-    // round of 16 partials from zero, absent splits adding +0
-#pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-      const int i = int(threadIdx.x) + j * NT;
-      float sum = 0.0f;
-#pragma unroll
-      for (int t = 0; t < NP; ++t) sum += pv[j][t];
-      if (qbias) sum += pb[j];
-      if (i < nval) qkvb[i] = sum;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < RP; ++i)
-      asm volatile("" ::"v"(rt[i].x), "v"(rt[i].y), "v"(qa[i]), "v"(qb[i]), "v"(ka[i]), "v"(kb[i]));
-#pragma unroll
-    for (int u = 0; u < VD; ++u) asm volatile("" ::"v"(vn[u]));
-  }
+  for (int u = 0; u < VD; ++u) asm volatile("" ::"v"(vn[u]));
   store_rows();   // the first chunk's rows
-  if constexpr (PARTS) {
-    __syncthreads();   // the summed rows are in qkvb
-    const float *qsrc = qkvb + (wave < hpw ? wave : 0) * HD;
-#pragma unroll
-    for (int i = 0; i < RP; ++i) {
-      const int d = min(lane + i * kWave, HALF - 1);
-      qa[i] = qsrc[d];
-      qb[i] = qsrc[d + HALF];
-      ka[i] = qkvb[nq + d];
-      kb[i] = qkvb[nq + d + HALF];
-    }
-#pragma unroll
-    for (int u = 0; u < VD; ++u) vn[u] = qkvb[nq + HD + u * kWave + lane];
-  }
   const bool live = t0 <= pos;                      // the unit holds positions of the sequence
   const bool own = pos / UNIT == unit;              // the unit holds the new position
   // RoPE: pairs (d, d + HD/2) rotated by the position's angle for d
@@ -839,7 +756,6 @@ struct lmx_decoder {
   float *attn_part = nullptr;            // [n_heads][chunks][m, l, -, -, o[head_dim]]
   float *attn_out = nullptr;             // [n_heads * head_dim] merged attention output
   unsigned *attn_tickets = nullptr;      // [n_kv_heads][kAttnMaxSplit] unit tickets (zero between steps)
-  float *normed = nullptr;   // batch > 1: RMSNorm output [hidden] rows
   float *act = nullptr;      // SiLU(gate)*up [ffn] rows
   unsigned *argmax_ticket = nullptr;         // batch > 1: argmax_rows_kernel's ticket
   unsigned long long *argmax_slots = nullptr;   // batch > 1: [batch][kArgmaxParts] keys
@@ -901,15 +817,6 @@ GemvArgs decode_args(const lmx_weight *w, int xmode, int epi) {
 // Whether one vector of this weight runs on the digit kernels (4 and 8 bits,
 // digit_linear's rule).
 bool one_on_digits(const lmx_weight *w) { return w->digit && w->d_codes; }
-
-// Whether every linear of the decoder can run on the digit kernels for any
-// number of rows.
-bool on_digits(const lmx_decoder *d) {
-  const auto ok = [](const lmx_weight *w) { return w->digit && w->d_digits; };
-  for (const lmx_decoder::Layer &L : d->layers)
-    if (!ok(L.qkv) || !ok(L.o) || !ok(L.gate_up) || !ok(L.down)) return false;
-  return ok(d->head);
-}
 
 // Whether the digit kernels form SiLU(gate)*up in the gate|up epilogue (whole
 // row tiles in each half).
@@ -993,11 +900,7 @@ int finish_embed(const lmx_decoder *d, hipStream_t st) {
   return launch_err("finish_embed");
 }
 
-// qparts: the q|k|v rows as the batched GEMV's split partials
-// [batch][qsplits][qnpad] (kEpiPartials) with the q|k|v bias qbias, summed by
-// the attention kernel itself; nullptr: the rows are in d->qkv.
-int attention(lmx_decoder *d, size_t layer, hipStream_t st, const float *qparts = nullptr, int qsplits = 0,
-              int qnpad = 0, const float *qbias = nullptr) {
+int attention(lmx_decoder *d, size_t layer, hipStream_t st) {
   const lmx_decoder_config &c = d->cfg;
   const int group = int(c.n_heads / c.n_kv_heads);
   const int nch = int(attn_chunks(c));
@@ -1024,23 +927,14 @@ int attention(lmx_decoder *d, size_t layer, hipStream_t st, const float *qparts 
   }
   const dim3 grid(unsigned(c.n_kv_heads * units * hsplit), unsigned(d->batch));
   const size_t qkv_stride = (c.n_heads + 2 * c.n_kv_heads) * c.head_dim;
-  if (qparts && (qsplits < 1 || qsplits > kAttnMaxParts || qnpad < int(qkv_stride)))
-    return fail(LMX_ERR_INVALID_ARGUMENT, "attention over %d q|k|v partials of %d rows", qsplits, qnpad);
-#define LMX_ATTN(HD, CPW, PARTS)                                                                                    \
-  attn_kernel<HD, CPW, PARTS><<<grid, dim3(512), 0, st>>>(                                                         \
+#define LMX_ATTN(HD, CPW)                                                                                           \
+  attn_kernel<HD, CPW><<<grid, dim3(512), 0, st>>>(                                                                \
       d->qkv, kc, vc, d->pos, d->rope, int(c.n_heads), int(c.n_kv_heads), group, int(c.max_seq), scale, \
-      d->attn_part, nch, d->attn_tickets, d->attn_out, qkv_stride, d->kv_seq, spec_units, hsplit, qparts, qsplits,  \
-      qnpad, qbias)
-  if (qparts) {
-    if (c.head_dim == 64) {
-      if (cpw == 2) LMX_ATTN(64, 2, true); else LMX_ATTN(64, 1, true);
-    } else {
-      if (cpw == 2) LMX_ATTN(128, 2, true); else LMX_ATTN(128, 1, true);
-    }
-  } else if (c.head_dim == 64) {
-    if (cpw == 2) LMX_ATTN(64, 2, false); else LMX_ATTN(64, 1, false);
+      d->attn_part, nch, d->attn_tickets, d->attn_out, qkv_stride, d->kv_seq, spec_units, hsplit)
+  if (c.head_dim == 64) {
+    if (cpw == 2) LMX_ATTN(64, 2); else LMX_ATTN(64, 1);
   } else {
-    if (cpw == 2) LMX_ATTN(128, 2, false); else LMX_ATTN(128, 1, false);
+    if (cpw == 2) LMX_ATTN(128, 2); else LMX_ATTN(128, 1);
   }
 #undef LMX_ATTN
   return launch_err("attention");
@@ -1060,80 +954,6 @@ int upload(lmx_decoder *d, float **dst, const float *src, size_t n) {
   hipError_t e = hipMemcpy(*dst, src, n * sizeof(float), hipMemcpyHostToDevice);
   return e == hipSuccess ? LMX_OK : hip_err(e, "hipMemcpy (decoder weights)");
 }
-
-// y[b] = W x[b] (+ bias) (+ resid[b]) for the decoder's `batch` rows: groups
-// of 16/8/4 through the batched kernel (weights read once per group), the
-// rest one GEMV per row (the residual then rides as that row's bias).
-int gemv_rows(const lmx_decoder *d, const lmx_weight *w, const float *x, float *y, const float *bias,
-              const float *resid, hipStream_t st) {
-  GemvArgs a = weight_args(w);
-  a.rotate = rotates(w->format) ? LMX_ROTATE_FWHT256 : LMX_ROTATE_NONE;
-  a.bias = bias;
-  a.resid = resid;
-  size_t done = 0;
-  int r = gemv_batched(w, a, x, y, d->batch, st, &done);
-  if (r) return r;
-  a.resid = nullptr;
-  for (size_t b = done; b < d->batch; ++b) {
-    a.x = x + b * w->cols;
-    a.y = y + b * w->rows;
-    a.partials = w->d_partials;
-    if (resid) a.bias = resid + b * w->rows;   // decoder rows never carry both
-    if ((r = launch_gemv(w->format, a, st))) return r;
-  }
-  return LMX_OK;
-}
-
-// The decoder's rows through the batched kernel with a fused epilogue:
-// kEpiNormOut (y = W x + resid, y2 = RMSNorm(y) with weight xw) or
-// kEpiSiluPair (y = SiLU(gate)*up rows); every row must be covered
-// (rows_fuse checks that first).
-int gemv_rows_epi(const lmx_decoder *d, const lmx_weight *w, const float *x, float *y, const float *resid, int epi,
-                  const float *xw, float *y2, hipStream_t st) {
-  GemvArgs a = weight_args(w);
-  a.rotate = rotates(w->format) ? LMX_ROTATE_FWHT256 : LMX_ROTATE_NONE;
-  a.resid = resid;
-  a.epi = epi;
-  a.xw = xw;
-  a.eps = d->cfg.rms_eps;
-  a.y2 = y2;
-  size_t done = 0;
-  const int r = gemv_batched(w, a, x, y, d->batch, st, &done);
-  if (r) return r;
-  return done == d->batch ? LMX_OK
-                          : fail(LMX_ERR_INVALID_ARGUMENT, "fused batched epilogue covered %zu of %zu rows", done,
-                                 d->batch);
-}
-
-// Whether every layer's o / gate|up / down serve the fused epilogues for the
-// decoder's batch (LMX_FUSED_ROWS=0: never; the norms and SiLU*up then run
-// as row kernels).
-bool rows_fuse(const lmx_decoder *d) {
-  const char *e = std::getenv("LMX_FUSED_ROWS");
-  if (e && std::atoi(e) == 0) return false;
-  for (const lmx_decoder::Layer &L : d->layers)
-    if (!batched_epilogue_ok(L.o, kEpiNormOut, d->batch) || !batched_epilogue_ok(L.gate_up, kEpiSiluPair, d->batch) ||
-        !batched_epilogue_ok(L.down, kEpiNormOut, d->batch))
-      return false;
-  return true;
-}
-
-// Whether a layer's qkv projection leaves its split partials to attention
-// (kEpiPartials): the decoder's rows are one batched group whose splits the
-// attention kernel sums (LMX_QKV_PARTS=0: never; the batched reduction then
-// writes the rows first).
-bool qkv_parts(const lmx_decoder *d, const lmx_weight *qkv) {
-  const char *e = std::getenv("LMX_QKV_PARTS");
-  return !(e && std::atoi(e) == 0) && batched_epilogue_ok(qkv, kEpiPartials, d->batch) &&
-         batched_launch_splits(qkv->Npad, qkv->Kp) <= kAttnMaxParts;
-}
-
-int rmsnorm_rows(const lmx_decoder *d, const float *x, const float *wt, float *y, hipStream_t st) {
-  rmsnorm_rows_kernel<<<dim3(unsigned(d->batch)), dim3(256), 0, st>>>(x, wt, int(d->cfg.hidden), d->cfg.rms_eps, y);
-  return launch_err("rmsnorm_rows");
-}
-
-int step_batched_rows(lmx_decoder *d, hipStream_t st);
 
 // y = W x' (+ bias) (+ resid) of `rows` rows on the digit kernels, x' the
 // RMSNorm of x with weight xw where given; epi kEpiSiluPair: SiLU(gate)*up.
@@ -1233,110 +1053,23 @@ int prefill(lmx_decoder *d, size_t n, hipStream_t st) {
   return d->batch == 1 ? embed(d->embed, d->tokens, d->pos, d->hidden, 1, int(c.max_seq + 1), 1, 0, st) : LMX_OK;
 }
 
-// The layers of a batched step on the digit kernels, and the logits.
-int step_batched_digits(lmx_decoder *d, float *lg, hipStream_t st) {
-  const lmx_decoder_config &c = d->cfg;
-  int r;
-  for (size_t l = 0; l < c.n_layers; ++l) {
-    const lmx_decoder::Layer &L = d->layers[l];
-    if ((r = digit_rows(d, L.qkv, d->hidden, d->qkv, d->batch, L.qkv_bias, nullptr, L.in_norm, kEpiStore, st)) ||
-        (r = attention(d, l, st)) ||
-        (r = digit_rows(d, L.o, d->attn_out, d->hidden, d->batch, nullptr, d->hidden, nullptr, kEpiStore, st)) ||
-        (r = digit_mlp(d, L, d->hidden, d->gate_up, d->act, d->batch, st)))
-      return r;
-  }
-  return digit_rows(d, d->head, d->hidden, lg, d->batch, nullptr, nullptr, d->final_norm, kEpiStore, st);
-}
-
-// Four rows of one linear in one group (the four-vector kernel where the
-// plan has it, else the batched kernel): y = W x' (+ bias) (+ resid), x' the
-// RMSNorm of x with weight xw when xmode asks.
-int gemv_group4(const lmx_decoder *d, const lmx_weight *w, const float *x, float *y, const float *bias,
-                const float *resid, int xmode, const float *xw, int epi, hipStream_t st) {
-  GemvArgs a = decode_args(w, xmode, epi);
-  a.bias = bias;
-  a.resid = resid;
-  a.xw = xw;
-  a.eps = d->cfg.rms_eps;
-  size_t done = 0;
-  const int r = gemv_batched(w, a, x, y, 4, st, &done);
-  if (r) return r;
-  return done == 4 ? LMX_OK : fail(LMX_ERR_INVALID_ARGUMENT, "a group of 4 rows covered %zu", done);
-}
-
-// Batch 4 with every layer's qkv and o on the four-vector kernel (LMX_QUAD_STEP=0:
-// never): the norms ride in the kernels' table builds and the residual in
-// their epilogues, so the o projection needs no reduction.
-bool quad_step(const lmx_decoder *d) {
-  const char *e = std::getenv("LMX_QUAD_STEP");
-  if (d->batch != 4 || (e && std::atoi(e) == 0) || !d->head->batched) return false;
-  for (const lmx_decoder::Layer &L : d->layers)
-    if (!quad_serves(decode_args(L.qkv, kXModeRmsNorm, kEpiStore)) || !quad_serves(decode_args(L.o, kXModeNone, kEpiStore)) ||
-        !L.qkv->batched || !L.o->batched || !L.gate_up->batched || !L.down->batched ||
-        !batched_epilogue_ok(L.gate_up, kEpiSiluPair, 4))
-      return false;
-  return true;
-}
-
 // One token step of `batch` sequences in lockstep: every linear reads its
-// weights once per group of sequences.  The batched GEMV splits K, so its
-// table build cannot apply the RMSNorm of its input; instead the reduction
-// that finishes the o and down projections also writes the normed rows, and
-// the gate|up reduction writes SiLU(gate)*up (when every row is in a batched
-// group; else the norms and SiLU*up run as row kernels).  Attention and the
-// argmax run per sequence.
+// weights once per step.  Attention and the argmax run per sequence.
 int step_batched(lmx_decoder *d, float *logits_out, hipStream_t st) {
   const lmx_decoder_config &c = d->cfg;
   const size_t B = d->batch;
+  float *lg = logits_out ? logits_out : d->logits;
   int r = embed(d->embed, d->tokens, d->pos, d->hidden, B, int(c.max_seq + 1), 1, 0, st);
   if (r) return r;
-  float *lg = logits_out ? logits_out : d->logits;
-  const bool digits = on_digits(d), quad = !digits && quad_step(d);
-  if (digits) {
-    if ((r = step_batched_digits(d, lg, st))) return r;
-  } else if (quad) {
-    // qkv: RMSNorm in the table build; o: + hidden in the epilogue; gate|up:
-    // RMSNorm in the batched table build, SiLU(gate)*up in its reduction;
-    // down: + hidden in its reduction; the head normalises its own input.
-    for (size_t l = 0; l < c.n_layers; ++l) {
-      const lmx_decoder::Layer &L = d->layers[l];
-      if ((r = gemv_group4(d, L.qkv, d->hidden, d->qkv, L.qkv_bias, nullptr, kXModeRmsNorm, L.in_norm, kEpiStore,
-                           st)) ||
-          (r = attention(d, l, st)) ||
-          (r = gemv_group4(d, L.o, d->attn_out, d->hidden, nullptr, d->hidden, kXModeNone, nullptr, kEpiStore, st)) ||
-          (r = gemv_group4(d, L.gate_up, d->hidden, d->act, nullptr, nullptr, kXModeRmsNorm, L.post_norm,
-                           kEpiSiluPair, st)) ||
-          (r = gemv_group4(d, L.down, d->act, d->hidden, nullptr, d->hidden, kXModeNone, nullptr, kEpiStore, st)))
-        return r;
-    }
-    if ((r = gemv_group4(d, d->head, d->hidden, lg, nullptr, nullptr, kXModeRmsNorm, d->final_norm, kEpiStore, st)))
+  for (size_t l = 0; l < c.n_layers; ++l) {
+    const lmx_decoder::Layer &L = d->layers[l];
+    if ((r = digit_rows(d, L.qkv, d->hidden, d->qkv, B, L.qkv_bias, nullptr, L.in_norm, kEpiStore, st)) ||
+        (r = attention(d, l, st)) ||
+        (r = digit_rows(d, L.o, d->attn_out, d->hidden, B, nullptr, d->hidden, nullptr, kEpiStore, st)) ||
+        (r = digit_mlp(d, L, d->hidden, d->gate_up, d->act, B, st)))
       return r;
-  } else if (rows_fuse(d)) {
-    // The o and down reductions write the hidden rows and the next linear's
-    // normed input; the gate|up reduction writes SiLU(gate)*up.
-    if ((r = rmsnorm_rows(d, d->hidden, d->layers[0].in_norm, d->normed, st))) return r;
-    for (size_t l = 0; l < c.n_layers; ++l) {
-      const lmx_decoder::Layer &L = d->layers[l];
-      const float *next_norm = l + 1 < c.n_layers ? d->layers[l + 1].in_norm : d->final_norm;
-      if (qkv_parts(d, L.qkv)) {
-        // the qkv split sums go straight to attention (no reduction launch)
-        if ((r = gemv_rows_epi(d, L.qkv, d->normed, d->qkv, nullptr, kEpiPartials, nullptr, nullptr, st)) ||
-            (r = attention(d, l, st, L.qkv->d_bpartials, batched_launch_splits(L.qkv->Npad, L.qkv->Kp),
-                           int(L.qkv->Npad), L.qkv_bias)))
-          return r;
-      } else if ((r = gemv_rows(d, L.qkv, d->normed, d->qkv, L.qkv_bias, nullptr, st)) || (r = attention(d, l, st))) {
-        return r;
-      }
-      if ((r = gemv_rows_epi(d, L.o, d->attn_out, d->hidden, d->hidden, kEpiNormOut, L.post_norm, d->normed, st)) ||
-          (r = gemv_rows_epi(d, L.gate_up, d->normed, d->act, nullptr, kEpiSiluPair, nullptr, nullptr, st)) ||
-          (r = gemv_rows_epi(d, L.down, d->act, d->hidden, d->hidden, kEpiNormOut, next_norm, d->normed, st)))
-        return r;
-    }
-  } else {
-    if ((r = step_batched_rows(d, st))) return r;
-    if ((r = rmsnorm_rows(d, d->hidden, d->final_norm, d->normed, st))) return r;
   }
-  if (!quad && !digits && (r = gemv_rows(d, d->head, d->normed, lg, nullptr, nullptr, st))) return r;
+  if ((r = digit_rows(d, d->head, d->hidden, lg, B, nullptr, nullptr, d->final_norm, kEpiStore, st))) return r;
   // parts per row: about 256 workgroups in all (LMX_ARGMAX_PARTS overrides)
   const char *ap = std::getenv("LMX_ARGMAX_PARTS");
   const int parts = std::max(1, std::min(kArgmaxParts, ap ? std::atoi(ap) : int(256 / B)));
@@ -1344,28 +1077,6 @@ int step_batched(lmx_decoder *d, float *logits_out, hipStream_t st) {
       lg, int(c.vocab), d->tokens, int(c.max_seq + 1), d->pos, d->n_forced, int(c.max_seq), d->argmax_ticket,
       d->argmax_slots, d->argmax_seq_tickets, d->penalty_counts(), d->penalty);
   return launch_err("argmax_rows");
-}
-
-// The layers of a batched step with the norms and SiLU*up as row kernels.
-int step_batched_rows(lmx_decoder *d, hipStream_t st) {
-  const lmx_decoder_config &c = d->cfg;
-  const size_t B = d->batch;
-  int r = LMX_OK;
-  for (size_t l = 0; l < c.n_layers; ++l) {
-    const lmx_decoder::Layer &L = d->layers[l];
-    if ((r = rmsnorm_rows(d, d->hidden, L.in_norm, d->normed, st)) ||
-        (r = gemv_rows(d, L.qkv, d->normed, d->qkv, L.qkv_bias, nullptr, st)) ||
-        (r = attention(d, l, st)) ||
-        (r = gemv_rows(d, L.o, d->attn_out, d->hidden, nullptr, d->hidden, st)) ||
-        (r = rmsnorm_rows(d, d->hidden, L.post_norm, d->normed, st)) ||
-        (r = gemv_rows(d, L.gate_up, d->normed, d->gate_up, nullptr, nullptr, st)))
-      return r;
-    silu_mul_rows_kernel<<<dim3(unsigned((c.ffn + 255) / 256), unsigned(B)), dim3(256), 0, st>>>(d->gate_up,
-                                                                                                int(c.ffn), d->act);
-    if ((r = launch_err("silu_mul_rows")) || (r = gemv_rows(d, L.down, d->act, d->hidden, nullptr, d->hidden, st)))
-      return r;
-  }
-  return LMX_OK;
 }
 
 // One token step of one sequence.  The hidden state already holds the
@@ -1497,7 +1208,6 @@ int lmx_decoder_create_batched(const lmx_decoder_config *cfg, size_t batch, lmx_
       (st = d->alloc(reinterpret_cast<void **>(&d->attn_out), B * c.n_heads * c.head_dim * sizeof(float))) ||
       (st = d->alloc(reinterpret_cast<void **>(&d->attn_tickets),
                      B * c.n_kv_heads * kAttnMaxSplit * kTicketPad * sizeof(unsigned))) ||
-      (B > 1 && (st = d->alloc(reinterpret_cast<void **>(&d->normed), B * c.hidden * 4))) ||
       (st = d->alloc(reinterpret_cast<void **>(&d->act), B * c.ffn * 4)) ||
       (B > 1 && (st = d->alloc(reinterpret_cast<void **>(&d->argmax_ticket), sizeof(unsigned)))) ||
       (B > 1 && (st = d->alloc(reinterpret_cast<void **>(&d->argmax_slots), B * kArgmaxParts * 8))) ||
@@ -1669,7 +1379,7 @@ int lmx_decoder_generate(lmx_decoder *d, const int32_t *prompt, size_t n_prompt,
   // All but the prompt's last position in passes of many rows; a pass costs
   // about as much as three steps, so a shorter prompt takes steps.
   size_t passed = 0;
-  if (e == hipSuccess && n_prompt > 4 && on_digits(d)) {
+  if (e == hipSuccess && n_prompt > 4) {
     passed = n_prompt - 1;
     if ((st = prefill(d, passed, s)) != LMX_OK) e = hipErrorUnknown;
   }

@@ -42,23 +42,16 @@ void tile_planes(int fmt, const uint8_t *planes, size_t rows, size_t row_bytes,
                  size_t Npad, size_t Kp, uint8_t *tiles);
 void untile_planes(int fmt, const uint8_t *tiles, size_t rows, size_t row_bytes,
                    size_t Npad, size_t Kp, uint8_t *planes);
-// 4-bit planes [4][rows][row_bytes] -> the matrix-core kernel's code layout
-// [Kp/128][Npad][4 lane groups kq][8 k-blocks][2 bytes]: byte b of k-block
-// kb, group kq holds codes k = 16 kb + 4 kq + 2b (low nibble) and + 1 (high
-// nibble) of the chunk; columns past row_bytes*8 and rows past `rows` hold
-// code 8 (value 0).
-void nibble_tiles(const uint8_t *planes, size_t rows, size_t row_bytes, size_t Npad, size_t Kp, uint8_t *out);
 
 // ---- device launches (lmx_kernels.hip) -----------------------------------
 struct GemvArgs {
   const void *planes;      // tiled planes
-  const void *nib;         // int4 codes in the matrix-core layout (nibble_tiles), or null
   const void *codes;       // digit kernels: 4- and 8-bit code copy (code_copy_bytes), or null
   const float *scales;     // [S][n_groups][Npad]
   const float *x;          // [cols]
   float *y;                // [rows]
   const float *bias;       // [rows] or null
-  const float *resid;      // batched kernel: [batch][rows] added to y (may alias y), or null
+  const float *resid;      // digit kernels: [batch][rows] added to y (may alias y), or null
   float *partials;         // [splits][Npad]
   unsigned *counters;      // [row_blocks]
   int rows, Npad, cols, Kp;
@@ -80,7 +73,6 @@ struct GemvArgs {
                            // argmax keys then rank repetition-penalised values (penalised_logit)
   float penalty;           // repetition penalty applied pcount[row] times
   int epi;                 // output epilogue (kEpi*)
-  float *y2;               // kEpiNormOut: RMSNorm of y with weight xw [rows] (batched GEMV only)
 };
 
 // Output epilogues of the full-K kernels:
@@ -90,19 +82,8 @@ struct GemvArgs {
 //                  workgroup computes gate rows and the matching up rows
 //                  (model.cpp:36,413-416), so the activation of the down
 //                  projection leaves the gate|up launch already formed
-//   kEpiNormOut:   (batched GEMV) y as kEpiStore (+ resid), and y2 = the
-//                  RMSNorm of each y row with weight xw and epsilon eps
-//                  (norm.cpp:18-34), the next linear's input
-//   kEpiPartials:  (batched GEMV, exactly one group of 4/8/16 vectors) no
-//                  reduction: the split sums stay in a.partials
-//                  [nb][splits][Npad] (batched_launch_splits of them) for a
-//                  consumer that sums them in split order itself (the decode
-//                  attention reads its q/k/v rows that way)
 constexpr int kEpiStore = 0;
 constexpr int kEpiSiluPair = 1;
-constexpr int kEpiNormOut = 2;
-constexpr int kEpiPartials = 3;
-constexpr int kNormOutMaxRows = 8192;   // kEpiNormOut keeps a whole row in LDS
 
 // Activation transforms applied while the tables are built:
 //   kXModeRmsNorm:  x'[k] = x[k] * inv_rms * xw[k], inv_rms = 1/sqrt(sum x^2 / cols + eps)
@@ -184,35 +165,9 @@ int launch_gemv(int fmt, const GemvArgs &a, void *stream);
 // the 4 x 4 x 1 and 16 x 4 x 1 plans (default), 2 the 4 x 4 x 1 plan only,
 // 0 neither.
 int plane_split_level();
-// Batched unrotated 4-bit GEMVs of 8 or 16 vectors, and of 4 except for
-// split partials left to a consumer, on the matrix cores (LMX_MFMA, read per
-// call): 1 (default), 0 the lookup-table kernel.
-int mfma_batched();
 // Rows of one output half a workgroup covers with kEpiSiluPair for these
 // arguments (format, plan, transform), 0 when that epilogue is not served.
 int silu_pair_rows(int fmt, const GemvArgs &a);
-// nb (2, 4, 8, 16) vectors at a.x + n*cols -> a.y + n*rows; a.partials holds
-// nb * (Kp/256) * Npad floats.
-int launch_gemv_batch(int fmt, const GemvArgs &a, int nb, void *stream);
-// k-slices of the batched kernel for a weight: 256-wide, or 128-wide where
-// the 256-wide grid at 64 rows per workgroup has fewer than kBatchMinGrid128
-// workgroups (CUs idle); the batched partials hold 16 x this x Npad floats.
-constexpr size_t kBatchMinGrid128 = 256;
-inline size_t batched_slice_splits(size_t Npad, size_t Kp) {
-  const size_t s256 = Kp / kRotChunk;
-  return (Npad / kWave) * s256 < kBatchMinGrid128 ? 2 * s256 : s256;
-}
-// The k-slices a batched launch actually uses: batched_slice_splits, or the
-// 256-wide ones when LMX_BATCH_S128=0 turns the 128-wide slices off.
-int batched_launch_splits(size_t Npad, size_t Kp);
-
-// Exactly 4 vectors (a.x [4][cols], a.y [4][rows], a.resid [4][rows]) in one
-// full-K launch with the transform a.xmode (none or RMSNorm with a.xw) and
-// epilogue a.epi (store or SiLU pair); returns 1, launching nothing, when
-// the handle's plan has no such form (split-K plans, K above 2048, more than
-// one round of workgroups; quad_serves tells beforehand).
-int launch_gemv_quad(int fmt, const GemvArgs &a, void *stream);
-bool quad_serves(const GemvArgs &a);
 // ---- digit kernels (lmx_digit.hip): exact products on the 8-bit matrix cores ----
 // Vectors split into signed-byte digits by launch_digit_split.
 struct DigitVectors {
@@ -280,13 +235,10 @@ struct lmx_weight {
   float *d_partials = nullptr;
   unsigned *d_counters = nullptr;
   float *d_xrot = nullptr;  // staging for LMX_ROTATE_FWHT_FULL (cols floats)
-  bool digit = true;             // digit kernels (LMX_DIGIT=0, or a lookup-table plan asked for: not)
-  bool batched = true;           // batch >= 2 through the batched kernel (LMX_BATCHED=0: one GEMV per vector)
-  float *d_bpartials = nullptr;  // batched partials [16][Kp/256][Npad] (the memory of d_partials)
+  bool digit = true;             // one vector of 4 or 8 bits on the digit kernels (LMX_DIGIT=0, or a
+                                 // lookup-table plan asked for: not)
   void *d_codes = nullptr;       // digit kernels: 4- and 8-bit code copy
-  void *d_nib = nullptr;         // int4 with the matrix-core kernel: codes in nibble_tiles layout
-  size_t bpartials_cap = 0;      // floats
-  void *d_digits = nullptr;      // scratch of the digit kernels: d_bpartials, or the caller's
+  void *d_digits = nullptr;      // scratch of the digit kernels: the memory of d_partials, or the caller's
   size_t digit_cap = 0;          // its bytes
 };
 
@@ -299,17 +251,9 @@ void plan_weight(lmx_weight *w, int fmt, size_t rows, size_t cols, size_t group)
 int gemv_impl(const lmx_weight *w, const float *x, float *y, size_t batch, unsigned flags, void *stream);
 // Kernel arguments of a handle (x, y, bias, rotation and transform unset).
 GemvArgs weight_args(const lmx_weight *w);
-// Vectors x[0..batch) in groups of 16/8/4 through the batched kernel (a.bias
-// per row, a.resid per vector row); *done = the vectors it covered (none
-// below 4).
-int gemv_batched(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream,
-                 size_t *done);
 // y = W x of `batch` vectors on the digit kernels (a.bias, a.resid, a.rotate, a.xmode none or RMSNorm,
 // a.epi store or SiLU pair; x of any alignment); *done = the vectors covered, the rest (one by one on
 // the lookup tables) left to the caller unless `all`
 int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done,
                  bool all);
-// Whether gemv_batched serves epilogue epi (kEpi*) for `batch` vectors of w
-// with no vector left to the single-vector path (x 16-byte aligned assumed).
-bool batched_epilogue_ok(const lmx_weight *w, int epi, size_t batch);
 }  // namespace lmx

@@ -89,7 +89,6 @@ extern "C" int lmx_gemv_tiles_noalloc(int format, const void *tiles, const float
     return fail(LMX_ERR_INVALID_ARGUMENT, "tiles must be 16-byte and scales 4-byte aligned");
   lmx_weight w;   // the plan lmx_weight_create would choose, over the caller's buffers
   plan_weight(&w, format, rows, cols, group);
-  w.batched = false;   // the batched lookup kernel's partials would not fit
   const size_t row_blocks = w.Npad / kWave;
   const size_t staging = round_up(w.Kp * sizeof(float), 256);
   // split-K plans, and the layered full-K plan (which runs the split-K
