@@ -155,8 +155,11 @@ __global__ __launch_bounds__(256) void digit_split_chunks_kernel(const float *__
 // Two row tiles per workgroup once that leaves a workgroup per CU: each makes
 // the digits of the whole K (4-bit, us, one tile against two: 2048 x 2048
 // 3.18 / 3.44, 3072 x 2048 3.35 / 3.56, 17920 x 1536 5.54 / 5.27, 8192 x 8192
-// 12.0 / 8.0).
-int digit_gemv_tiles(const GemvArgs &a) { return a.epi == kEpiSiluPair || a.Npad / kTile >= 512 ? 2 : 1; }
+// 12.0 / 8.0).  A workgroup has a wave per 256-chunk and a thread per output
+// of its 4 vectors, so a K of one 256-chunk keeps to one tile.
+int digit_gemv_tiles(const GemvArgs &a) {
+  return a.epi == kEpiSiluPair || (a.Npad / kTile >= 512 && a.Kp > kRotChunk) ? 2 : 1;
+}
 
 size_t digit_argmax_slots(const GemvArgs &a) { return size_t(a.Npad) / (kTile * digit_gemv_tiles(a)); }
 

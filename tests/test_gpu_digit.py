@@ -71,6 +71,20 @@ def test_digit_linear(cuda, fmt, rows, cols, batch):
     w.close()
 
 
+# From 8192 rows a workgroup takes two row tiles, if its waves have a thread for
+# each output of 4 vectors.
+@pytest.mark.parametrize("fmt", [1, 3, 6, 7])
+@pytest.mark.parametrize("cols", [256, 512])
+@pytest.mark.parametrize("batch", [3, 4])
+def test_digit_many_rows(cuda, fmt, cols, batch):
+    planes, scales, g, w = make(fmt, 8190, cols, seed=cols + fmt)
+    x = vectors(batch, cols, seed=batch)
+    y = torch.full((batch, 8190), torch.nan, device="cuda")
+    w.linear(torch.from_numpy(x).cuda(), y=y)
+    check(fmt, planes, scales, 8190, cols, g, x, y.cpu().numpy(), rotate=fmt in (1, 2, 3, 4))
+    w.close()
+
+
 # The tile kernel takes over at 192 workgroups (8 row tiles x 32 vectors
 # each): a shape on either side, a last row group and vector group partly
 # filled, and a group scale of three chunks.
