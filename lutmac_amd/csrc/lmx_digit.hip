@@ -203,9 +203,12 @@ DigitVectors digit_vectors(const lmx_weight *w, void *scratch, size_t count) {
   d.exp = reinterpret_cast<int *>(d.fac + quads * 4);
   d.partials = reinterpret_cast<float *>(d.exp + quads * 4);
   d.count = int(count);
-  // The tile kernel where it has most of a workgroup per CU (2048 columns,
-  // us: 192 workgroups 21 against 25, 128 workgroups 20 / 18).
-  d.tile = (w->Npad / kTile + 7) / 8 * ((quads + 7) / 8) >= 192;
+  // The tile kernel from a workgroup of 8 row tiles x 4 quads for every other
+  // CU (us, tile / rows form: 8192 x 2048 x 32 vectors 11.9 / 10.8, 17920 x
+  // 1536 x 16 10.8 / 12.7, 3001 x 1400 x 128 11.1 / 13.3); with fewer than 4
+  // quads from as many products (17920 x 1536 x 8 11.7 / 9.7, 128256 x 2048 x
+  // 8 33 / 48).
+  d.tile = (w->Npad / kTile + 7) / 8 * quads > 512;
   return d;
 }
 

@@ -414,14 +414,18 @@ __global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVecto
 // ---------------------------------------------------------------------------
 // Many vectors: 4 waves of RT row tiles x the same NQ quads, the quads'
 // fragments of a chunk staged in LDS (two chunks deep).
-template <int FMT, bool COPY, int NQ, int RT, int EPI>
-__global__ __launch_bounds__(256, 3) void digit_tile_kernel(GemvArgs a, DigitVectors d) {
+constexpr int tile_waves(int nq, int ks) { return ks == 1 ? (nq == 8 ? 3 : 4) : nq == 8 ? 2 : 4; }
+
+template <int FMT, bool COPY, int NQ, int RT, int KS, int EPI>
+__global__ __launch_bounds__(256 * KS, tile_waves(NQ, KS)) void digit_tile_kernel(GemvArgs a, DigitVectors d) {
   constexpr int CW = Source<FMT, COPY>::CW, S = Fmt<FMT>::S;
   constexpr bool PAIR = EPI == kEpiSiluPair;
   constexpr int WAVES = 4;
-  __shared__ __attribute__((aligned(16))) char frags[2][NQ * kQuadChunk];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
+  __shared__ __attribute__((aligned(16))) char frags_all[KS][2][NQ * kQuadChunk];
+  const int lane = threadIdx.x & (kWave - 1), tid = int(threadIdx.x) % 256;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int kg = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(int(threadIdx.x) / 256);   // the wave's part of k
+  auto &frags = frags_all[kg];
   const int li = lane & 15, kq = lane >> 4;
   const int Kc = a.Kp / kChunk;
   const uint32_t Npad = uint32_t(a.Npad);
@@ -449,7 +453,7 @@ __global__ __launch_bounds__(256, 3) void digit_tile_kernel(GemvArgs a, DigitVec
   const char *fsrc[LD];
 #pragma unroll
   for (int i = 0; i < LD; ++i) {
-    const int p = int(threadIdx.x) + 256 * i, q = p / 128, o = p % 128;
+    const int p = tid + 256 * i, q = p / 128, o = p % 128;
     fsrc[i] = d.digits + size_t(min(q0 + q, quads - 1)) * qbytes + o * 16;
   }
   const auto load_f = [&](int b, int ch) {
@@ -458,7 +462,7 @@ __global__ __launch_bounds__(256, 3) void digit_tile_kernel(GemvArgs a, DigitVec
   };
   const auto store_f = [&](int b) {
 #pragma unroll
-    for (int i = 0; i < LD; ++i) *reinterpret_cast<v4i *>(frags[b] + (int(threadIdx.x) + 256 * i) * 16) = st[b][i];
+    for (int i = 0; i < LD; ++i) *reinterpret_cast<v4i *>(frags[b] + (tid + 256 * i) * 16) = st[b][i];
   };
   const auto load_w = [&](int b, int ch) {
     ch = min(ch, Kc - 1);
@@ -477,7 +481,7 @@ __global__ __launch_bounds__(256, 3) void digit_tile_kernel(GemvArgs a, DigitVec
 #pragma unroll
     for (int q = 0; q < NQ; ++q) acc[t][q] = 0.0f;
   const auto chunk = [&](int ch, const int b) {   // b = ch % 2
-    load_f(b, ch + 2);
+    load_f(b, ch + 2 * KS);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       uint32_t wb[RT][8];
@@ -485,9 +489,9 @@ __global__ __launch_bounds__(256, 3) void digit_tile_kernel(GemvArgs a, DigitVec
 #pragma unroll
       for (int t = 0; t < RT; ++t) {
         source_bytes<FMT, COPY>(w[b][t], s, wb[t]);
-        cs[t] = sc[b][t][s];
+        cs[t] = KS == 1 || ch < Kc ? sc[b][t][s] : 0.0f;   // past the last chunk: adds nothing
       }
-      if (s == S - 1) load_w(b, ch + 2);   // the words are bytes now
+      if (s == S - 1) load_w(b, ch + 2 * KS);   // the words are bytes now
       // The products of quad q run while quad q - 1's sums are joined and quad
       // q + 1's fragments arrive; the barriers keep the compiler from issuing
       // every quad's reads and products first (registers).
@@ -519,16 +523,35 @@ __global__ __launch_bounds__(256, 3) void digit_tile_kernel(GemvArgs a, DigitVec
     store_f(b ^ 1);
     __syncthreads();
   };
-  load_f(0, 0);
-  load_w(0, 0);
-  load_f(1, 1);
-  load_w(1, 1);
+  load_f(0, 2 * kg);
+  load_w(0, 2 * kg);
+  load_f(1, 2 * kg + 1);
+  load_w(1, 2 * kg + 1);
   store_f(0);
   __syncthreads();
 #pragma unroll 1
-  for (int ch = 0; ch < Kc; ch += 2) {   // Kc is even
-    chunk(ch, 0);
-    chunk(ch + 1, 1);
+  for (int c0 = 0; c0 < Kc; c0 += 2 * KS) {   // Kc is even; every part makes the same rounds
+    chunk(c0 + 2 * kg, 0);
+    chunk(c0 + 2 * kg + 1, 1);
+  }
+  if constexpr (KS > 1) {   // the parts of k, in order
+    float *red = reinterpret_cast<float *>(frags_all[0][0]);
+    constexpr int SUMS = RT * NQ * 256;
+    static_assert((KS - 1) * SUMS * sizeof(float) <= sizeof(frags_all), "sums in place of the fragments");
+    if (kg > 0) {
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) red[(kg - 1) * SUMS + (t * NQ + q) * 256 + tid] = acc[t][q];
+    }
+    __syncthreads();
+    if (kg > 0) return;   // wave-uniform; no barrier follows
+#pragma unroll
+    for (int p = 0; p < KS - 1; ++p)
+#pragma unroll
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) acc[t][q] += red[p * SUMS + (t * NQ + q) * 256 + tid];
   }
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
@@ -583,22 +606,43 @@ int launch_rows(const GemvArgs &a, const DigitVectors &d, hipStream_t st) {
   return launched("digit_rows");
 }
 
-template <int FMT, int NQ, int RT>
+template <int FMT, int NQ, int RT, int KS>
 int launch_tile(const GemvArgs &a, const DigitVectors &d, hipStream_t st) {
   constexpr bool COPY = has_copy<FMT>();
   const int quads = (d.count + 3) / 4;
   const int groups = a.epi == kEpiSiluPair ? (a.rows / 2 / kTile + RT / 2 - 1) / (RT / 2) : (a.Npad / kTile + RT - 1) / RT;
   const dim3 grid{unsigned((groups + 3) / 4), unsigned((quads + NQ - 1) / NQ)};
-  if (a.epi == kEpiSiluPair) digit_tile_kernel<FMT, COPY, NQ, RT, kEpiSiluPair><<<grid, dim3(256), 0, st>>>(a, d);
-  else digit_tile_kernel<FMT, COPY, NQ, RT, kEpiStore><<<grid, dim3(256), 0, st>>>(a, d);
+  if (a.epi == kEpiSiluPair) digit_tile_kernel<FMT, COPY, NQ, RT, KS, kEpiSiluPair><<<grid, dim3(256 * KS), 0, st>>>(a, d);
+  else digit_tile_kernel<FMT, COPY, NQ, RT, KS, kEpiStore><<<grid, dim3(256 * KS), 0, st>>>(a, d);
   return launched("digit_tile");
 }
 
 template <int FMT>
 int launch_gemm_fmt(const GemvArgs &a, const DigitVectors &d, hipStream_t st) {
-  if (d.tile) return launch_tile<FMT, 8, 2>(a, d, st);
-  const int quads = (d.count + 3) / 4;
-  if (quads <= 2) return launch_rows<FMT, 2, 2>(a, d, st);
+  const int quads = (d.count + 3) / 4, tiles = a.Npad / kTile;
+  if (d.tile) {
+    // 8 quads a workgroup where that leaves two of them per CU and no more
+    // padding than 4 quads would (us: 16384 x 2048 x 256 vectors 47 / 51,
+    // 8192 x 2048 x 256 30.4 / 29.9, x 128 21.3 / 18.7; 16 vectors 52 / 35 of
+    // 128256 rows).  Up to two workgroups per CU, two of their halves of k
+    // each (2048 x 8192 x 512 57.4 against 60.8, 8192 x 2048 x 64 12.7 / 14.9,
+    // 17920 x 1536 x 64, with 560 workgroups, 20.9 / 18.8).
+    const int q4 = (quads + 3) / 4, q8 = (quads + 7) / 8, blocks = (tiles + 7) / 8;
+    if (blocks * q8 >= 512 && 10 * 2 * q8 < 11 * q4) return launch_tile<FMT, 8, 2, 1>(a, d, st);
+    if (blocks * q4 > 512) return launch_tile<FMT, 4, 2, 1>(a, d, st);
+    return launch_tile<FMT, 4, 2, 2>(a, d, st);
+  }
+  // The smallest tile that one workgroup per CU covers the call with: then the
+  // reads of one workgroup, a chunk or two per wave, are what takes the time
+  // (us, 4 quads x 2 row tiles / chosen: 2048 x 2048 x 16 vectors 6.9 / 5.8,
+  // 1536 x 8960 x 16 9.7 / 8.9, x 8 9.4 / 7.5); beyond that the largest, which
+  // reads the codes least often (17920 x 1536 x 16 12.8, 2 quads 13.4).
+  const auto fits = [&](int nq, int rt) { return tiles / rt * ((quads + nq - 1) / nq) <= 256; };
+  const bool one = a.epi != kEpiSiluPair;
+  if (one && fits(1, 1)) return launch_rows<FMT, 1, 1>(a, d, st);
+  if (one && quads > 1 && fits(2, 1)) return launch_rows<FMT, 2, 1>(a, d, st);
+  if (quads == 1 || fits(1, 2)) return launch_rows<FMT, 1, 2>(a, d, st);
+  if (quads == 2 || fits(2, 2)) return launch_rows<FMT, 2, 2>(a, d, st);
   return launch_rows<FMT, 4, 2>(a, d, st);
 }
 
@@ -608,7 +652,7 @@ int launch_digit_gemv_cfg(const GemvArgs &a, int nv, int W, hipStream_t st) {
   const bool pair = a.epi == kEpiSiluPair;
   const dim3 grid{unsigned(pair ? a.rows / 2 / (kTile * RT / 2) : a.Npad / (kTile * RT))};
   if (pair) {
-    if constexpr (RT >= 2)
+    if constexpr (RT == 2)
       digit_gemv_kernel<FMT, COPY, NV, RT, PPW, kXModeRmsNorm, kEpiSiluPair><<<grid, block, 0, st>>>(a, nv);
   } else if (a.xmode == kXModeRmsNorm) {
     digit_gemv_kernel<FMT, COPY, NV, RT, PPW, kXModeRmsNorm, kEpiStore><<<grid, block, 0, st>>>(a, nv);
@@ -634,6 +678,15 @@ template <int FMT, bool COPY>
 int launch_digit_gemv_src(const GemvArgs &a, int nv, hipStream_t st) {
   const bool two = digit_gemv_tiles(a) == 2;
   if (nv == 1) return two ? launch_digit_gemv_rt<FMT, COPY, 1, 2>(a, nv, st) : launch_digit_gemv_rt<FMT, COPY, 1, 1>(a, nv, st);
+  // Four row tiles share one making of four vectors' digits (us, two tiles /
+  // four: 4-bit 10240 x 2048 5.76 / 5.26, 16384 x 4096 11.4 / 8.3, ternary
+  // 32768 x 2048 14.1 / 12.1; 8192 x 2048 4.34 / 5.18, 17920 x 1536 7.3 / 8.3).
+  // (Not the 8-bit and three-stage formats, whose codes and scales of four
+  // tiles spill.)
+  if constexpr (FMT != LMX_FMT_INT8 && FMT != LMX_FMT_RRQ3) {
+    if (a.epi != kEpiSiluPair && a.Npad / kTile >= 640 && a.Kp >= 2048)
+      return launch_digit_gemv_rt<FMT, COPY, 4, 4>(a, nv, st);
+  }
   return two ? launch_digit_gemv_rt<FMT, COPY, 4, 2>(a, nv, st) : launch_digit_gemv_rt<FMT, COPY, 4, 1>(a, nv, st);
 }
 

@@ -72,24 +72,27 @@ def test_digit_linear(cuda, fmt, rows, cols, batch):
 
 
 # From 8192 rows a workgroup takes two row tiles, if its waves have a thread for
-# each output of 4 vectors.
+# each output of 4 vectors, and from 10240 rows and 2048 columns four.
 @pytest.mark.parametrize("fmt", [1, 3, 6, 7])
-@pytest.mark.parametrize("cols", [256, 512])
+@pytest.mark.parametrize("rows,cols", [(8190, 256), (8190, 512), (10230, 2048)])
 @pytest.mark.parametrize("batch", [3, 4])
-def test_digit_many_rows(cuda, fmt, cols, batch):
-    planes, scales, g, w = make(fmt, 8190, cols, seed=cols + fmt)
+def test_digit_many_rows(cuda, fmt, rows, cols, batch):
+    planes, scales, g, w = make(fmt, rows, cols, seed=cols + fmt)
     x = vectors(batch, cols, seed=batch)
-    y = torch.full((batch, 8190), torch.nan, device="cuda")
+    y = torch.full((batch, rows), torch.nan, device="cuda")
     w.linear(torch.from_numpy(x).cuda(), y=y)
-    check(fmt, planes, scales, 8190, cols, g, x, y.cpu().numpy(), rotate=fmt in (1, 2, 3, 4))
+    check(fmt, planes, scales, rows, cols, g, x, y.cpu().numpy(), rotate=fmt in (1, 2, 3, 4))
     w.close()
 
 
-# The tile kernel takes over at 192 workgroups (8 row tiles x 32 vectors
-# each): a shape on either side, a last row group and vector group partly
-# filled, and a group scale of three chunks.
+# Split vectors: one case per tile size of the rows kernel (1, 2, 4 quads, 1 or
+# 2 row tiles), then of the tile kernel (4 quads and halves of k, even and
+# uneven; 4 quads; 8 quads), last row and vector groups partly filled, and a
+# group scale of three chunks.
 @pytest.mark.parametrize("fmt", [1, 3, 4, 6, 7])
-@pytest.mark.parametrize("rows,cols,batch,group", [(2040, 512, 353, 128), (2040, 512, 383, 128), (6100, 768, 129, 384)])
+@pytest.mark.parametrize("rows,cols,batch,group", [
+    (2040, 512, 13, 128), (2600, 768, 9, 384), (4090, 512, 13, 128), (4090, 512, 30, 128),
+    (2040, 512, 353, 128), (6100, 768, 129, 384), (16380, 512, 70, 128), (16380, 512, 125, 128)])
 def test_digit_tiles(cuda, fmt, rows, cols, batch, group):
     planes, scales, g, w = make(fmt, rows, cols, seed=7 + fmt, group=group)
     x = vectors(batch, cols, seed=50)
