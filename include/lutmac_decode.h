@@ -105,13 +105,15 @@ int lmx_decoder_reset(lmx_decoder *d, const int32_t *tokens, size_t n);
 int lmx_decoder_step(lmx_decoder *d, float *d_logits, void *stream);
 /* Copies tokens[0..n) of the device token buffer to the host (synchronous). */
 int lmx_decoder_tokens(lmx_decoder *d, int32_t *out, size_t n, void *stream);
-/* Greedy generation as inference.cpp does it (prompt token by token, then
- * n_new tokens), with the step captured once in a HIP graph and replayed.
+/* Greedy generation with the results of inference.cpp's loop (prompt token by
+ * token, then n_new tokens).  All but the last position of a prompt of more
+ * than 4 tokens go through the layers in passes of up to 512 rows; for
+ * more than 3 new tokens the step is captured in a HIP graph and replayed.
  * out_tokens (host) receives n_prompt + n_new tokens.  The work runs on the
  * decoder's own stream after the work already queued on `stream`; the call
- * returns when it is done.  Timings (ms, HIP events): prefill = the n_prompt
- * steps over the prompt (the last one yields the first new token), decode =
- * the n_new - 1 steps that yield the remaining tokens. */
+ * returns when it is done.  Timings (ms, HIP events): prefill = the prompt,
+ * whose last position yields the first new token, decode = the n_new - 1
+ * steps that yield the remaining tokens. */
 int lmx_decoder_generate(lmx_decoder *d, const int32_t *prompt, size_t n_prompt,
                          size_t n_new, int32_t *out_tokens, float *prefill_ms,
                          float *decode_ms, void *stream);
