@@ -60,6 +60,7 @@ __global__ __launch_bounds__(1024) void digit_gemv_kernel(GemvArgs a, int nv) {
   const int pairs = a.Kp / kRotChunk;
   const bool rot = a.rotate == LMX_ROTATE_FWHT256;
   const DigitLane dl(lane);
+  const v4i start = sum_start();
 
   // first row of each tile; PAIR: RT/2 tiles of gate rows, then the matching up rows
   uint32_t row0[RT];
@@ -185,7 +186,7 @@ __global__ __launch_bounds__(1024) void digit_gemv_kernel(GemvArgs a, int nv) {
 #pragma unroll
       for (int t = 0; t < RT; ++t)
 #pragma unroll
-        for (int s = 0; s < S; ++s) sum[t][s] = v4i{0, 0, 0, 0};
+        for (int s = 0; s < S; ++s) sum[t][s] = start;
 #pragma unroll
       for (int q = 0; q < G; ++q) {
         const int ch = G * i + q;
@@ -291,6 +292,9 @@ __global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVecto
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
   const int li = lane & 15, kq = lane >> 4;
   const int Kc = a.Kp / kChunk;
+  constexpr bool TIGHT = NQ * RT > 4;   // of 128 registers a wave
+  v4i start = {0, 0, 0, 0};
+  if constexpr (!TIGHT) start = sum_start();
   const uint32_t Npad = uint32_t(a.Npad);
   const int quads = (d.count + 3) / 4, q0 = int(blockIdx.y) * NQ;
   const int slices = int(gridDim.z), slice = int(blockIdx.z);
@@ -338,8 +342,10 @@ __global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVecto
         uint32_t wb[8];
         source_bytes<FMT, COPY>(w[b][t], s, wb);
 #pragma unroll
-        for (int q = 0; q < NQ; ++q)
-          acc[t][q] = fmaf(join_digits(chunk_product(wb, f[b][q][0], f[b][q][1])) * sc[b][t][s], mu[b][q], acc[t][q]);
+        for (int q = 0; q < NQ; ++q) {
+          const v4i sum = chunk_product(wb, f[b][q][0], f[b][q][1], start);
+          acc[t][q] = fmaf((TIGHT ? join_digits_int(sum) : join_digits(sum)) * sc[b][t][s], mu[b][q], acc[t][q]);
+        }
       }
   };
   if (ch0 + wave < ch1) load(0, ch0 + wave);
@@ -413,11 +419,21 @@ __global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVecto
 
 // ---------------------------------------------------------------------------
 // Many vectors: 4 waves of RT row tiles x the same NQ quads, the quads'
-// fragments of a chunk staged in LDS (two chunks deep).
-constexpr int tile_waves(int nq, int ks) { return ks == 1 ? (nq == 8 ? 3 : 4) : nq == 8 ? 2 : 4; }
+// fragments of a chunk staged in LDS (two chunks deep); with KS = 2 a second
+// set of 4 waves takes every other pair of chunks and the two sums are added
+// at the end (half the serial chain where few workgroups are in flight).
+// Bound by instruction issue: per 64 products 192 float operations join the
+// sums and 64 unpack codes and address; products alone take 32 ns of the 73 ns
+// that 4 products and their share take a SIMD (8192 x 2048 x 512 vectors: 46 us
+// for 14 us of products).  So 4 waves per SIMD (128 registers) come first: 8
+// quads request fragments one chunk ahead, not two.  Halving the LDS reads (2 x
+// 2 waves of 4 row tiles) was 20 % slower for its extra unpacking.
+template <int FMT, bool COPY, int NQ> constexpr int tile_waves() {
+  return NQ == 8 && (Source<FMT, COPY>::CW > 4 || Fmt<FMT>::S > 1) ? 3 : 4;
+}
 
 template <int FMT, bool COPY, int NQ, int RT, int KS, int EPI>
-__global__ __launch_bounds__(256 * KS, tile_waves(NQ, KS)) void digit_tile_kernel(GemvArgs a, DigitVectors d) {
+__global__ __launch_bounds__(256 * KS, (tile_waves<FMT, COPY, NQ>())) void digit_tile_kernel(GemvArgs a, DigitVectors d) {
   constexpr int CW = Source<FMT, COPY>::CW, S = Fmt<FMT>::S;
   constexpr bool PAIR = EPI == kEpiSiluPair;
   constexpr int WAVES = 4;
@@ -428,6 +444,7 @@ __global__ __launch_bounds__(256 * KS, tile_waves(NQ, KS)) void digit_tile_kerne
   auto &frags = frags_all[kg];
   const int li = lane & 15, kq = lane >> 4;
   const int Kc = a.Kp / kChunk;
+  const v4i start = sum_start();
   const uint32_t Npad = uint32_t(a.Npad);
   const int quads = (d.count + 3) / 4, q0 = int(blockIdx.y) * NQ;
   const int wg = int(blockIdx.x) * WAVES + wave;   // the wave's group of RT tiles
@@ -444,25 +461,25 @@ __global__ __launch_bounds__(256 * KS, tile_waves(NQ, KS)) void digit_tile_kerne
   const size_t qbytes = size_t(Kc) * kQuadChunk;
   constexpr int LD = NQ * int(kQuadChunk) / (256 * 16);   // 16-byte pieces per thread and chunk
   static_assert(LD * 256 * 16 == NQ * int(kQuadChunk), "whole pieces");
-  // A chunk's codes and fragments are requested two chunks ahead (they come
-  // from the MALL where another XCD wrote or read them first); past the last
-  // chunk the last one is requested again.
+  // A chunk's codes (and fragments: FD) are requested two chunks ahead: they
+  // come from the MALL where another XCD wrote or read them first.  Past the
+  // last chunk the last one is requested again.
   uint32_t w[2][RT][CW];
   float sc[2][RT][S];
-  v4i st[2][LD];
-  const char *fsrc[LD];
+  constexpr int FD = NQ == 8 ? 1 : 2;   // chunks the fragments are requested ahead
+  v4i st[FD][LD];
+  const char *fsrc[LD];   // wave-uniform: a wave's piece i is half of quad 2 i + wave / 2
 #pragma unroll
-  for (int i = 0; i < LD; ++i) {
-    const int p = tid + 256 * i, q = p / 128, o = p % 128;
-    fsrc[i] = d.digits + size_t(min(q0 + q, quads - 1)) * qbytes + o * 16;
-  }
+  for (int i = 0; i < LD; ++i) fsrc[i] = d.digits + size_t(min(q0 + 2 * i + wave / 2, quads - 1)) * qbytes;
+  const uint32_t foff = uint32_t(tid % 128) * 16;
   const auto load_f = [&](int b, int ch) {
+    const size_t c = size_t(min(ch, Kc - 1)) * kQuadChunk;
 #pragma unroll
-    for (int i = 0; i < LD; ++i) st[b][i] = *reinterpret_cast<const v4i *>(fsrc[i] + size_t(min(ch, Kc - 1)) * kQuadChunk);
+    for (int i = 0; i < LD; ++i) st[b % FD][i] = *reinterpret_cast<const v4i *>(fsrc[i] + c + foff);
   };
   const auto store_f = [&](int b) {
 #pragma unroll
-    for (int i = 0; i < LD; ++i) *reinterpret_cast<v4i *>(frags[b] + (tid + 256 * i) * 16) = st[b][i];
+    for (int i = 0; i < LD; ++i) *reinterpret_cast<v4i *>(frags[b] + (tid + 256 * i) * 16) = st[b % FD][i];
   };
   const auto load_w = [&](int b, int ch) {
     ch = min(ch, Kc - 1);
@@ -481,7 +498,8 @@ __global__ __launch_bounds__(256 * KS, tile_waves(NQ, KS)) void digit_tile_kerne
 #pragma unroll
     for (int q = 0; q < NQ; ++q) acc[t][q] = 0.0f;
   const auto chunk = [&](int ch, const int b) {   // b = ch % 2
-    load_f(b, ch + 2 * KS);
+    if constexpr (FD == 2) load_f(b, ch + 2 * KS);
+    else load_f(b ^ 1, b == 0 ? ch + 1 : ch - 1 + 2 * KS);
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       uint32_t wb[RT][8];
@@ -508,7 +526,7 @@ __global__ __launch_bounds__(256 * KS, tile_waves(NQ, KS)) void digit_tile_kerne
         if (q + 1 < NQ) read(q + 1);
         if (q < NQ) {
 #pragma unroll
-          for (int t = 0; t < RT; ++t) sum[q & 1][t] = chunk_product(wb[t], f[q & 1][0], f[q & 1][1]);
+          for (int t = 0; t < RT; ++t) sum[q & 1][t] = chunk_product(wb[t], f[q & 1][0], f[q & 1][1], start);
         }
         if (q > 0) {
 #pragma unroll
@@ -525,7 +543,7 @@ __global__ __launch_bounds__(256 * KS, tile_waves(NQ, KS)) void digit_tile_kerne
   };
   load_f(0, 2 * kg);
   load_w(0, 2 * kg);
-  load_f(1, 2 * kg + 1);
+  if constexpr (FD == 2) load_f(1, 2 * kg + 1);
   load_w(1, 2 * kg + 1);
   store_f(0);
   __syncthreads();
