@@ -291,12 +291,13 @@ int stage_if_needed(const lmx_weight *w, GemvArgs &a, void *stream) {
 // 17.9 / 15.7).  *done = the vectors covered; `all`: every one, the single
 // vectors of those formats too (a.xmode and a.epi have no other form there).
 int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done,
-                 bool all) {
+                 bool all, void *scratch, size_t scratch_bytes) {
+  if (!scratch) scratch = w->d_digits, scratch_bytes = w->digit_cap;
   const float *resid = a.resid;
   const size_t out_rows = a.epi == kEpiSiluPair ? w->rows / 2 : w->rows;
   const bool copies = code_copy_bytes(w->format, 1, kRotChunk) != 0;
   // (the split kernels read the code copy where the format has one)
-  const size_t cap = w->d_digits && (!copies || w->d_codes) ? digit_capacity(w->Kp, w->digit_cap) : 0;
+  const size_t cap = scratch && (!copies || w->d_codes) ? digit_capacity(w->Kp, scratch_bytes) : 0;
   a.cols = int(w->cols);
   for (*done = 0; *done < batch;) {
     const size_t left = batch - *done;
@@ -311,7 +312,7 @@ int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size
     // ternary 11.4 against 9.4 split, 4-bit 8.0 / 9.1).
     if (cap && (left > 4 || (!copies && w->Kp > 4096 && (left > 1 || all)))) {
       n = std::min(left, cap);
-      const DigitVectors d = digit_vectors(w, w->d_digits, n);
+      const DigitVectors d = digit_vectors(w, scratch, n);
       if ((st = launch_digit_split(w->format, a, d, stream)) || (st = launch_digit_gemm(w->format, a, d, stream)))
         return st;
     } else {

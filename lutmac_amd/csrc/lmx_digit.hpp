@@ -184,8 +184,8 @@ __device__ __forceinline__ v4i sum_start() {
 // 256 d - kSumStart is exact, so each pair of digits rounds once, as a 32-bit
 // integer of the pair would.  Additions and multiply-adds only: integer shifts
 // and conversions take 1.6 times their issue time (1.95 against 1.2 ns per
-// SIMD; 8192 x 2048 x 384
-// vectors 39.7 to 38.6 us, RRQ-3 17920 x 1536 127 to 122).
+// SIMD; with 384 vectors, us: 8192 x 2048 39.7 to 38.6, RRQ-3 17920 x 1536 127
+// to 122).
 __device__ __forceinline__ float join_digits(const v4i d) {
   const float lo = fmaf(__int_as_float(d[1]), 256.0f, -257.0f * kSumStart) + __int_as_float(d[0]);
   const float hi = fmaf(__int_as_float(d[3]), 256.0f, -257.0f * kSumStart) + __int_as_float(d[2]);

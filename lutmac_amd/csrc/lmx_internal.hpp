@@ -253,7 +253,7 @@ int gemv_impl(const lmx_weight *w, const float *x, float *y, size_t batch, unsig
 GemvArgs weight_args(const lmx_weight *w);
 // y = W x of `batch` vectors on the digit kernels (a.bias, a.resid, a.rotate, a.xmode none or RMSNorm,
 // a.epi store or SiLU pair; x of any alignment); *done = the vectors covered, the rest (one by one on
-// the lookup tables) left to the caller unless `all`
+// the lookup tables) left to the caller unless `all`; scratch: for the split digits, else the handle's
 int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done,
-                 bool all);
+                 bool all, void *scratch = nullptr, size_t scratch_bytes = 0);
 }  // namespace lmx
