@@ -815,9 +815,21 @@ GemvArgs decode_args(const lmx_weight *w, int xmode, int epi) {
   return a;
 }
 
-// Whether one vector of this weight runs on the digit kernels (4 and 8 bits,
-// digit_linear's rule).
-bool one_on_digits(const lmx_weight *w) { return w->digit && w->d_codes; }
+// Whether a step's vector of this weight runs on the digit kernels: 4 and 8
+// bits as in digit_linear, but for 4-bit weights whose lookup plan has one
+// step per wave and a chunk for every k-slice.  Between a step's dependent
+// launches that plan finishes sooner, its tables being built from the
+// activations while the planes arrive, where the digits wait for a chunk's
+// maximum; with slices left empty it does not (us a step of 4 layers, digits
+// for all / for the others only: Llama-3.2-1B width, K of 2048 and 8192, 134.5
+// / 130.5; Qwen-2.5-1.5B width, K of 1536 and 8960, 135.8 / 141 with such plans
+// forced).
+bool one_on_digits(const lmx_weight *w) {
+  if (!w->digit || !w->d_codes) return false;
+  if (w->format != LMX_FMT_INT4 || w->fullk == kFullK_None) return true;
+  const FullKShape f = fullk_shape(w->fullk);
+  return f.cps > 1 || size_t(f.waves * f.h) != w->Kp / kChunk;
+}
 
 // Whether the digit kernels form SiLU(gate)*up in the gate|up epilogue (whole
 // row tiles in each half).
