@@ -149,10 +149,11 @@ int lmx_weight_read_tiles(const lmx_weight *w, uint8_t *tiles, size_t bytes);
 /* ---- compute (device pointers, asynchronous on `stream`; NULL = default) */
 /* y[b*rows + r] = sum_k W[r,k] * R(x[b*cols + .])[k] for b < batch, where R is
  * the rotation selected by flags.  x holds `cols` floats per batch row (the
- * kernel zero-extends to the padded width).  With batch >= 4 (x 16-byte
- * aligned, cols % 4 == 0) groups of 16/8/4 rows share one pass over the
- * weights, through scratch allocated with the handle (no call allocates,
- * so calls can be captured into a HIP graph).  Replaces the raw per-format
+ * kernel zero-extends to the padded width).  The rows of a batch share
+ * one pass over the weights, up to 4 in one launch, more through scratch
+ * allocated with the handle (no call allocates, so calls can be captured
+ * into a HIP graph).  A vector of 4- or 8-bit weights, or of any batch, with
+ * an element that is not finite gives NaN in all of its outputs.  Replaces the raw per-format
  * dispatchers lut_gemv / lut_gemv_binary / int2_gemv / int3_gemv /
  * int4_gemv / int8_gemv (lut_gemm.hpp:172-408). */
 int lmx_gemv(const lmx_weight *w, const float *x, float *y, size_t batch,
@@ -183,12 +184,12 @@ int lmx_extract_indices(const uint8_t *sign_plane, const uint8_t *zero_plane,
  * the lmx_tile_scales layout; format, rows, cols, group, x, y, batch, flags
  * and stream mean what they mean for lmx_gemv, with the same kernel plan, so
  * y is bit-identical to lmx_gemv's for up to 4 vectors (larger batches run in
- * groups of 4).  It allocates nothing: the split-K partials, ticket counters and the staging
- * copy of x live in an 8 MiB device array that each GPU holds until the
- * process ends: a fixed 64 KiB of split-K ticket counters (one per 64-row
- * block), then the staging copy of x (Kp*4 B), then the split-K partials
- * ((Kp/kslice)*Npad*4 B); shapes needing more return
- * LMX_ERR_INVALID_ARGUMENT.  The first call on a device looks the array up,
+ * groups of 4).  It allocates nothing: the split-K partials, ticket counters
+ * and the staging copy of x live in an 8 MiB device array that each GPU holds
+ * until the process ends: a fixed 64 KiB of split-K ticket counters (one per
+ * 64-row block), then the staging copy of x (Kp*4 B), then the split-K
+ * partials ((Kp/kslice)*Npad*4 B) or the digits of up to 4 vectors; shapes
+ * whose staging and partials need more return LMX_ERR_INVALID_ARGUMENT.  The first call on a device looks the array up,
  * zeroes it with a kernel on `stream` and waits for that kernel before it
  * returns or launches anything else, so make it outside graph capture; every
  * later call, on any stream or thread, then finds the counters zeroed.  Calls

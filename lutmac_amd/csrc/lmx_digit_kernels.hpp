@@ -35,6 +35,12 @@ __device__ __forceinline__ int scale_group(const GemvArgs &a, int ch) {
 // 3, zeros elsewhere), so four chunks' digit sums land in four lane groups of
 // one accumulator and are joined and scaled once.
 // NV = 4: one accumulator per chunk, its four lane groups the four vectors.
+// From about 20 MB of codes bound by HBM (4-bit 8192 x 8192 7.5 us, 4.8 TB/s,
+// 8.0 on the lookup tables; 8-bit 15.2 us, 4.6 TB/s, 16.5), below that by one
+// chain of launch, activations, digits, products and the waves' sum: so every
+// load of a round is requested at the start, activations first, and 16 waves
+// share the K.  Four vectors cost 4-bit 17920 x 1536 6.9 us where the bf16
+// matrix cores and their reduction took 10.8.
 template <int FMT, bool COPY, int NV, int RT, int PPW, int XM, int EPI>
 __global__ __launch_bounds__(1024) void digit_gemv_kernel(GemvArgs a, int nv) {
   constexpr int CW = Source<FMT, COPY>::CW, S = Fmt<FMT>::S;
@@ -281,6 +287,12 @@ __device__ __forceinline__ float vector_scale(float sum, float fac, int ex) {
 // one slice the workgroups of a row block leave their sums in d.partials and
 // the last one to finish (a ticket) adds them in slice order: agent-scope
 // relaxed stores and loads, which need no write-back of the XCDs' L2s.
+// Bound by the latency of a wave's one or two chunks (codes, digits, scales in
+// one round trip, the second chunk's requested before the first is used):
+// hence small tiles, k over 16 waves and slices up to a workgroup per CU.  us,
+// with the split, before on the bf16 matrix cores or lookup tables: 4-bit 1536
+// x 8960 x 16 vectors 10.9 to 9.0, 3001 x 1400 x 13 17.7 to 8.3, ternary 2048 x
+// 2048 x 64 34.3 to 8.6.
 template <int FMT, bool COPY, int NQ, int RT, int EPI>
 __global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVectors d) {
   constexpr int CW = Source<FMT, COPY>::CW, S = Fmt<FMT>::S;
@@ -717,6 +729,8 @@ int launch_digit_gemv_fmt(const GemvArgs &a, int nv, hipStream_t st) {
 }
 
 // The code copy of 4- and 8-bit planes: one thread per plane word of a row.
+// HBM-bound (128256 x 2048 of 4 bits: 42 us); made here and not on the host,
+// creating a 17920 x 1536 handle takes 2 ms where it took 13.
 template <int FMT>
 __global__ __launch_bounds__(256) void code_copy_kernel(const uint32_t *__restrict__ planes, uint32_t Npad, size_t n,
                                                         uint32_t *__restrict__ codes) {

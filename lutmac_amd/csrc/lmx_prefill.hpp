@@ -15,7 +15,8 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 // RoPE of the pass's q (in place) and k, k and v appended to the cache: the
 // decode attention's rotation (pairs (d, d + HD/2), each product rounded).
-// One thread per pair; blockIdx.y = row.
+// One thread per pair; blockIdx.y = row.  Latency-bound: 5 us for 383 rows of
+// 3072 (4.7 MB read, 6.3 MB written).
 template <int HD>
 __global__ __launch_bounds__(256) void prefill_rope_kernel(float *__restrict__ qkv, const float2 *__restrict__ rope,
                                                            float *__restrict__ kc, float *__restrict__ vc, int n_heads,
@@ -58,6 +59,9 @@ __global__ __launch_bounds__(256) void prefill_rope_kernel(float *__restrict__ q
 //     C lane (r, g) item v = key 4 g + v of the tile;
 //   O^T = V^T P^T: step v takes key 4 kk + v from lane group kk, which is where
 //     S^T left it, so P needs no transpose; A lane (dim, kk) = V[4 kk + v][dim].
+// Bound by the serial chain over the last rows' key tiles: 32 heads of 64, 383
+// positions 18 us, where one position's step takes 5.6 us in attention.  The 4
+// waves share the keys, not the rows, to shorten that chain.
 template <int HD>
 __global__ __launch_bounds__(256) void prefill_attention_kernel(const float *__restrict__ qkv,
                                                                 const float *__restrict__ kc,
