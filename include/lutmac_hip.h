@@ -135,7 +135,8 @@ int lmx_weight_destroy(lmx_weight *w);
 /* Format, shape and device bytes (planes + scales) of a handle. */
 int lmx_weight_info(const lmx_weight *w, int *format, size_t *rows,
                     size_t *cols, size_t *device_bytes);
-/* Kernel plan chosen for a handle at creation: full-K configuration
+/* Lookup-table plan chosen for a handle at creation (calls on the digit
+ * kernels do not use it): full-K configuration
  * (0 = split-K kernel, 1..6 = LMX_FULLK values), split-K k-slice, and
  * whether the full-K kernel stages its weight loads.  Diagnostic only; the
  * environment variables LMX_FULLK, LMX_KSLICE, LMX_WAVES, LMX_STAGED and
