@@ -835,13 +835,14 @@ bool one_on_digits(const lmx_weight *w) {
 // row tiles in each half).
 bool digit_pairs(const lmx_weight *gate_up) { return gate_up->rows % 32 == 0; }
 
-// The gate|up launch writes SiLU(gate)*up itself (kEpiSiluPair) where its
-// kernel plan serves that epilogue; else (or with LMX_SILU_PAIR=0) the down
-// projection forms it in its table prologue.
+// The gate|up launch writes SiLU(gate)*up itself (kEpiSiluPair) where the
+// kernel that gemv() sends it to serves that epilogue; else (or with
+// LMX_SILU_PAIR=0) the down projection forms it in its table prologue.
 bool gate_up_pairs(const lmx_weight *gate_up) {
   const char *e = std::getenv("LMX_SILU_PAIR");
-  if ((!e || std::atoi(e) != 0) && one_on_digits(gate_up) && digit_pairs(gate_up)) return true;
-  return (!e || std::atoi(e) != 0) && silu_pair_rows(gate_up->format, decode_args(gate_up, kXModeRmsNorm, kEpiSiluPair)) > 0;
+  if (e && std::atoi(e) == 0) return false;
+  if (one_on_digits(gate_up)) return digit_pairs(gate_up);
+  return silu_pair_rows(gate_up->format, decode_args(gate_up, kXModeRmsNorm, kEpiSiluPair)) > 0;
 }
 
 int gemv(const lmx_weight *w, const float *x, float *y, const float *bias, int xmode, const float *xw, float eps,

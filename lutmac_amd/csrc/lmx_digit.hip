@@ -168,7 +168,19 @@ int digit_gemv_tiles(const GemvArgs &a) {
 
 size_t digit_argmax_slots(const GemvArgs &a) { return size_t(a.Npad) / (kTile * digit_gemv_tiles(a)); }
 
+// The epilogues and transforms every digit kernel serves: a SiLU pair has
+// whole 16-row tiles in each half.
+static int check_digit_args(const GemvArgs &a, bool norm_pairs) {
+  const bool pair = a.epi == kEpiSiluPair;
+  if (pair && a.rows % (2 * kTile))
+    return fail(LMX_ERR_INVALID_ARGUMENT, "a SiLU pair of %d rows has no whole row tiles", a.rows);
+  if ((a.xmode != kXModeNone && a.xmode != kXModeRmsNorm) || (pair && norm_pairs && a.xmode != kXModeRmsNorm))
+    return fail(LMX_ERR_INVALID_ARGUMENT, "the digit kernels do not serve transform %d with epilogue %d", a.xmode, a.epi);
+  return LMX_OK;
+}
+
 int launch_digit_gemv(int fmt, const GemvArgs &a, int nv, void *stream) {
+  if (const int st = check_digit_args(a, true)) return st;
   switch (fmt) {
   case LMX_FMT_TERNARY: return digit_gemv_fmt<LMX_FMT_TERNARY>(a, nv, stream);
   case LMX_FMT_BINARY: return digit_gemv_fmt<LMX_FMT_BINARY>(a, nv, stream);
@@ -241,6 +253,7 @@ int launch_digit_split(int fmt, const GemvArgs &a, const DigitVectors &d, void *
 }
 
 int launch_digit_gemm(int fmt, const GemvArgs &a, const DigitVectors &d, void *stream) {
+  if (const int st = check_digit_args(a, false)) return st;
   if (code_copy_bytes(fmt, 1, kRotChunk) && !a.codes)
     return fail(LMX_ERR_INVALID_ARGUMENT, "the split digit kernels need the code copy of format %d", fmt);
   switch (fmt) {

@@ -18,6 +18,7 @@ import lutmac_amd as L
 import oracle
 from conftest import rel_max_err
 from lutmac_amd import decode as D
+from lutmac_amd import synth
 
 pytestmark = pytest.mark.gpu
 
@@ -124,6 +125,24 @@ def test_decoder_silu_pair_epilogue(cuda, monkeypatch, ffn, ps):
         want = ref.step(t, pos)
         assert rel_max_err(paired[pos], unpaired[pos]) < 1e-6, pos
         assert rel_max_err(paired[pos], want) < DECODE_TOL, pos
+
+
+# 4-bit gate|up whose halves hold no whole 16-row tiles, on lookup plans with
+# idle k-slices (so the digit kernels run it): the 4 x 4 x 1 plan (K 256) and
+# the 8 x 8 x 1 plan (K 2304).  SiLU(gate)*up then has every row.
+@pytest.mark.parametrize("hidden,ffn,plan", [(256, 264, 6), (512, 1000, 6), (2304, 72, 5)])
+def test_decoder_silu_pair_ragged_ffn(cuda, hidden, ffn, plan):
+    cfg = D.small_config(hidden=hidden, ffn=ffn, vocab=400, rope_mode=D.ROPE_REFERENCE, rope_factor=1.0,
+                         rope_theta=1e6)
+    formats = {n: (L.FMT_INT4, 128, 0) for n in ("q", "k", "v", "o", "gate", "up", "embed")}
+    m = D.QuantizedModel(cfg, {**formats, "down": (L.FMT_BINARY, 128, 0)}, seed=45 + ffn)
+    for i, layer in enumerate(m.layers):   # 4 bits, one scale a row (the oracle's groups are whole)
+        planes, scales, _ = synth.make_weights(L.FMT_INT4, hidden, ffn, seed=i, group=128)
+        layer["down"] = (planes, np.ascontiguousarray(scales[:, :, :1]), L.FMT_INT4, 0)
+    toks = np.random.default_rng(46).integers(0, cfg.vocab, 6)
+    dec = D.Decoder(m)
+    assert dec.weights[2].kernel_config()[0] == plan
+    check_against(dec, oracle.OracleDecoder(m), toks)
 
 
 @pytest.mark.parametrize("hs", [None, "1", "group"])
