@@ -165,9 +165,10 @@ void plan_weight(lmx_weight *w, int fmt, size_t rows, size_t cols, size_t group)
   w->fullk = choose_fullk(fmt, w->Npad, w->Kp, w->kfamily);
   w->staged = choose_staged();
   // One vector of 4 or 8 bits on the digit kernels, unless a lookup-table plan
-  // was asked for.
+  // or form was asked for.
   w->digit = env_int("LMX_DIGIT", 1) != 0;
-  for (const char *name : {"LMX_FULLK", "LMX_KERNEL", "LMX_KSLICE", "LMX_REDUCE", "LMX_WAVES"})
+  for (const char *name : {"LMX_FULLK", "LMX_FULLK_WIDE", "LMX_KERNEL", "LMX_KSLICE", "LMX_PS", "LMX_REDUCE",
+                           "LMX_STAGED", "LMX_WAVES"})
     if (std::getenv(name)) w->digit = false;
 }
 

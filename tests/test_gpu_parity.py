@@ -267,6 +267,11 @@ def test_int4_plane_split(cuda, monkeypatch, ps, rows, cols):
     y = w.gemv(dev(x), flags=L.ROTATE_NONE).cpu().numpy()
     ref = oracle_planes_gemv(L.FMT_INT4, planes, scales, rows, cols, g, x, L.ROTATE_NONE)
     assert rel_max_err(y, ref) < TOL
+    # LMX_PS asks for the lookup tables: the bits of a handle that never runs the digit kernels
+    monkeypatch.setenv("LMX_DIGIT", "0")
+    tables = L.Weight.from_planes(L.FMT_INT4, planes, scales, rows, cols, g)
+    assert np.array_equal(tables.gemv(dev(x), flags=L.ROTATE_NONE).cpu().numpy().view(np.uint32), y.view(np.uint32))
+    tables.close()
     w.close()
 
 
