@@ -699,7 +699,10 @@ int launch_digit_gemv_rt(const GemvArgs &a, int nv, hipStream_t st) {
   const int per = (pairs + 15) / 16;
   const int W = (pairs + per - 1) / per;
   if constexpr (NV == 1) {
-    if (per >= 2) return launch_digit_gemv_cfg<FMT, COPY, NV, RT, 2>(a, nv, W, st);
+    // two 256-chunks per wave and round; in the last of several rounds few waves
+    // have a second one, so all 16 share them (us, W even over single chunks / 16:
+    // 256 x 8960 5.49 / 4.92, from planes 7.20 / 6.06)
+    if (per >= 2) return launch_digit_gemv_cfg<FMT, COPY, NV, RT, 2>(a, nv, per == 2 ? W : 16, st);
   }
   return launch_digit_gemv_cfg<FMT, COPY, NV, RT, 1>(a, nv, W, st);
 }
@@ -707,7 +710,15 @@ int launch_digit_gemv_rt(const GemvArgs &a, int nv, hipStream_t st) {
 template <int FMT, bool COPY>
 int launch_digit_gemv_src(const GemvArgs &a, int nv, hipStream_t st) {
   const bool two = digit_gemv_tiles(a) == 2;
-  if (nv == 1) return two ? launch_digit_gemv_rt<FMT, COPY, 1, 2>(a, nv, st) : launch_digit_gemv_rt<FMT, COPY, 1, 1>(a, nv, st);
+  if (nv == 1) {
+    // 8-bit codes of one vector from the planes: their loads are whole 16-byte
+    // rows side by side, the copy's alternate 16 of a row's 32 bytes (us, copy /
+    // planes: 512 x 2048 3.89 / 3.48, 8192 x 8192 16.4 / 14.5, 512 x 8960 10.2 /
+    // 8.5; four vectors, whose codes come once for four products, 3.07 / 3.25 at
+    // 512 x 640, 6.16 / 6.35 at 8192 x 2048, 11.4 / 10.4 at 512 x 8960)
+    constexpr bool C = COPY && FMT != LMX_FMT_INT8;
+    return two ? launch_digit_gemv_rt<FMT, C, 1, 2>(a, nv, st) : launch_digit_gemv_rt<FMT, C, 1, 1>(a, nv, st);
+  }
   // Four row tiles share one making of four vectors' digits (us, two tiles /
   // four: 4-bit 10240 x 2048 5.76 / 5.26, 16384 x 4096 11.4 / 8.3, ternary
   // 32768 x 2048 14.1 / 12.1; 8192 x 2048 4.34 / 5.18, 17920 x 1536 7.3 / 8.3).

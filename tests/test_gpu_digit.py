@@ -183,3 +183,22 @@ def test_one_vector_route(cuda, monkeypatch, rows, cols, tables):
     check(L.FMT_INT4, planes, scales, rows, cols, g, x.cpu().numpy(), a.cpu().numpy()[None], rotate=False)
     w.close()
     lut.close()
+
+
+# The digits' products with codes read from the planes (no handle, so no code
+# copy; 8 bits: one vector of a handle too): the handle's bits, for one and two
+# row tiles, one and more 256-chunks per wave, the last of them alone.
+@pytest.mark.parametrize("fmt", [L.FMT_INT4, L.FMT_INT8])
+@pytest.mark.parametrize("rows,cols", [(70, 256), (300, 2560), (8190, 1000), (130, 8960), (65, 16640)])
+@pytest.mark.parametrize("batch", [1, 3])
+def test_digit_codes_from_planes(cuda, fmt, rows, cols, batch):
+    planes, scales, g, w = make(fmt, rows, cols, seed=rows + cols)
+    tiles = torch.from_numpy(L.tile_planes(fmt, planes, rows, cols)).cuda()
+    sc = torch.from_numpy(L.tile_scales(fmt, scales, rows, cols, g)).cuda()
+    x = torch.from_numpy(vectors(batch, cols, seed=rows)).cuda()
+    y = torch.full((batch * rows,), torch.nan, device="cuda")
+    L.gemv_tiles_noalloc(fmt, tiles, sc, rows, cols, g, x, y, batch)
+    a = w.gemv(x)
+    assert torch.equal(y, a)
+    check(fmt, planes, scales, rows, cols, g, x.cpu().numpy(), a.cpu().numpy().reshape(batch, rows), rotate=False)
+    w.close()
