@@ -12,18 +12,20 @@ template <int FMT> int code_copy_fmt(const void *planes, size_t Npad, size_t Kp,
 namespace {
 
 // ---------------------------------------------------------------------------
-// Digits of many vectors relative to each vector, one workgroup per vector
-// (tile form): dig[quad][chunk][step][lane][16 B].  Bound by the latency of the
-// row's read and its maximum; up to K = 8192 the row stays in registers between
-// the passes (512 vectors of 2048: 4.4 us, once a call, where every row block of
-// the products would make them again).
+// Digits of many vectors, one workgroup per vector (tile form):
+// dig[quad][chunk][step][lane][16 B].  Relative to the vector's largest, which
+// saves the products a multiplier per chunk, where every 128-chunk's own largest
+// is within 2^-6 of it: the fixed point then ends 2^-24 or less below a chunk's
+// largest.  Else (d.exp kFarVector) relative to each chunk's.  Bound by the
+// latency of the row's read and its maximum; up to K = 8192 the row stays in
+// registers between the passes (512 vectors of 2048: 4.4 us, once a call, where
+// every row block of the products would make them again).
 template <bool ROT, int XM>
 __global__ __launch_bounds__(512) void digit_split_kernel(const float *__restrict__ x, int cols, int Kp,
                                                           const float *__restrict__ xw, float eps, float factor,
-                                                          char *__restrict__ dig, float *__restrict__ vfac,
-                                                          int *__restrict__ vexp) {
+                                                          DigitVectors d) {
   constexpr int NW = 8;
-  __shared__ uint32_t mx[NW];
+  __shared__ uint32_t mx[NW], mn[NW];
   __shared__ float ssw[NW];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int v = blockIdx.x;
@@ -47,52 +49,60 @@ __global__ __launch_bounds__(512) void digit_split_kernel(const float *__restric
   };
   constexpr int KEEP = 4;   // 256-chunks of a wave kept between the passes (K <= 8192)
   float keep[KEEP][4];
-  uint32_t m = 0;
+  uint32_t hi = 0, lo = 0xFFFFFFFFu;   // largest chunk maximum, smallest one less 1 (of zeros: the largest number)
+  const auto look = [&](const float (&o)[4]) {
+    const uint32_t m = chunk_max_bits(o);
+    hi = max(hi, m);
+    lo = min(lo, m - 1u);
+  };
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
     if (wave + j * NW < pairs) {
       values(wave + j * NW, keep[j]);
-#pragma unroll
-      for (int b = 0; b < 4; ++b) m = max(m, __float_as_uint(keep[j][b]) & 0x7FFFFFFFu);
+      look(keep[j]);
     }
   }
   for (int c2 = wave + KEEP * NW; c2 < pairs; c2 += NW) {
     float o[4];
     values(c2, o);
-#pragma unroll
-    for (int b = 0; b < 4; ++b) m = max(m, __float_as_uint(o[b]) & 0x7FFFFFFFu);
+    look(o);
   }
-  m = row_max(m);
-  m = max(m, lane_xor_u32<16>(m, lane));
-  m = max(m, lane_xor_u32<32>(m, lane));
+  hi = max(hi, lane_xor_u32<32>(hi, lane));
+  lo = min(lo, lane_xor_u32<32>(lo, lane));
   if constexpr (XM == kXModeRmsNorm) ss = lane_sum<32>(ss, lane);
   if (lane == 0) {
-    mx[wave] = m;
+    mx[wave] = hi;
+    mn[wave] = lo;
     ssw[wave] = ss;
   }
   __syncthreads();
   float sum = 0.0f;
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
-    m = max(m, mx[i]);
+    hi = max(hi, mx[i]);
+    lo = min(lo, mn[i]);
     sum += ssw[i];
   }
-  const int e = split_exponent(m);
+  const bool finite = hi < kNotFinite;
+  const bool far = finite && lo < hi - min(hi, 6u << 23);
   if (threadIdx.x == 0) {
     float f = factor;
     if constexpr (XM == kXModeRmsNorm) f *= 1.0f / sqrtf(sum / float(cols) + eps);
-    vfac[v] = m >= kNotFinite ? __builtin_nanf("") : f;
-    vexp[v] = e - 156;
+    d.fac[v] = finite ? f : __builtin_nanf("");
+    d.exp[v] = far ? kFarVector : split_exponent(hi) - 156;
   }
   const int t = 7 - dl.kl;
-  char *base = dig + size_t(v >> 2) * (size_t(Kp / kChunk) * kQuadChunk) + (t >> 2) * 1024 +
-               (dl.kq * 16 + (v & 3) * 4) * 16 + (t & 3) * 4;
+  const size_t first = size_t(v >> 2) * size_t(Kp / kChunk);
+  char *base = d.digits + first * kQuadChunk + (t >> 2) * 1024 + (dl.kq * 16 + (v & 3) * 4) * 16 + (t & 3) * 4;
   const auto emit = [&](int c2, const float (&o)[4]) {
+    const int e = split_exponent(far ? chunk_max_bits(o) : hi);
     uint32_t dg[4];
     digits4(o, e, dg);
     char *dst = base + size_t(2 * c2 + dl.c) * kQuadChunk;
 #pragma unroll
     for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t *>(dst + q * 16) = dg[q];
+    if (far && (lane & 31) == 0)
+      d.mult[(first + size_t(2 * c2 + dl.c)) * 4 + (v & 3)] = __builtin_amdgcn_ldexpf(1.0f, e - 156);
   };
 #pragma unroll
   for (int j = 0; j < KEEP; ++j)
@@ -201,7 +211,7 @@ static float code_factor(int fmt, unsigned rotate) {
   return (rotate == LMX_ROTATE_FWHT256 ? 0.0625f : 1.0f) / float(1 << sh);
 }
 
-// digits, mult (rows form), fac and exp of `vectors` vectors
+// digits, mult, fac and exp of `vectors` vectors
 size_t digit_bytes(size_t Kp, size_t vectors) {
   const size_t quads = (vectors + 3) / 4;
   return quads * (Kp / kChunk) * (kQuadChunk + 16) + quads * 32;
@@ -242,7 +252,7 @@ int launch_digit_split(int fmt, const GemvArgs &a, const DigitVectors &d, void *
     return launched("digit_split_chunks");
   }
 #define LMX_SP(R, XM) \
-  digit_split_kernel<R, XM><<<dim3(unsigned(d.count)), dim3(512), 0, st>>>(a.x, a.cols, a.Kp, a.xw, a.eps, f, d.digits, d.fac, d.exp)
+  digit_split_kernel<R, XM><<<dim3(unsigned(d.count)), dim3(512), 0, st>>>(a.x, a.cols, a.Kp, a.xw, a.eps, f, d)
   if (a.xmode == kXModeRmsNorm) {
     if (rot) LMX_SP(true, kXModeRmsNorm); else LMX_SP(false, kXModeRmsNorm);
   } else {

@@ -484,6 +484,8 @@ __global__ __launch_bounds__(256 * KS, (tile_waves<FMT, COPY, NQ>())) void digit
 #pragma unroll
   for (int i = 0; i < LD; ++i) fsrc[i] = d.digits + size_t(min(q0 + 2 * i + wave / 2, quads - 1)) * qbytes;
   const uint32_t foff = uint32_t(tid % 128) * 16;
+  // exponents of the workgroup's vectors, in every wave: lane 4 q + n that of vector n of quad q
+  const int ex_lane = d.exp[min(4 * q0 + lane % (4 * NQ), d.count - 1)];
   const auto load_f = [&](int b, int ch) {
     const size_t c = size_t(min(ch, Kc - 1)) * kQuadChunk;
 #pragma unroll
@@ -564,6 +566,35 @@ __global__ __launch_bounds__(256 * KS, (tile_waves<FMT, COPY, NQ>())) void digit
     chunk(c0 + 2 * kg, 0);
     chunk(c0 + 2 * kg + 1, 1);
   }
+  // Far vectors (rare): their sums start again, chunk by chunk with the chunk's
+  // multiplier, a quad at a time straight from memory; the others add 0.
+  const uint64_t far = __builtin_amdgcn_ballot_w64(ex_lane == kFarVector);   // bit 4 q + n: vector n of quad q
+  if (far) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int t = 0; t < RT; ++t) acc[t][q] = (far >> (4 * q + kq)) & 1 ? 0.0f : acc[t][q];
+#pragma unroll 1
+    for (int ch = kg; ch < Kc; ch += KS) {
+      load_w(0, ch);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        if (!((far >> (4 * q)) & 15)) continue;   // wave-uniform
+        const size_t qc = size_t(min(q0 + q, quads - 1)) * Kc + ch;
+        const v4i *src = reinterpret_cast<const v4i *>(d.digits + qc * kQuadChunk) + lane;
+        const v4i f0 = src[0], f1 = src[64];
+        const float mu = (far >> (4 * q + kq)) & 1 ? d.mult[qc * 4 + kq] : 0.0f;
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+          for (int s = 0; s < S; ++s) {
+            uint32_t wb[8];
+            source_bytes<FMT, COPY>(w[0][t], s, wb);
+            acc[t][q] = fmaf(join_digits(chunk_product(wb, f0, f1, start)) * mu, sc[0][t][s], acc[t][q]);
+          }
+      }
+    }
+  }
   if constexpr (KS > 1) {   // the parts of k, in order
     float *red = reinterpret_cast<float *>(frags_all[0][0]);
     constexpr int SUMS = RT * NQ * 256;
@@ -588,7 +619,7 @@ __global__ __launch_bounds__(256 * KS, (tile_waves<FMT, COPY, NQ>())) void digit
     const int vec = 4 * (q0 + q) + kq;
     if (vec >= d.count) continue;
     const float fac = d.fac[vec];
-    const int ex = d.exp[vec];
+    const int ev = d.exp[vec], ex = ev == kFarVector ? 0 : ev;
 #pragma unroll
     for (int t = 0; t < (PAIR ? RT / 2 : RT); ++t) {
       float v = vector_scale(acc[t][q], fac, ex);

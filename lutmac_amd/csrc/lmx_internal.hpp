@@ -173,12 +173,13 @@ int silu_pair_rows(int fmt, const GemvArgs &a);
 struct DigitVectors {
   char *digits;       // [quads of 4 vectors][Kp/128][2 KiB]
   float *fac;         // [count] factor of a vector's sums (norm, rotation, code scale; NaN: not finite)
-  int *exp;           // tile form: [count] the power of two of a vector's digits
-  float *mult;        // rows form: [quads][Kp/128][4] that of each vector's chunk
+  int *exp;           // tile form: [count] the power of two of a vector's digits, or kFarVector
+  float *mult;        // rows form and far vectors: [quads][Kp/128][4] that of each vector's chunk
   float *partials;    // rows form: sums of k-slices (kDigitPartials bytes)
   int count;
   int tile;           // for the tile kernel (many vectors and rows), else the rows kernel
 };
+constexpr int kFarVector = 0x7FFFFFFF;    // a vector whose chunks' digits each have their own power of two (d.mult)
 constexpr unsigned kDigitTickets = 256;   // row blocks of a sliced rows launch, at most
 // Bytes of slice sums: up to 256 workgroups of 2 row tiles x 4 quads x 64 sums.
 constexpr size_t kDigitPartials = 256 * 512 * sizeof(float);

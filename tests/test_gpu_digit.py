@@ -202,3 +202,41 @@ def test_digit_codes_from_planes(cuda, fmt, rows, cols, batch):
     assert torch.equal(y, a)
     check(fmt, planes, scales, rows, cols, g, x.cpu().numpy(), a.cpu().numpy().reshape(batch, rows), rotate=False)
     w.close()
+
+
+# One channel far above the rest, which the rows have no weight for (the planes'
+# code of 0 in its columns): what it leaves of the other channels counts in full.
+# An output is then off by the rounding of its own terms alone, each 128-chunk's
+# fixed point relative to that chunk's largest.
+def zero_columns(fmt, planes, cols):
+    """The code of weight 0 in these columns of canonical planes."""
+    one = {L.FMT_TERNARY: 1, L.FMT_INT4: 3}.get(fmt)      # the one plane whose bit is set there
+    for k in cols:
+        bit = 1 << (7 - k % 8)
+        planes[:, :, k // 8] &= 255 - bit
+        if one is not None:
+            planes[one, :, k // 8] |= bit
+    return planes
+
+
+SPIKES = [2.0 ** 10, 2.0 ** 20, 1e10]
+
+
+@pytest.mark.parametrize("fmt", [L.FMT_TERNARY, L.FMT_INT4, L.FMT_INT8])
+@pytest.mark.parametrize("spike", SPIKES)
+@pytest.mark.parametrize("rows,cols,batch", [(2050, 512, 1), (2050, 512, 3), (1030, 1024, 11), (16380, 512, 70),
+                                             (6100, 1280, 129)])
+def test_digit_far_channel_in_another_chunk(cuda, fmt, spike, rows, cols, batch):
+    planes, scales, g = synth.make_weights(fmt, rows, cols, seed=rows + fmt, group=128)
+    zero_columns(fmt, planes, range(128, 256))
+    w = L.Weight.from_planes(fmt, planes, scales, rows, cols, g)
+    x = np.random.default_rng(batch).standard_normal((batch, cols)).astype(np.float32)
+    x[:, 200] = spike
+    y = w.gemv(torch.from_numpy(x).cuda()).cpu().numpy().reshape(batch, rows)
+    W = synth.dequant_f64(fmt, planes, scales, rows, cols, g)
+    err = np.abs(y - x.astype(np.float64) @ W.T)
+    xc, wc = np.abs(x).reshape(batch, -1, 128), np.abs(W).reshape(rows, -1, 128)
+    big = xc.max(axis=2) @ wc.sum(axis=2).T
+    bound = (cols // 128 + 18) * EPS * (np.abs(x).astype(np.float64) @ np.abs(W).T) + 2.0 ** -30 * big
+    assert (err <= bound).all(), float((err / bound).max())
+    w.close()
