@@ -11,12 +11,27 @@ template <int FMT> int code_copy_fmt(const void *planes, size_t Npad, size_t Kp,
 
 namespace {
 
+// A lane's four activations of vector n of a quad's chunk qc: their digits, or
+// the activations themselves (16 bytes where the digits have 4 rows of 4).
+__device__ __forceinline__ void store_digits(const DigitVectors &d, size_t qc, int n, const DigitLane &dl,
+                                             const float (&o)[4], int e, bool wide) {
+  const int t = 7 - dl.kl;
+  char *dst = d.digits + qc * kQuadChunk + (t >> 2) * 1024 + (dl.kq * 16 + n * 4) * 16;
+  if (wide) {
+    *reinterpret_cast<float4 *>(dst + (t & 3) * 16) = make_float4(o[0], o[1], o[2], o[3]);
+    return;
+  }
+  uint32_t dg[4];
+  digits4(o, e, dg);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t *>(dst + q * 16 + (t & 3) * 4) = dg[q];
+}
+
 // ---------------------------------------------------------------------------
 // Digits of many vectors, one workgroup per vector (tile form):
 // dig[quad][chunk][step][lane][16 B].  Relative to the vector's largest, which
-// saves the products a multiplier per chunk, where every 128-chunk's own largest
-// is within 2^-6 of it: the fixed point then ends 2^-24 or less below a chunk's
-// largest.  Else (d.exp kFarVector) relative to each chunk's.  Bound by the
+// saves the products a multiplier per chunk, unless its values lie too far apart
+// (wide_chunks); then (d.exp kFarVector) relative to each chunk's.  Bound by the
 // latency of the row's read and its maximum; up to K = 8192 the row stays in
 // registers between the passes (512 vectors of 2048: 4.4 us, once a call, where
 // every row block of the products would make them again).
@@ -25,7 +40,7 @@ __global__ __launch_bounds__(512) void digit_split_kernel(const float *__restric
                                                           const float *__restrict__ xw, float eps, float factor,
                                                           DigitVectors d) {
   constexpr int NW = 8;
-  __shared__ uint32_t mx[NW], mn[NW];
+  __shared__ uint32_t mx[NW], wd[NW];
   __shared__ float ssw[NW];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int v = blockIdx.x;
@@ -49,60 +64,67 @@ __global__ __launch_bounds__(512) void digit_split_kernel(const float *__restric
   };
   constexpr int KEEP = 4;   // 256-chunks of a wave kept between the passes (K <= 8192)
   float keep[KEEP][4];
-  uint32_t hi = 0, lo = 0xFFFFFFFFu;   // largest chunk maximum, smallest one less 1 (of zeros: the largest number)
-  const auto look = [&](const float (&o)[4]) {
-    const uint32_t m = chunk_max_bits(o);
-    hi = max(hi, m);
-    lo = min(lo, m - 1u);
-  };
+  uint32_t m = 0;
 #pragma unroll
   for (int j = 0; j < KEEP; ++j) {
     if (wave + j * NW < pairs) {
       values(wave + j * NW, keep[j]);
-      look(keep[j]);
+      m = max(m, lane_max_bits(keep[j]));
     }
   }
   for (int c2 = wave + KEEP * NW; c2 < pairs; c2 += NW) {
     float o[4];
     values(c2, o);
-    look(o);
+    m = max(m, lane_max_bits(o));
   }
-  hi = max(hi, lane_xor_u32<32>(hi, lane));
-  lo = min(lo, lane_xor_u32<32>(lo, lane));
+  m = row_max(m);
+  m = max(m, lane_xor_u32<16>(m, lane));
+  m = max(m, lane_xor_u32<32>(m, lane));
   if constexpr (XM == kXModeRmsNorm) ss = lane_sum<32>(ss, lane);
   if (lane == 0) {
-    mx[wave] = hi;
-    mn[wave] = lo;
+    mx[wave] = m;
     ssw[wave] = ss;
   }
   __syncthreads();
   float sum = 0.0f;
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
-    hi = max(hi, mx[i]);
-    lo = min(lo, mn[i]);
+    m = max(m, mx[i]);
     sum += ssw[i];
   }
-  const bool finite = hi < kNotFinite;
-  const bool far = finite && lo < hi - min(hi, 6u << 23);
+  const int ev = split_exponent(m);
+  bool far = false;
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j)
+    if (wave + j * NW < pairs) far |= wide_chunks(lane_max_bits(keep[j]), ev) != 0;
+  for (int c2 = wave + KEEP * NW; c2 < pairs; c2 += NW) {
+    float o[4];
+    values(c2, o);
+    far |= wide_chunks(lane_max_bits(o), ev) != 0;
+  }
+  if (lane == 0) wd[wave] = far;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NW; ++i) far |= wd[i] != 0;
+  if (m >= kNotFinite) far = false;
   if (threadIdx.x == 0) {
     float f = factor;
     if constexpr (XM == kXModeRmsNorm) f *= 1.0f / sqrtf(sum / float(cols) + eps);
-    d.fac[v] = finite ? f : __builtin_nanf("");
-    d.exp[v] = far ? kFarVector : split_exponent(hi) - 156;
+    d.fac[v] = m >= kNotFinite ? __builtin_nanf("") : f;
+    d.exp[v] = far ? kFarVector : ev - 156;
   }
-  const int t = 7 - dl.kl;
   const size_t first = size_t(v >> 2) * size_t(Kp / kChunk);
-  char *base = d.digits + first * kQuadChunk + (t >> 2) * 1024 + (dl.kq * 16 + (v & 3) * 4) * 16 + (t & 3) * 4;
   const auto emit = [&](int c2, const float (&o)[4]) {
-    const int e = split_exponent(far ? chunk_max_bits(o) : hi);
-    uint32_t dg[4];
-    digits4(o, e, dg);
-    char *dst = base + size_t(2 * c2 + dl.c) * kQuadChunk;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t *>(dst + q * 16) = dg[q];
-    if (far && (lane & 31) == 0)
-      d.mult[(first + size_t(2 * c2 + dl.c)) * 4 + (v & 3)] = __builtin_amdgcn_ldexpf(1.0f, e - 156);
+    const size_t qc = first + size_t(2 * c2 + dl.c);
+    int e = ev;
+    bool wide = false;
+    if (far) {
+      const uint32_t lm = lane_max_bits(o), mb = chunk_max_bits(lm);
+      e = split_exponent(mb);
+      wide = (wide_chunks(lm, e) >> dl.c) & 1;
+      if ((lane & 31) == 0) d.mult[qc * 4 + (v & 3)] = chunk_mult(mb, e, wide);
+    }
+    store_digits(d, qc, v & 3, dl, o, e, wide);
   };
 #pragma unroll
   for (int j = 0; j < KEEP; ++j)
@@ -152,17 +174,12 @@ __global__ __launch_bounds__(256) void digit_split_chunks_kernel(const float *__
   }
   if (c2 * kRotChunk >= Kp) return;   // wave-uniform; no barrier follows
   if (rotate == LMX_ROTATE_FWHT256) fwht256_regs_x16(o[0], o[1], o[2], o[3], lane);
-  const uint32_t mb = chunk_max_bits(o);
+  const uint32_t lm = lane_max_bits(o), mb = chunk_max_bits(lm);
   const int e = split_exponent(mb);
-  uint32_t dg[4];
-  digits4(o, e, dg);
-  const int t = 7 - dl.kl;
+  const bool wide = (wide_chunks(lm, e) >> dl.c) & 1;
   const size_t qc = size_t(v >> 2) * size_t(Kp / kChunk) + size_t(2 * c2 + dl.c);
-  char *dst = d.digits + qc * kQuadChunk + (t >> 2) * 1024 + (dl.kq * 16 + (v & 3) * 4) * 16 + (t & 3) * 4;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t *>(dst + q * 16) = dg[q];
-  if ((lane & 31) == 0)
-    d.mult[qc * 4 + (v & 3)] = mb >= kNotFinite ? __builtin_nanf("") : __builtin_amdgcn_ldexpf(1.0f, e - 156);
+  store_digits(d, qc, v & 3, dl, o, e, wide);
+  if ((lane & 31) == 0) d.mult[qc * 4 + (v & 3)] = chunk_mult(mb, e, wide);
 }
 
 }  // namespace

@@ -7,8 +7,11 @@
 // power of two at or above their largest magnitude, each split into four
 // signed bytes ("digits", v = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3); the weight
 // codes become signed bytes; v_mfma_i32_16x16x64_i8 sums their products
-// exactly.  Only the fixed point (below 2^-30 of the largest activation) and
-// the fp32 sums over chunks round.
+// exactly.  Only the fixed point (2^-31 of that power of two) and the joins and
+// fp32 sums over chunks round.  A chunk whose values lie too far apart for a
+// fixed point (wide_chunks) is multiplied in fp32 instead: its activations are
+// kept as they are in the place of their digits, its multiplier is 0, and
+// raw_sum adds their products.
 //
 // Matrix-core layout (A 16 x 64 = digits, B 64 x 16 = weights, C 16 x 16):
 //   A: lane (i = lane % 16, kq = lane / 16) holds row i's bytes of k-slot kq
@@ -190,17 +193,29 @@ __device__ __forceinline__ void source_bytes(const uint32_t *w, int s, uint32_t 
 }
 
 // Largest-magnitude bits of a 31-bit split: the biased exponent field e such
-// that every |x| < 2^(e - 126), from the largest |x|'s bits.  At least 8, so
-// that 2^(e - 156) is a float (smaller values keep an absolute 2^-148).
-__device__ __forceinline__ int split_exponent(uint32_t max_bits) { return max(int(max_bits >> 23), 8); }
+// that every |x| < 2^(e - 126), from the largest |x|'s bits.  At least 29, so
+// that 2^(156 - e) and 2^(e - 156) are floats (smaller values are multiplied in
+// fp32, see wide_chunks).
+__device__ __forceinline__ int split_exponent(uint32_t max_bits) { return max(int(max_bits >> 23), 29); }
 constexpr uint32_t kNotFinite = 0x7F800000u;   // bits of |x| at or above: infinite or NaN
 
-// Four activations (x[B], B = 0..3) at 2^(156 - e) fixed point, truncated
-// (below 2^-30 of the largest) -> dg[d] = their digits d, byte B from x[B].
+// The factor of the fixed point, a power of two (a product, where ldexp takes
+// 1.7 times its issue time).
+__device__ __forceinline__ float fixed_factor(int e) { return __uint_as_float(uint32_t(283 - e) << 23); }
+
+__device__ __forceinline__ int round_int(float v) {   // floor(v + 0.5) in one operation, exact
+  int r;
+  asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+
+// Four activations (x[B], B = 0..3) at 2^(156 - e) fixed point, rounded ->
+// dg[d] = their digits d, byte B from x[B].
 __device__ __forceinline__ void digits4(const float (&x)[4], int e, uint32_t (&dg)[4]) {
+  const float f = fixed_factor(e);
   uint32_t u[4];   // digits 0..2 each 128 up
 #pragma unroll
-  for (int b = 0; b < 4; ++b) u[b] = uint32_t(int(__builtin_amdgcn_ldexpf(x[b], 156 - e))) + 0x00808080u;
+  for (int b = 0; b < 4; ++b) u[b] = uint32_t(round_int(x[b] * f)) + 0x00808080u;
   const uint32_t a = __builtin_amdgcn_perm(u[1], u[0], 0x05010400u), b = __builtin_amdgcn_perm(u[1], u[0], 0x07030602u);
   const uint32_t c = __builtin_amdgcn_perm(u[3], u[2], 0x05010400u), d = __builtin_amdgcn_perm(u[3], u[2], 0x07030602u);
   dg[0] = __builtin_amdgcn_perm(c, a, 0x05040100u) ^ 0x80808080u;
@@ -248,6 +263,25 @@ __device__ __forceinline__ v4i chunk_product(const uint32_t (&wb)[8], const v4i 
   return __builtin_amdgcn_mfma_i32_16x16x64_i8(f1, b1, acc, 0, 0, 0);
 }
 
+// The products of a chunk that is kept as it is: the sum over the 32 weights of
+// plane word kq in wb against their activations, 16 floats from `lo` (step 0)
+// and 16 from `hi` (step 1): x[B] of the lane whose k is bit t of the bytes is
+// float 4 (t % 4) + B of step t / 4.  Seldom run: it takes as few registers as it
+// can, so that the kernels keep the waves they have without it.
+__device__ __forceinline__ float raw_sum(const uint32_t (&wb)[8], const char *lo, const char *hi) {
+  float s = 0.0f;
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    const float4 x = *reinterpret_cast<const float4 *>((t < 4 ? lo : hi) + (t & 3) * 16);
+    s = fmaf(float(int(wb[t] << 24) >> 24), x.x, s);
+    s = fmaf(float(int(wb[t] << 16) >> 24), x.y, s);
+    s = fmaf(float(int(wb[t] << 8) >> 24), x.z, s);
+    s = fmaf(float(int(wb[t]) >> 24), x.w, s);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  return s;
+}
+
 // Lane roles while digits are made, a 256-chunk per wave: lane = chunk c (1
 // bit), plane word kq (2), k within the byte kl (3); item B is k =
 // 128 c + 32 kq + 8 B + kl, bit t = 7 - kl of byte B.
@@ -265,14 +299,44 @@ __device__ __forceinline__ uint32_t row_max(uint32_t m) {
   return max(m, dpp_u32<0x140>(m));   // lane ^ 15: the other eight of sixteen
 }
 
-// |x| bits of four activations, largest over the 32 lanes of a chunk.
-__device__ __forceinline__ uint32_t chunk_max_bits(const float (&x)[4]) {
+// |x| bits of a lane's four activations, the largest; and over the 32 lanes of a chunk.
+__device__ __forceinline__ uint32_t lane_max_bits(const float (&x)[4]) {
   uint32_t b[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) b[i] = __float_as_uint(x[i]) & 0x7FFFFFFFu;
-  const uint32_t m = row_max(max(max(b[0], b[1]), max(b[2], b[3])));
+  return max(max(b[0], b[1]), max(b[2], b[3]));
+}
+__device__ __forceinline__ uint32_t chunk_max_bits(uint32_t lane_max) {
+  const uint32_t m = row_max(lane_max);
   const auto r = __builtin_amdgcn_permlane16_swap(m, m, false, false);
   return max(uint32_t(r[0]), uint32_t(r[1]));
+}
+
+// Which of a wave's two 128-chunks are wide (bits 0 and 1): more than a quarter
+// of the lanes with a nonzero value have their largest of four below 2^-8 of the
+// power of two that the fixed point is relative to (exponent e).  Rounding leaves
+// each value off by about 2^-32 of that power; up to there (70 % of Gaussian
+// values below it) that is at most 2^-23.7 of a typical value, what fp32 sums of
+// the values round off too (1.0e-7 to 1.3e-7 of an output), even for a row
+// without weight for the largest.  Wave-uniform, as is maybe_wide: whether one may be, `zeros` of
+// the lanes being known to be zero, without a branch.
+__device__ __forceinline__ uint64_t small_lanes(uint32_t lane_max, int e) {
+  return __builtin_amdgcn_ballot_w64(lane_max < uint32_t(e - 7) << 23);
+}
+__device__ __forceinline__ bool maybe_wide(uint32_t lane_max, int e, int zeros) {
+  return __builtin_popcountll(small_lanes(lane_max, e)) - zeros > (zeros ? 0 : 8);
+}
+__device__ __forceinline__ unsigned wide_chunks(uint32_t lane_max, int e) {
+  const uint64_t nonzero = __builtin_amdgcn_ballot_w64(lane_max != 0), small = small_lanes(lane_max, e) & nonzero;
+  const bool lo = 4 * __builtin_popcount(uint32_t(small)) > __builtin_popcount(uint32_t(nonzero));
+  const bool hi = 4 * __builtin_popcount(uint32_t(small >> 32)) > __builtin_popcount(uint32_t(nonzero >> 32));
+  return unsigned(lo) | unsigned(hi) << 1;
+}
+
+// The multiplier of a chunk's digits.
+__device__ __forceinline__ float chunk_mult(uint32_t max_bits, int e, bool wide) {
+  if (max_bits >= kNotFinite) return __builtin_nanf("");
+  return wide ? 0.0f : __builtin_amdgcn_ldexpf(1.0f, e - 156);
 }
 
 }  // namespace lmx

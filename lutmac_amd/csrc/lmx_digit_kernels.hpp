@@ -27,6 +27,14 @@ __device__ __forceinline__ int scale_group(const GemvArgs &a, int ch) {
   return a.gshift >= 0 ? ch >> a.gshift : ch / a.group_chunks;
 }
 
+// The lane once more, for loops that seldom run: what they derive from it then
+// takes no register through the loops before them.
+__device__ __forceinline__ int lane_again() {
+  int lane = int(threadIdx.x) & (kWave - 1);
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
 // ---------------------------------------------------------------------------
 // 1..4 vectors, one launch: RT row tiles per workgroup, the whole K over its
 // waves (wave w takes the 256-chunks w, w + W, ... , PPW of them a round).
@@ -79,6 +87,7 @@ __global__ __launch_bounds__(1024) void digit_gemv_kernel(GemvArgs a, int nv) {
   }
   if (NV == 1 && threadIdx.x < 4) zeros[threadIdx.x] = 0u;
 
+  bool any_wide = false;   // of the wave's chunks, perhaps
   float acc[RT], ss[NV];
 #pragma unroll
   for (int t = 0; t < RT; ++t) acc[t] = 0.0f;
@@ -169,16 +178,16 @@ __global__ __launch_bounds__(1024) void digit_gemv_kernel(GemvArgs a, int nv) {
           }
         }
         if (rot) fwht256_regs_x16(x[0], x[1], x[2], x[3], lane);
-        const uint32_t mb = chunk_max_bits(x);
+        const uint32_t lm = lane_max_bits(x), mb = chunk_max_bits(lm);
         const int e = split_exponent(mb);
+        any_wide |= maybe_wide(lm, e, full || rot ? 0 : ((c2 + 1) * kRotChunk - max(a.cols, c2 * kRotChunk)) / 32 * 8);
         uint32_t dg[4];
         digits4(x, e, dg);
         const int t = 7 - dl.kl;
         char *dst = frags[wave][2 * p + dl.c][t >> 2] + (dl.kq * ROWS + 4 * n) * 16 + (t & 3) * 4;
 #pragma unroll
         for (int q = 0; q < 4; ++q) *reinterpret_cast<uint32_t *>(dst + q * 16) = dg[q];
-        if ((lane & 31) == 0)
-          mults[wave][2 * p + dl.c][n] = mb >= kNotFinite ? __builtin_nanf("") : __builtin_amdgcn_ldexpf(1.0f, e - 156);
+        if ((lane & 31) == 0) mults[wave][2 * p + dl.c][n] = chunk_mult(mb, e, false);
       }
     }
     // a wave reads only the digits it wrote; its LDS operations complete in order
@@ -223,10 +232,80 @@ __global__ __launch_bounds__(1024) void digit_gemv_kernel(GemvArgs a, int nv) {
 #pragma unroll
       for (int t = 0; t < RT; ++t)
 #pragma unroll
-        for (int s = 0; s < S; ++s) acc[t] = fmaf(join_digits(sum[t][s]) * sc[i][t][s], mult, acc[t]);
+        for (int s = 0; s < S; ++s) acc[t] = fmaf(join_digits(sum[t][s]) * mult, sc[i][t][s], acc[t]);
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
+  }
+
+  // ---- wide chunks: the wave goes through its own once more and adds, in fp32,
+  // what the fixed point left of their activations (exact: their low bits) ----
+  if (any_wide) {
+    char *raw = frags[wave][0][0];   // [chunk][vector][step][plane word][64 B]
+#pragma unroll 1
+    for (int c2 = wave; c2 < pairs; c2 += W) {
+      const int lane = lane_again(), li = lane & 15, kq = lane >> 4;
+      const DigitLane dl(lane);
+      unsigned vecs[2] = {0, 0};   // the vectors whose first and second chunk are wide
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        float x[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const int k = c2 * kRotChunk + dl.k(b);
+          const uint32_t kc = uint32_t(min(k, a.cols - 1));
+          const float v = (a.x + size_t(min(n, nv - 1)) * a.cols)[kc];
+          x[b] = k < a.cols ? v : 0.0f;
+          if constexpr (NORM) x[b] *= a.xw[kc];
+        }
+        if (rot) fwht256_regs_x16(x[0], x[1], x[2], x[3], lane);
+        const uint32_t lm = lane_max_bits(x);
+        const int e = split_exponent(chunk_max_bits(lm)), t = 7 - dl.kl;
+        const unsigned wide = wide_chunks(lm, e);
+        if (!wide) continue;
+        vecs[0] |= (wide & 1) << n;
+        vecs[1] |= (wide >> 1) << n;
+        const float f = fixed_factor(e), back = __builtin_amdgcn_ldexpf(1.0f, e - 156);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) x[b] = fmaf(float(round_int(x[b] * f)), -back, x[b]);
+        *reinterpret_cast<float4 *>(raw + (dl.c * NV + n) * 512 + (t >> 2) * 256 + dl.kq * 64 + (t & 3) * 16) =
+            make_float4(x[0], x[1], x[2], x[3]);
+      }
+      if (!(vecs[0] | vecs[1])) continue;
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+      for (int c = 0; c < 2; ++c) {
+        const unsigned mine = c ? vecs[1] : vecs[0];
+        if (!mine) continue;
+        const uint32_t g = uint32_t(scale_group(a, 2 * c2 + c));
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          uint32_t w[CW], wb[8];
+          __builtin_amdgcn_sched_barrier(0);   // registers before latency
+          load_codes<FMT, COPY, false>(a, uint32_t(2 * c2 + c), row0[t], uint32_t(li), uint32_t(kq), w);
+#pragma unroll
+          for (int s = 0; s < S; ++s) {
+            const float scale = (a.scales + row0[t])[uint32_t(s * a.n_groups + g) * uint32_t(a.Npad) + uint32_t(li)];
+            source_bytes<FMT, COPY>(w, s, wb);
+#pragma unroll 1
+            for (int n = 0; n < NV; ++n) {
+              if (!((mine >> n) & 1)) continue;
+              const char *src = raw + (c * NV + n) * 512 + kq * 64;
+              float v = raw_sum(wb, src, src + 256);
+              if constexpr (NV > 1) {   // lane group n holds vector n
+                v += lane_xor<16>(v, lane);
+                v += lane_xor<32>(v, lane);
+                v = kq == n ? v : 0.0f;
+              }
+              acc[t] = fmaf(v, scale, acc[t]);
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
   }
 
   // ---- the lane groups of a wave (NV = 1), then the waves in order ----
@@ -278,6 +357,29 @@ __global__ __launch_bounds__(1024) void digit_gemv_kernel(GemvArgs a, int nv) {
 // SiLU pair's product, of one output.
 __device__ __forceinline__ float vector_scale(float sum, float fac, int ex) {
   return __builtin_amdgcn_ldexpf(sum * fac, ex);
+}
+
+// The vectors of a split quad (index `quad`, its chunk qc) that keep the chunk as
+// it is: bit 16 n for vector n (and 15 more above it).
+__device__ __forceinline__ uint64_t raw_vectors(const DigitVectors &d, int quad, size_t qc, int kq) {
+  return __builtin_amdgcn_ballot_w64(4 * quad + kq < d.count && d.mult[qc * 4 + kq] == 0.0f);
+}
+
+// Their products with the weights wb of a row tile: lane group n that of vector
+// n, 0 for the others.
+__device__ __forceinline__ float raw_quad(const uint32_t (&wb)[8], const char *chunk, uint64_t mask, int lane) {
+  const int kq = lane >> 4;
+  float r = 0.0f;
+#pragma unroll 1
+  for (int n = 0; n < 4; ++n) {
+    if (!((mask >> (16 * n)) & 1)) continue;
+    const char *src = chunk + (kq * 16 + n * 4) * 16;
+    float v = raw_sum(wb, src, src + 1024);
+    v += lane_xor<16>(v, lane);
+    v += lane_xor<32>(v, lane);
+    r = kq == n ? v : r;
+  }
+  return r;
 }
 
 // ---------------------------------------------------------------------------
@@ -341,12 +443,15 @@ __global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVecto
         f[b][q][m] = reinterpret_cast<const v4i *>(d.digits + size_t(qq) * qbytes + size_t(ch) * kQuadChunk + m * 1024)[lane];
     }
   };
+  uint64_t any_wide = 0;   // lanes with a multiplier of 0 among the wave's chunks
   float acc[RT][NQ];
 #pragma unroll
   for (int t = 0; t < RT; ++t)
 #pragma unroll
     for (int q = 0; q < NQ; ++q) acc[t][q] = 0.0f;
   const auto work = [&](int b) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) any_wide |= __builtin_amdgcn_ballot_w64(mu[b][q] == 0.0f);
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
@@ -356,7 +461,7 @@ __global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVecto
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
           const v4i sum = chunk_product(wb, f[b][q][0], f[b][q][1], start);
-          acc[t][q] = fmaf((TIGHT ? join_digits_int(sum) : join_digits(sum)) * sc[b][t][s], mu[b][q], acc[t][q]);
+          acc[t][q] = fmaf((TIGHT ? join_digits_int(sum) : join_digits(sum)) * mu[b][q], sc[b][t][s], acc[t][q]);
         }
       }
   };
@@ -367,6 +472,30 @@ __global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVecto
     if (ch + W >= ch1) break;
     if (ch + 2 * W < ch1) load(0, ch + 2 * W);
     work(1);
+  }
+  if (any_wide) {   // chunks kept as they are: the wave goes through its own once more
+#pragma unroll 1
+    for (int ch = ch0 + wave; ch < ch1; ch += W) {
+      const int lane = lane_again(), li = lane & 15, kq = lane >> 4;
+      const uint32_t g = uint32_t(scale_group(a, ch));
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+        const size_t qc = size_t(min(q0 + q, quads - 1)) * Kc + ch;
+        const uint64_t mask = raw_vectors(d, q0 + q, qc, kq);
+        if (!mask) continue;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+          uint32_t cw[CW], wb[8];
+          load_codes<FMT, COPY, false>(a, uint32_t(ch), row0[t], uint32_t(li), uint32_t(kq), cw);
+#pragma unroll
+          for (int s = 0; s < S; ++s) {
+            const float scale = (a.scales + size_t(s * a.n_groups + g) * Npad + row0[t])[uint32_t(li)];
+            source_bytes<FMT, COPY>(cw, s, wb);
+            acc[t][q] = fmaf(raw_quad(wb, d.digits + qc * kQuadChunk, mask, lane), scale, acc[t][q]);
+          }
+        }
+      }
+    }
   }
 #pragma unroll
   for (int t = 0; t < RT; ++t)
@@ -578,20 +707,42 @@ __global__ __launch_bounds__(256 * KS, (tile_waves<FMT, COPY, NQ>())) void digit
     for (int ch = kg; ch < Kc; ch += KS) {
       load_w(0, ch);
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        if (!((far >> (4 * q)) & 15)) continue;   // wave-uniform
-        const size_t qc = size_t(min(q0 + q, quads - 1)) * Kc + ch;
-        const v4i *src = reinterpret_cast<const v4i *>(d.digits + qc * kQuadChunk) + lane;
-        const v4i f0 = src[0], f1 = src[64];
-        const float mu = (far >> (4 * q + kq)) & 1 ? d.mult[qc * 4 + kq] : 0.0f;
+      for (int s = 0; s < S; ++s) {
+        uint32_t wb[RT][8];
 #pragma unroll
-        for (int t = 0; t < RT; ++t)
+        for (int t = 0; t < RT; ++t) source_bytes<FMT, COPY>(w[0][t], s, wb[t]);
 #pragma unroll
-          for (int s = 0; s < S; ++s) {
-            uint32_t wb[8];
-            source_bytes<FMT, COPY>(w[0][t], s, wb);
-            acc[t][q] = fmaf(join_digits(chunk_product(wb, f0, f1, start)) * mu, sc[0][t][s], acc[t][q]);
+        for (int q1 = 0; q1 < NQ; q1 += 2) {   // two quads' loads at a time
+          if (!((far >> (4 * q1)) & 255)) continue;   // wave-uniform
+          __builtin_amdgcn_sched_barrier(0);
+          const int lane = lane_again(), kq = lane >> 4;
+          v4i f[2][2];
+          float mu[2];
+          const char *chunk[2];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const size_t qc = size_t(min(q0 + q1 + i, quads - 1)) * Kc + ch;
+            chunk[i] = d.digits + qc * kQuadChunk;
+            const v4i *src = reinterpret_cast<const v4i *>(chunk[i]) + lane;
+            f[i][0] = src[0], f[i][1] = src[64];
+            mu[i] = d.mult[qc * 4 + kq];
           }
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int q = q1 + i;
+            const bool mine = (far >> (4 * q + kq)) & 1;
+            const uint64_t raw = __builtin_amdgcn_ballot_w64(mine && mu[i] == 0.0f);
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+              const float j = join_digits(chunk_product(wb[t], f[i][0], f[i][1], start));
+              acc[t][q] = fmaf(mine ? j * mu[i] : 0.0f, sc[0][t][s], acc[t][q]);
+            }
+            if (raw) {
+#pragma unroll
+              for (int t = 0; t < RT; ++t) acc[t][q] = fmaf(raw_quad(wb[t], chunk[i], raw, lane), sc[0][t][s], acc[t][q]);
+            }
+          }
+        }
       }
     }
   }

@@ -174,7 +174,8 @@ struct DigitVectors {
   char *digits;       // [quads of 4 vectors][Kp/128][2 KiB]
   float *fac;         // [count] factor of a vector's sums (norm, rotation, code scale; NaN: not finite)
   int *exp;           // tile form: [count] the power of two of a vector's digits, or kFarVector
-  float *mult;        // rows form and far vectors: [quads][Kp/128][4] that of each vector's chunk
+  float *mult;        // rows form and far vectors: [quads][Kp/128][4] that of each vector's chunk (0: the
+                      // chunk holds the activations themselves)
   float *partials;    // rows form: sums of k-slices (kDigitPartials bytes)
   int count;
   int tile;           // for the tile kernel (many vectors and rows), else the rows kernel

@@ -1,8 +1,8 @@
 """The digit kernels (exact products on the 8-bit matrix cores) at the edges of
 their tiles, slices and groups, against 64-bit sums.
 
-An output sums K products whose activations are fixed point below 2^-30 of
-their chunk's (or vector's) largest magnitude, and ceil(K / 128) chunk sums
+An output sums K products whose activations are fixed point to 2^-30 of their
+chunk's (or vector's) largest magnitude, or as they are, and ceil(K / 128) chunk sums
 rounded to fp32: the bound is that rounding over the sum of the chunks'
 magnitudes, plus the FWHT's 10 roundings where the call rotates."""
 import numpy as np
@@ -239,4 +239,32 @@ def test_digit_far_channel_in_another_chunk(cuda, fmt, spike, rows, cols, batch)
     big = xc.max(axis=2) @ wc.sum(axis=2).T
     bound = (cols // 128 + 18) * EPS * (np.abs(x).astype(np.float64) @ np.abs(W).T) + 2.0 ** -30 * big
     assert (err <= bound).all(), float((err / bound).max())
+    w.close()
+
+
+# The same within the channel's own chunk: the others are either rounded to
+# 2^-31 of a power of two less than 2^8 above most lanes' largest, or kept as
+# they are.  So the bound holds no term of the far channel.
+@pytest.mark.parametrize("fmt", [L.FMT_TERNARY, L.FMT_INT4, L.FMT_INT8])
+@pytest.mark.parametrize("spike", SPIKES)
+@pytest.mark.parametrize("rows,cols,batch", [(2050, 512, 1), (70, 8960, 1), (2050, 512, 3), (10230, 2048, 4),
+                                             (1030, 1024, 11), (130, 8192, 22), (16380, 512, 70), (6100, 1280, 129)])
+def test_digit_far_channel(cuda, fmt, spike, rows, cols, batch):
+    planes, scales, g = synth.make_weights(fmt, rows, cols, seed=rows + fmt, group=128)
+    zero_columns(fmt, planes, [200, 511])
+    w = L.Weight.from_planes(fmt, planes, scales, rows, cols, g)
+    x = np.random.default_rng(batch).standard_normal((batch, cols)).astype(np.float32)
+    rest = np.abs(x).max()
+    x[::2, 200] = spike      # a vector with and one without, in the same quad
+    x[:, 511] = -3.0 * spike
+    y = w.gemv(torch.from_numpy(x).cuda()).cpu().numpy().reshape(batch, rows)
+    W = synth.dequant_f64(fmt, planes, scales, rows, cols, g)
+    err = np.abs(y - x.astype(np.float64) @ W.T)
+    mag = np.abs(x).astype(np.float64) @ np.abs(W).T
+    # a chunk kept as it is adds 32 products a lane and four lanes in fp32
+    bound = (cols // 128 + 18 + 34) * EPS * mag + 2.0 ** -31 * 2.0 ** 8 * rest * np.abs(W).sum(axis=1)
+    assert (err <= bound).all(), float((err / bound).max())
+    # the error of fp32 sums of the same terms, which the far channel is none of
+    fp32 = np.linalg.norm(y - x.astype(np.float64) @ W.T) / np.linalg.norm(x.astype(np.float64) @ W.T)
+    assert fp32 < 3e-7, fp32
     w.close()
