@@ -107,8 +107,11 @@ int lmx_decoder_step(lmx_decoder *d, float *d_logits, void *stream);
 int lmx_decoder_tokens(lmx_decoder *d, int32_t *out, size_t n, void *stream);
 /* Greedy generation with the results of inference.cpp's loop (prompt token by
  * token, then n_new tokens).  All but the last position of a prompt of more
- * than 4 tokens go through the layers in passes of up to 512 rows; for
- * more than 3 new tokens the step is captured in a HIP graph and replayed.
+ * than 4 tokens go through the layers in passes of up to 512 rows, whose
+ * buffers the first such prompt allocates (49 MB at the 1B width) and the
+ * decoder keeps; where the device has no memory for them the prompt goes token
+ * by token.  For more than 3 new tokens the step is captured in a HIP graph and
+ * replayed.
  * out_tokens (host) receives n_prompt + n_new tokens.  The work runs on the
  * decoder's own stream after the work already queued on `stream`; the call
  * returns when it is done.  Timings (ms, HIP events): prefill = the prompt,

@@ -36,6 +36,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <iterator>
 #include <vector>
 
 #include "lmx_device.hpp"
@@ -772,9 +773,12 @@ struct lmx_decoder {
   unsigned *penalty_counts() const { return penalty != 1.0f ? pcount : nullptr; }
   int n_forced = 0;
   size_t host_pos = 0;
-  // Rows of a prompt pass (prefill_rows of them), allocated by the first prompt long enough
+  // Rows of a prompt pass (prefill_rows of them), allocated by the first prompt
+  // long enough: all of them or none
   float *p_hidden = nullptr, *p_qkv = nullptr, *p_attn = nullptr, *p_gate_up = nullptr, *p_act = nullptr;
-  float *p_digits = nullptr;   // digits of a pass; they serve the steps too, all on this stream
+  // Digits of a pass; the steps of a batch use them too, also those that
+  // lmx_decoder_step puts on the caller's stream (a decoder's calls are ordered)
+  float *p_digits = nullptr;
   size_t p_digit_bytes = 0;
   int prompt_pos = 0;        // where the steps start after the prompt passes
   float pos_div = 1.0f;
@@ -786,12 +790,6 @@ struct lmx_decoder {
   std::vector<void *> allocs;
   hipStream_t stream = nullptr;   // capture/replay stream of lmx_decoder_generate
 
-  int alloc_rows(float **p, size_t n) {   // uninitialised
-    const hipError_t e = hipMalloc(reinterpret_cast<void **>(p), n * sizeof(float));
-    if (e != hipSuccess) return hip_err(e, "hipMalloc (decoder)");
-    allocs.push_back(*p);
-    return LMX_OK;
-  }
   int alloc(void **p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) return hip_err(e, "hipMalloc (decoder)");
@@ -1044,31 +1042,59 @@ int prefill_pass(lmx_decoder *d, int p0, int T, hipStream_t st) {
   return LMX_OK;
 }
 
+// The rows of the prompt passes, uninitialised.  False, with nothing allocated,
+// where the device has no memory for them, or where they take more than
+// LMX_PROMPT_BYTES.
+bool prefill_buffers(lmx_decoder *d) {
+  if (d->p_hidden) return true;
+  const lmx_decoder_config &c = d->cfg;
+  const size_t rows = prefill_rows(d);
+  bool pairs = true;
+  size_t Kp = 0;
+  for (const lmx_decoder::Layer &L : d->layers) {
+    pairs = pairs && digit_pairs(L.gate_up);
+    for (const lmx_weight *w : {L.qkv, L.o, L.gate_up, L.down}) Kp = std::max(Kp, w->Kp);
+  }
+  // all of a pass's rows in one launch of every linear (a handle's own
+  // scratch holds 256 vectors of a small matrix: two launches, 25 us
+  // against 19 for the 3072 x 2048 linear of 383 rows)
+  const size_t dig = digit_bytes(Kp, rows) + kDigitPartials;
+  struct { float **p; size_t floats; } want[] = {
+      {&d->p_qkv, rows * (c.n_heads + 2 * c.n_kv_heads) * c.head_dim},
+      {&d->p_attn, rows * c.n_heads * c.head_dim},
+      {&d->p_gate_up, pairs ? 0 : rows * 2 * c.ffn},
+      {&d->p_act, rows * c.ffn},
+      {&d->p_digits, (dig + 3) / 4},
+      {&d->p_hidden, rows * c.hidden}};
+  const char *lim = std::getenv("LMX_PROMPT_BYTES");
+  size_t left = lim ? size_t(std::strtoull(lim, nullptr, 10)) : SIZE_MAX;
+  void *got[std::size(want)] = {};
+  for (size_t i = 0; i < std::size(want); ++i) {
+    const size_t bytes = want[i].floats * sizeof(float);
+    if (!bytes) continue;
+    if (bytes > left || hipMalloc(&got[i], bytes) != hipSuccess) {
+      (void)hipGetLastError();   // the launches after this one look at it
+      for (void *p : got)
+        if (p) (void)hipFree(p);
+      return false;
+    }
+    left -= bytes;
+  }
+  for (size_t i = 0; i < std::size(want); ++i) {
+    if (!got[i]) continue;
+    d->allocs.push_back(got[i]);
+    *want[i].p = static_cast<float *>(got[i]);
+  }
+  d->p_digit_bytes = dig;
+  return true;
+}
+
 // The prompt's first n positions in passes, then the position and (one
 // sequence) its embedding set for the steps from position n on.
 int prefill(lmx_decoder *d, size_t n, hipStream_t st) {
   const lmx_decoder_config &c = d->cfg;
-  const size_t rows = prefill_rows(d), T = rows / d->batch;
+  const size_t T = prefill_rows(d) / d->batch;
   int r;
-  if (!d->p_hidden) {
-    bool pairs = true;
-    size_t Kp = 0;
-    for (const lmx_decoder::Layer &L : d->layers) {
-      pairs = pairs && digit_pairs(L.gate_up);
-      for (const lmx_weight *w : {L.qkv, L.o, L.gate_up, L.down}) Kp = std::max(Kp, w->Kp);
-    }
-    // all of a pass's rows in one launch of every linear (a handle's own
-    // scratch holds 256 vectors of a small matrix: two launches, 25 us
-    // against 19 for the 3072 x 2048 linear of 383 rows)
-    const size_t dig = digit_bytes(Kp, rows) + kDigitPartials;
-    if ((r = d->alloc_rows(&d->p_qkv, rows * (c.n_heads + 2 * c.n_kv_heads) * c.head_dim)) ||
-        (r = d->alloc_rows(&d->p_attn, rows * c.n_heads * c.head_dim)) ||
-        (!pairs && (r = d->alloc_rows(&d->p_gate_up, rows * 2 * c.ffn))) ||
-        (r = d->alloc_rows(&d->p_act, rows * c.ffn)) ||
-        (r = d->alloc_rows(&d->p_digits, (dig + 3) / 4)) || (r = d->alloc_rows(&d->p_hidden, rows * c.hidden)))
-      return r;
-    d->p_digit_bytes = dig;
-  }
   for (size_t p = 0; p < n; p += T)
     if ((r = prefill_pass(d, int(p), int(std::min(T, n - p)), st))) return r;
   d->prompt_pos = int(n);
@@ -1391,9 +1417,10 @@ int lmx_decoder_generate(lmx_decoder *d, const int32_t *prompt, size_t n_prompt,
     if (e == hipSuccess) e = hipEventCreate(&x);
   if (e == hipSuccess) e = hipEventRecord(ev[0], s);
   // All but the prompt's last position in passes of many rows; a pass costs
-  // about as much as three steps, so a shorter prompt takes steps.
+  // about as much as three steps, so a shorter prompt takes steps, and so does
+  // one whose passes the device has no memory for.
   size_t passed = 0;
-  if (e == hipSuccess && n_prompt > 4) {
+  if (e == hipSuccess && n_prompt > 4 && prefill_buffers(d)) {
     passed = n_prompt - 1;
     st = prefill(d, passed, s);
   }

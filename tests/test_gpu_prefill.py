@@ -56,3 +56,33 @@ def quantized(cfg):
                                   "v": (L.FMT_TERNARY, 128, 0), "o": (L.FMT_RRQ2, 128, L.QUANT_RESIDUAL),
                                   "gate": (L.FMT_INT8, 256, 0), "up": (L.FMT_INT8, 256, 0),
                                   "down": (L.FMT_BINARY, 128, 0), "embed": (L.FMT_INT4, 128, 0)}, seed=4)
+
+
+# Passes without the memory for their rows (for none of them, not for all, not for
+# the last) leave the prompt to steps, and nothing behind them: the tokens and the
+# logits after it are those of the passes, once there is memory.
+@pytest.mark.parametrize("batch,limit", [(1, 0), (1, 150000), (1, 900000), (6, 0), (6, 1000000), (6, 2850000)])
+def test_prompt_without_memory_for_passes(cuda, monkeypatch, batch, limit):
+    cfg = D.small_config(max_seq=40, vocab=515)
+    model = D.SyntheticModel(cfg, seed=2, group=128, random_norms=True)
+    prompt = np.random.default_rng(batch).integers(0, cfg.vocab, (batch, 30)).astype(np.int32)
+    p = prompt if batch > 1 else prompt[0]
+    dec = D.Decoder(model, batch=batch)
+    logits = {}
+    for name in ("steps", "steps again", "passes"):
+        if name == "passes":
+            monkeypatch.delenv("LMX_PROMPT_BYTES")
+        else:
+            monkeypatch.setenv("LMX_PROMPT_BYTES", str(limit))
+        out, _, _ = dec.generate(p, 6)
+        lg = torch.empty(batch * cfg.vocab, device="cuda")
+        dec.step(lg)
+        torch.cuda.synchronize()
+        logits[name] = out, lg.cpu().numpy().reshape(batch, cfg.vocab)
+    dec.close()
+    want_out, want = logits["passes"]
+    for name in ("steps", "steps again"):
+        out, got = logits[name]
+        assert np.array_equal(out, want_out)
+        for b in range(batch):
+            assert rel_max_err(got[b], want[b]) < DECODE_TOL, (name, b)
