@@ -309,7 +309,11 @@ static bool one_vector_on_digits(const lmx_weight *w) {
 // vectors of those formats too (a.xmode and a.epi have no other form there).
 int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done,
                  bool all, void *scratch, size_t scratch_bytes) {
-  if (!scratch) scratch = w->d_digits, scratch_bytes = w->digit_cap;
+  unsigned *tickets = static_cast<unsigned *>(scratch);
+  if (scratch)
+    scratch = static_cast<char *>(scratch) + kDigitTicketBytes, scratch_bytes -= kDigitTicketBytes;
+  else
+    scratch = w->d_digits, scratch_bytes = w->digit_cap, tickets = w->d_counters;
   const float *resid = a.resid;
   const size_t out_rows = a.epi == kEpiSiluPair ? w->rows / 2 : w->rows;
   const bool copies = code_copy_bytes(w->format, 1, kRotChunk) != 0;
@@ -329,7 +333,7 @@ int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size
     // ternary 11.4 against 9.4 split, 4-bit 8.0 / 9.1).
     if (cap && (left > 4 || (!copies && w->Kp > 4096 && (left > 1 || all)))) {
       n = std::min(left, cap);
-      const DigitVectors d = digit_vectors(w, scratch, n);
+      const DigitVectors d = digit_vectors(w, scratch, tickets, n);
       if ((st = launch_digit_split(w->format, a, d, stream)) || (st = launch_digit_gemm(w->format, a, d, stream)))
         return st;
     } else {

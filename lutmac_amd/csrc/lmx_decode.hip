@@ -776,8 +776,10 @@ struct lmx_decoder {
   // Rows of a prompt pass (prefill_rows of them), allocated by the first prompt
   // long enough: all of them or none
   float *p_hidden = nullptr, *p_qkv = nullptr, *p_attn = nullptr, *p_gate_up = nullptr, *p_act = nullptr;
-  // Digits of a pass; the steps of a batch use them too, also those that
-  // lmx_decoder_step puts on the caller's stream (a decoder's calls are ordered)
+  // Digits of a pass and their tickets, none of the handles': decoders that share
+  // weights fill their caches side by side.  The steps of a batch use them too,
+  // also those that lmx_decoder_step puts on the caller's stream (a decoder's
+  // calls are ordered)
   float *p_digits = nullptr;
   size_t p_digit_bytes = 0;
   int prompt_pos = 0;        // where the steps start after the prompt passes
@@ -1045,7 +1047,7 @@ int prefill_pass(lmx_decoder *d, int p0, int T, hipStream_t st) {
 // The rows of the prompt passes, uninitialised.  False, with nothing allocated,
 // where the device has no memory for them, or where they take more than
 // LMX_PROMPT_BYTES.
-bool prefill_buffers(lmx_decoder *d) {
+bool prefill_buffers(lmx_decoder *d, hipStream_t st) {
   if (d->p_hidden) return true;
   const lmx_decoder_config &c = d->cfg;
   const size_t rows = prefill_rows(d);
@@ -1058,7 +1060,7 @@ bool prefill_buffers(lmx_decoder *d) {
   // all of a pass's rows in one launch of every linear (a handle's own
   // scratch holds 256 vectors of a small matrix: two launches, 25 us
   // against 19 for the 3072 x 2048 linear of 383 rows)
-  const size_t dig = digit_bytes(Kp, rows) + kDigitPartials;
+  const size_t dig = kDigitTicketBytes + digit_bytes(Kp, rows) + kDigitPartials;
   struct { float **p; size_t floats; } want[] = {
       {&d->p_qkv, rows * (c.n_heads + 2 * c.n_kv_heads) * c.head_dim},
       {&d->p_attn, rows * c.n_heads * c.head_dim},
@@ -1072,7 +1074,9 @@ bool prefill_buffers(lmx_decoder *d) {
   for (size_t i = 0; i < std::size(want); ++i) {
     const size_t bytes = want[i].floats * sizeof(float);
     if (!bytes) continue;
-    if (bytes > left || hipMalloc(&got[i], bytes) != hipSuccess) {
+    // (the digits' tickets start at zero)
+    if (bytes > left || hipMalloc(&got[i], bytes) != hipSuccess ||
+        (want[i].p == &d->p_digits && hipMemsetAsync(got[i], 0, kDigitTicketBytes, st) != hipSuccess)) {
       (void)hipGetLastError();   // the launches after this one look at it
       for (void *p : got)
         if (p) (void)hipFree(p);
@@ -1420,7 +1424,7 @@ int lmx_decoder_generate(lmx_decoder *d, const int32_t *prompt, size_t n_prompt,
   // about as much as three steps, so a shorter prompt takes steps, and so does
   // one whose passes the device has no memory for.
   size_t passed = 0;
-  if (e == hipSuccess && n_prompt > 4 && prefill_buffers(d)) {
+  if (e == hipSuccess && n_prompt > 4 && prefill_buffers(d, s)) {
     passed = n_prompt - 1;
     st = prefill(d, passed, s);
   }

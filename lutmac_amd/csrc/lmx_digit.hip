@@ -238,8 +238,9 @@ size_t digit_capacity(size_t Kp, size_t bytes) {
   return bytes > kDigitPartials ? (bytes - kDigitPartials) / digit_bytes(Kp, 4) * 4 : 0;
 }
 
-DigitVectors digit_vectors(const lmx_weight *w, void *scratch, size_t count) {
+DigitVectors digit_vectors(const lmx_weight *w, void *scratch, unsigned *tickets, size_t count) {
   DigitVectors d{};
+  d.tickets = tickets;
   const size_t quads = (count + 3) / 4, chunks = w->Kp / kChunk;
   d.digits = static_cast<char *>(scratch);
   d.mult = reinterpret_cast<float *>(d.digits + quads * chunks * kQuadChunk);

@@ -515,10 +515,10 @@ __global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVecto
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (threadIdx.x == 0)
-      ticket = __hip_atomic_fetch_add(a.counters + block, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      ticket = __hip_atomic_fetch_add(d.tickets + block, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (ticket != unsigned(slices - 1)) return;   // uniform over the workgroup
-    if (threadIdx.x == 0) __hip_atomic_store(a.counters + block, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) __hip_atomic_store(d.tickets + block, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   const auto total = [&](int o) {
     if (slices == 1) return wg_sum(o);

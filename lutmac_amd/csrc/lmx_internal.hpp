@@ -177,6 +177,7 @@ struct DigitVectors {
   float *mult;        // rows form and far vectors: [quads][Kp/128][4] that of each vector's chunk (0: the
                       // chunk holds the activations themselves)
   float *partials;    // rows form: sums of k-slices (kDigitPartials bytes)
+  unsigned *tickets;  // rows form: [kDigitTickets], zero between launches
   int count;
   int tile;           // for the tile kernel (many vectors and rows), else the rows kernel
 };
@@ -184,9 +185,10 @@ constexpr int kFarVector = 0x7FFFFFFF;    // a vector whose chunks' digits each 
 constexpr unsigned kDigitTickets = 256;   // row blocks of a sliced rows launch, at most
 // Bytes of slice sums: up to 256 workgroups of 2 row tiles x 4 quads x 64 sums.
 constexpr size_t kDigitPartials = 256 * 512 * sizeof(float);
+constexpr size_t kDigitTicketBytes = kDigitTickets * sizeof(unsigned);
 size_t digit_bytes(size_t Kp, size_t vectors);
 size_t digit_capacity(size_t Kp, size_t bytes);   // vectors (a multiple of 4) that fit in bytes
-DigitVectors digit_vectors(const lmx_weight *w, void *scratch, size_t count);
+DigitVectors digit_vectors(const lmx_weight *w, void *scratch, unsigned *tickets, size_t count);
 // a.x [count][cols], transform a.xmode (a.xw, a.eps), a.rotate -> d
 int launch_digit_split(int fmt, const GemvArgs &a, const DigitVectors &d, void *stream);
 // y = W x of the split vectors (+ a.bias per row) (+ a.resid per vector row), or the SiLU pair (a.epi)
@@ -255,7 +257,8 @@ int gemv_impl(const lmx_weight *w, const float *x, float *y, size_t batch, unsig
 GemvArgs weight_args(const lmx_weight *w);
 // y = W x of `batch` vectors on the digit kernels (a.bias, a.resid, a.rotate, a.xmode none or RMSNorm,
 // a.epi store or SiLU pair; x of any alignment); *done = the vectors covered, the rest (one by one on
-// the lookup tables) left to the caller unless `all`; scratch: for the split digits, else the handle's
+// the lookup tables) left to the caller unless `all`; scratch: kDigitTicketBytes of tickets (zero) and
+// room for the split digits, else the handle's
 int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done,
                  bool all, void *scratch = nullptr, size_t scratch_bytes = 0);
 }  // namespace lmx

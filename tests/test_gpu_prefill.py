@@ -1,6 +1,8 @@
 """Prompt passes (many positions at once) against the same prompt taken one
 position a step: the logits of the position after the prompt, from a cache
 that the passes filled and from one that the steps filled."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -86,3 +88,40 @@ def test_prompt_without_memory_for_passes(cuda, monkeypatch, batch, limit):
         assert np.array_equal(out, want_out)
         for b in range(batch):
             assert rel_max_err(got[b], want[b]) < DECODE_TOL, (name, b)
+
+
+# Two decoders that share their weights, each in a thread of its own: the passes
+# share no scratch or ticket (down, K 4096, is summed over k-slices).
+def test_prompt_passes_side_by_side(cuda):
+    cfg = D.small_config(max_seq=72, ffn=4096, vocab=515)
+    model = D.SyntheticModel(cfg, seed=3, group=128, random_norms=True)
+    a, b = D.Decoder(model), D.Decoder(model)
+    for i, layer in enumerate(model.layers):
+        L.check(L.lib().lmx_decoder_set_layer(b._h, i, *[w.handle for w in a.weights[4 * i:4 * i + 4]],
+                                              L._np_ptr(layer["in_norm"]), L._np_ptr(layer["post_norm"]), None))
+    rng = np.random.default_rng(4)
+    prompts = [rng.integers(0, cfg.vocab, 60).astype(np.int32) for _ in range(2)]
+
+    def logits(dec, prompt, out):
+        for _ in range(8):
+            tokens, _, _ = dec.generate(prompt, 2)
+            lg = torch.empty(cfg.vocab, device="cuda")
+            dec.step(lg)
+            torch.cuda.synchronize()
+            out.append((tokens, lg.cpu().numpy()))
+
+    alone = [[], []]
+    for dec, prompt, out in zip((a, b), prompts, alone):
+        logits(dec, prompt, out)
+    together = [[], []]
+    threads = [threading.Thread(target=logits, args=t) for t in zip((a, b), prompts, together)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for want, got in zip(alone, together):
+        assert len(got) == 8
+        for (wt, wl), (gt, gl) in zip(want, got):
+            assert np.array_equal(wt, gt) and np.array_equal(wl.view(np.uint32), gl.view(np.uint32))
+    b.close()
+    a.close()
