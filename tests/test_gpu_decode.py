@@ -66,11 +66,15 @@ def test_decoder_matches_oracle_qwen_style(cuda):
     check_against(D.Decoder(m), oracle.OracleDecoder(m), toks)
 
 
-def test_decoder_long_ffn(cuda, monkeypatch):
-    # FFN 8960 (Qwen-2.5-1.5B's width): the down projection's K = 8960 takes
-    # the layered 8 x 8 x 2 plan (70 chunks on 64 slices), gate|up (17920
-    # rows) the 8 x 32 small-K configuration; with LMX_SILU_PAIR=0 the down
-    # projection forms SiLU*up in its own table build
+@pytest.mark.parametrize("digit", [None, "0"])
+def test_decoder_long_ffn(cuda, monkeypatch, digit):
+    # FFN 8960 (Qwen-2.5-1.5B's width): gate|up and down on the digit kernels, or
+    # (LMX_DIGIT=0) on the lookup tables: down, K = 8960, on the layered 8 x 8 x 2
+    # plan (70 chunks on 64 slices), gate|up (17920 rows) on the 8 x 32 small-K
+    # configuration; with LMX_SILU_PAIR=0 the down projection forms SiLU*up in its
+    # own table build
+    if digit:
+        monkeypatch.setenv("LMX_DIGIT", digit)
     cfg = D.small_config(hidden=256, ffn=8960, vocab=1000, rope_mode=D.ROPE_REFERENCE, rope_factor=1.0,
                          rope_theta=1e6)
     m = D.SyntheticModel(cfg, seed=31, group=128, random_norms=True)
@@ -82,10 +86,14 @@ def test_decoder_long_ffn(cuda, monkeypatch):
     check_against(D.Decoder(m), oracle.OracleDecoder(m), toks)
 
 
-def test_decoder_layered_head_takes_split_k(cuda):
-    # hidden 8960: the tied 1000 x 8960 head gets the layered 8 x 8 x 2 plan,
-    # which has no argmax form, so the head GEMV (RMSNorm in, argmax keys out)
-    # runs the split-K kernel; the down projection (8960 x 256) is full-K
+@pytest.mark.parametrize("digit", [None, "0"])
+def test_decoder_layered_head_takes_split_k(cuda, monkeypatch, digit):
+    # hidden 8960: the tied 1000 x 8960 head on the digit kernels, three
+    # 256-chunks a wave, or (LMX_DIGIT=0) on the layered 8 x 8 x 2 plan, which has
+    # no argmax form, so that the head GEMV (RMSNorm in, argmax keys out) runs the
+    # split-K kernel; the down projection (8960 x 256) is full-K
+    if digit:
+        monkeypatch.setenv("LMX_DIGIT", digit)
     cfg = D.small_config(hidden=8960, n_layers=1, n_heads=2, n_kv_heads=1, head_dim=64, ffn=256, vocab=1000,
                          max_seq=32, rope_mode=D.ROPE_REFERENCE, rope_factor=1.0, rope_theta=1e6)
     m = D.SyntheticModel(cfg, seed=45, group=128, random_norms=True)
@@ -288,8 +296,8 @@ def batched_check(dec, m, toks, tol=DECODE_TOL):
             assert err < tol, f"sequence {b} step {pos}: rel err {err:.3e}"
 
 
-# B = 4: one group of the batched GEMV; B = 6: a group of 4 and two rows by the
-# single-vector GEMV; 70 positions cross a 64-position attention chunk.
+# B = 4: the linears in one launch each; B = 6: on split vectors, the second quad
+# half filled; 70 positions cross a 64-position attention chunk.
 @pytest.mark.parametrize("batch", [4, 6])
 def test_batched_decoder_matches_oracle(cuda, batch):
     cfg = D.small_config(max_seq=128, rope_mode=D.ROPE_LLAMA3, rope_factor=32.0, rope_orig_max_pos=64,
@@ -300,70 +308,25 @@ def test_batched_decoder_matches_oracle(cuda, batch):
 
 
 @pytest.mark.parametrize("batch", [8, 16])
-def test_batched_decoder_fused_epilogues(cuda, monkeypatch, batch):
-    # o/down reductions writing the normed rows and the gate|up reduction
-    # writing SiLU(gate)*up (every row in a batched group) against the row
-    # kernels (LMX_FUSED_ROWS=0): the same bits, and the oracle's logits.
-    # The qkv split partials summed inside attention (the default for one
-    # group) against the batched reduction writing the rows first
-    # (LMX_QKV_PARTS=0): the same bits as well.
+def test_batched_decoder_fused_epilogues(cuda, batch):
+    # Split vectors with the norms in the split, the bias and the residual in the
+    # products' epilogues and SiLU(gate)*up in gate|up's: the oracle's logits
     cfg = D.small_config(hidden=512, n_heads=8, n_kv_heads=2, head_dim=64, ffn=1024, vocab=700, max_seq=64,
                          rope_mode=D.ROPE_REFERENCE, rope_factor=1.0, rope_theta=1e6, qkv_bias=True)
     m = D.SyntheticModel(cfg, seed=35 + batch, group=128, random_norms=True)
     toks = np.random.default_rng(36).integers(0, cfg.vocab, (batch, 12))
-
-    def logits(dec):
-        dec.reset(toks)
-        lg = torch.empty(batch * cfg.vocab, dtype=torch.float32, device="cuda")
-        out = []
-        for _ in range(toks.shape[1]):
-            dec.step(lg)
-            out.append(lg.cpu().numpy().reshape(batch, cfg.vocab).copy())
-        return out
-
-    fused = logits(D.Decoder(m, batch=batch))
-    monkeypatch.setenv("LMX_QKV_PARTS", "0")
-    reduced = logits(D.Decoder(m, batch=batch))
-    monkeypatch.setenv("LMX_FUSED_ROWS", "0")
-    rows = logits(D.Decoder(m, batch=batch))
-    refs = [oracle.OracleDecoder(m) for _ in range(batch)]
-    for pos in range(toks.shape[1]):
-        assert np.array_equal(fused[pos].view(np.uint32), reduced[pos].view(np.uint32)), pos
-        assert np.array_equal(fused[pos].view(np.uint32), rows[pos].view(np.uint32)), pos
-        for b in range(batch):
-            assert rel_max_err(fused[pos][b], refs[b].step(toks[b, pos], pos)) < DECODE_TOL, (b, pos)
+    batched_check(D.Decoder(m, batch=batch), m, toks)
 
 
-@pytest.mark.parametrize("plan", [3, 6])
-def test_batched_decoder_four_vector_kernel(cuda, monkeypatch, plan):
-    # batch 4 on K <= 2048 plans: qkv and gate|up (SiLU(gate)*up written by
-    # the workgroup) take the four-vector full-K kernel; against the batched
-    # kernel with its reductions (LMX_NO_QUAD=1) and the oracle's logits
-    monkeypatch.setenv("LMX_FULLK", str(plan))
+@pytest.mark.parametrize("batch", [2, 3, 4])
+def test_batched_decoder_four_vector_kernel(cuda, batch):
+    # up to 4 sequences: every linear in one launch, norms, bias, residual and
+    # SiLU(gate)*up in it; the oracle's logits
     cfg = D.small_config(hidden=512, n_heads=8, n_kv_heads=2, head_dim=64, ffn=1024, vocab=700, max_seq=64,
                          rope_mode=D.ROPE_REFERENCE, rope_factor=1.0, rope_theta=1e6, qkv_bias=True)
-    m = D.SyntheticModel(cfg, seed=51 + plan, group=128, random_norms=True)
-    toks = np.random.default_rng(52).integers(0, cfg.vocab, (4, 12))
-    dec = D.Decoder(m, batch=4)
-    assert all(w.kernel_config()[0] == plan for w in dec.weights[:4])
-
-    def logits(dec):
-        dec.reset(toks)
-        lg = torch.empty(4 * cfg.vocab, dtype=torch.float32, device="cuda")
-        out = []
-        for _ in range(toks.shape[1]):
-            dec.step(lg)
-            out.append(lg.cpu().numpy().reshape(4, cfg.vocab).copy())
-        return out
-
-    quad = logits(dec)
-    monkeypatch.setenv("LMX_NO_QUAD", "1")
-    batched = logits(dec)
-    refs = [oracle.OracleDecoder(m) for _ in range(4)]
-    for pos in range(toks.shape[1]):
-        for b in range(4):
-            assert rel_max_err(quad[pos][b], batched[pos][b]) < 1e-5, (b, pos)
-            assert rel_max_err(quad[pos][b], refs[b].step(toks[b, pos], pos)) < DECODE_TOL, (b, pos)
+    m = D.SyntheticModel(cfg, seed=51 + batch, group=128, random_norms=True)
+    toks = np.random.default_rng(52).integers(0, cfg.vocab, (batch, 12))
+    batched_check(D.Decoder(m, batch=batch), m, toks)
 
 
 def test_batched_decoder_qwen_style(cuda):
@@ -375,8 +338,7 @@ def test_batched_decoder_qwen_style(cuda):
     batched_check(D.Decoder(m, batch=4), m, toks)
 
 
-# B = 4: the four-vector step; B = 16: one group of the batched kernel with
-# the qkv partials summed inside attention, captured and replayed
+# B = 4: linears of one launch each; B = 16: split vectors; captured and replayed
 @pytest.mark.parametrize("B", [4, 16])
 def test_batched_generate_graph_equals_eager_and_oracle(cuda, B):
     cfg = D.small_config(max_seq=96)
@@ -485,45 +447,22 @@ def test_decoder_past_4096_positions(cuda):
 
 
 @pytest.mark.parametrize("batch,hs", [(8, None), (8, "3"), (4, None)])
-def test_batched_qkv_partials_head_dim_128(cuda, monkeypatch, batch, hs):
+def test_batched_attention_head_dim_128(cuda, monkeypatch, batch, hs):
     # Qwen attention geometry (head_dim 128, 6 query heads per KV head, QKV
-    # bias) with the qkv split partials summed inside attention: the KV
-    # head's query heads over 2 workgroups (the default for this small
-    # grid) or 3 (LMX_ATTN_HS), batch 8 and 4 (the fused-reduction step,
-    # LMX_QUAD_STEP=0); the same bits as the reduced rows (LMX_QKV_PARTS=0)
-    # and the oracle's logits, across two attention chunks.  At batch 4 the
-    # reduced path's qkv takes the four-vector kernel, unsplit here
-    # (LMX_QPS=0): its chunk sums are then the batched reduction's bits.
-    monkeypatch.setenv("LMX_QUAD_STEP", "0")
-    monkeypatch.setenv("LMX_QPS", "0")
+    # bias): the KV head's query heads over 2 workgroups (the default for this
+    # small grid) or 3 (LMX_ATTN_HS), batch 8 and 4; the oracle's logits, across
+    # two attention chunks
     if hs:
         monkeypatch.setenv("LMX_ATTN_HS", hs)
     cfg = qwen_small(max_seq=128)
     m = D.SyntheticModel(cfg, seed=57 + batch, group=128, random_norms=True)
     toks = np.random.default_rng(58).integers(0, cfg.vocab, (batch, 70))
-
-    def logits(dec):
-        dec.reset(toks)
-        lg = torch.empty(batch * cfg.vocab, dtype=torch.float32, device="cuda")
-        out = []
-        for _ in range(toks.shape[1]):
-            dec.step(lg)
-            out.append(lg.cpu().numpy().reshape(batch, cfg.vocab).copy())
-        return out
-
-    parts = logits(D.Decoder(m, batch=batch))
-    monkeypatch.setenv("LMX_QKV_PARTS", "0")
-    reduced = logits(D.Decoder(m, batch=batch))
-    refs = [oracle.OracleDecoder(m) for _ in range(batch)]
-    for pos in range(toks.shape[1]):
-        assert np.array_equal(parts[pos].view(np.uint32), reduced[pos].view(np.uint32)), pos
-        for b in range(batch):
-            assert rel_max_err(parts[pos][b], refs[b].step(toks[b, pos], pos)) < DECODE_TOL, (b, pos)
+    batched_check(D.Decoder(m, batch=batch), m, toks)
 
 
 @pytest.mark.parametrize("cpw", [None, "2"])
 def test_batched_decoder_batch16_past_512(cuda, monkeypatch, cpw):
-    # batch 16 = one full group of the batched GEMV, with the attention of every
+    # batch 16 = four whole quads of split vectors, with the attention of every
     # sequence past 512 positions (32-chunk merge); one chunk per workgroup
     # (the automatic choice at this cache size) or two (5 units over 9 chunks)
     if cpw is not None:
@@ -571,18 +510,29 @@ UNIFORM = {"q": (L.FMT_INT8, 128, 0), "k": (L.FMT_INT8, 128, 0), "v": (L.FMT_INT
            "down": (L.FMT_INT8, 256, 0), "embed": (L.FMT_INT8, 128, 0)}
 
 
+@pytest.mark.parametrize("digit", [None, "0"])
 @pytest.mark.parametrize("formats", [MIXED, UNIFORM], ids=["mixed", "uniform"])
-def test_mixed_format_model_and_lutmac_v2_round_trip(cuda, tmp_path, formats):
+def test_mixed_format_model_and_lutmac_v2_round_trip(cuda, tmp_path, monkeypatch, formats, digit):
     # linears quantized by lmx_quantize (mixed: ternary / binary / RRQ-3 /
     # residual RRQ-2 at group 128, weights FWHT-rotated as the quantize tool
     # does; uniform: 8- and 3-bit at groups 128 and 256), decoded on the
     # device from memory and from a version-2 file, against the oracle's
     # decode step (which rotates the 1-2 bit formats' activations as
-    # lut_linear does)
+    # lut_linear does); the 4- and 8-bit linears and heads on the digit kernels or
+    # (LMX_DIGIT=0) on the lookup tables, greedy picks included
+    if digit:
+        monkeypatch.setenv("LMX_DIGIT", digit)
     cfg = D.small_config(rope_mode=D.ROPE_REFERENCE, rope_factor=1.0, rope_theta=10000.0, max_seq=64)
     m = D.QuantizedModel(cfg, formats, seed=61)
     toks = np.random.default_rng(62).integers(0, cfg.vocab, 16)
-    check_against(D.Decoder(m), oracle.OracleDecoder(m), toks)
+    dec = D.Decoder(m)
+    check_against(dec, oracle.OracleDecoder(m), toks)
+    out, _, _ = dec.generate(toks[:3], 6)
+    o = oracle.OracleDecoder(m)
+    for pos in range(len(out) - 1):
+        lg = o.step(out[pos], pos)
+        if pos + 1 >= 3:
+            assert lg[out[pos + 1]] >= lg.max() - DECODE_TOL * np.linalg.norm(lg)
     path = tmp_path / "mixed.lutmac"
     m.save_v2(path)
     ours = D.LutmacModel(path, max_seq=64)
@@ -592,53 +542,21 @@ def test_mixed_format_model_and_lutmac_v2_round_trip(cuda, tmp_path, formats):
     check_against(ours, oracle.OracleDecoder(m), toks)
 
 
-@pytest.mark.parametrize("batch,max_blocks", [(4, None), (4, "50"), (8, None)])
-def test_batched_mixed_format_decoder(cuda, monkeypatch, batch, max_blocks):
+@pytest.mark.parametrize("batch", [4, 8])
+def test_batched_mixed_format_decoder(cuda, batch):
     # the batched decoder on ternary / binary / RRQ-3 / RRQ-2 linears, whose
     # activations the kernels rotate, against one oracle decoder per
-    # sequence: batch 8 with the fused norm / SiLU epilogues, batch 4 with
-    # the four-vector kernels (LMX_QUAD_MAX_BLOCKS = 50: gate|up (64
-    # workgroups) and the head (63) on the batched kernel with its RMSNorm
-    # prologue and the rotation after it)
-    if max_blocks:
-        monkeypatch.setenv("LMX_QUAD_MAX_BLOCKS", max_blocks)
+    # sequence: batch 8 on split vectors, batch 4 in one launch each
     cfg = D.small_config(rope_mode=D.ROPE_REFERENCE, rope_factor=1.0, rope_theta=10000.0, max_seq=64)
     m = D.QuantizedModel(cfg, MIXED, seed=63)
     toks = np.random.default_rng(64).integers(0, cfg.vocab, (batch, 12))
     batched_check(D.Decoder(m, batch=batch), m, toks)
 
 
-@pytest.mark.parametrize("max_blocks", [None, "100"])
-def test_batched_decoder_quad_step(cuda, monkeypatch, max_blocks):
-    # Batch 4 with qkv and o on the four-vector kernel (RMSNorm in its table
-    # build, the residual in its epilogue, no reduction).  LMX_QUAD_MAX_BLOCKS
-    # = 100 keeps gate|up and the head (256 workgroups each) on the batched
-    # kernel with the RMSNorm in its own prologue.  Against the step with
-    # the fused reductions (LMX_QUAD_STEP=0) and the oracle's logits.
-    if max_blocks:
-        monkeypatch.setenv("LMX_QUAD_MAX_BLOCKS", max_blocks)
+def test_batched_decoder_quad_step(cuda):
+    # Batch 4, 256 workgroups of gate|up and of the head: the oracle's logits
     cfg = D.small_config(hidden=256, n_heads=8, n_kv_heads=2, head_dim=64, ffn=2048, vocab=4096, max_seq=64,
                          rope_mode=D.ROPE_REFERENCE, rope_factor=1.0, rope_theta=1e6, qkv_bias=True)
     m = D.SyntheticModel(cfg, seed=71, group=128, random_norms=True)
     toks = np.random.default_rng(72).integers(0, cfg.vocab, (4, 10))
-
-    def logits(dec):
-        dec.reset(toks)
-        lg = torch.empty(4 * cfg.vocab, dtype=torch.float32, device="cuda")
-        out = []
-        for _ in range(toks.shape[1]):
-            dec.step(lg)
-            out.append(lg.cpu().numpy().reshape(4, cfg.vocab).copy())
-        return out
-
-    dec = D.Decoder(m, batch=4)
-    assert [w.kernel_config()[0] for w in dec.weights[:3]] == [6, 6, 6]   # qkv, o, gate|up: 4 x 4 x 1
-    quad = logits(dec)
-    monkeypatch.setenv("LMX_QUAD_STEP", "0")
-    fused = logits(dec)
-    refs = [oracle.OracleDecoder(m) for _ in range(4)]
-    for pos in range(toks.shape[1]):
-        for b in range(4):
-            want = refs[b].step(toks[b, pos], pos)
-            assert rel_max_err(quad[pos][b], fused[pos][b]) < 1e-5, (b, pos)
-            assert rel_max_err(quad[pos][b], want) < DECODE_TOL, (b, pos)
+    batched_check(D.Decoder(m, batch=4), m, toks)

@@ -319,7 +319,8 @@ def test_splitk_reductions(cuda, monkeypatch, reduce, kslice, fmt):
     assert rel_max_err(yb, refb) < TOL
 
 
-# ---- batched GEMV (weights read once per group of 2/4/8/16 vectors) ----------
+# ---- batched GEMV (the digit kernels: one launch up to 4 vectors, split ones
+# beyond; tests/test_gpu_digit.py has their edges) ------------------------------
 @pytest.mark.parametrize("fmt", [1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("batch", [4, 7, 8, 16, 21])
 @pytest.mark.parametrize("rows,cols", [(300, 640), (513, 1536)])
@@ -333,20 +334,13 @@ def test_batched_gemv(cuda, fmt, batch, rows, cols):
         assert rel_max_err(y[b], ref) < TOL, f"vector {b}"
 
 
-# Unrotated 4-bit groups of 8 and 16 vectors, and groups of 4 the
-# four-vector kernel does not take (K past 2048 here), run on the matrix
-# cores (LMX_MFMA=1, the default: 8 waves per workgroup, the codes from the
-# handle's nibble copy; 2: two row tiles per wave; 3: the codes from the
-# planes; 4: four waves; 0 the
-# lookup-table kernel): 128- and 256-wide
-# k-slices, K past the last whole 256 (640), group scales of 128 and 256
-# and one per row, a last group of fewer vectors (9, 21), against the oracle.
-@pytest.mark.parametrize("mfma", ["1", "2", "3", "4", "0"])
+# Unrotated 4-bit batches on the 8-bit matrix cores: one and two row tiles, whole
+# and partly filled quads of vectors (9, 21), K past the last whole 256 (640),
+# group scales of 128 and 256 and one per row, against the oracle.
 @pytest.mark.parametrize("group", [128, 256, 0])
 @pytest.mark.parametrize("batch", [8, 16, 9, 21, 4, 12])
 @pytest.mark.parametrize("rows,cols", [(300, 640), (513, 1536), (2048, 2048), (4160, 4096)])
-def test_batched_int4_matrix_cores(cuda, monkeypatch, mfma, group, batch, rows, cols):
-    monkeypatch.setenv("LMX_MFMA", mfma)
+def test_batched_int4_matrix_cores(cuda, group, batch, rows, cols):
     planes, scales, g = synth.make_weights(L.FMT_INT4, rows, cols, seed=batch * 31 + rows, group=group or 128)
     if group == 0:
         scales = np.ascontiguousarray(scales[:, :, :1])
@@ -363,8 +357,8 @@ def test_batched_int4_matrix_cores(cuda, monkeypatch, mfma, group, batch, rows, 
 @pytest.mark.parametrize("batch", [7, 8, 16])
 @pytest.mark.parametrize("rows,cols", [(4160, 4096), (2112, 4096)])
 def test_batched_gemv_row_groups(cuda, fmt, batch, rows, cols):
-    # 256 rows per workgroup (4160 x 4096) and 128 (2112 x 4096), each with a
-    # last workgroup whose upper row groups lie past the matrix
+    # as many row tiles as fill the chip, and half as many, the rows no multiple
+    # of a workgroup's
     planes, scales, g = synth.make_weights(fmt, rows, cols, seed=fmt * 7 + batch, group=128)
     xs = np.stack([synth.make_activations(cols, seed=2000 + s, outliers=True) for s in range(batch)])
     w = L.Weight.from_planes(fmt, planes, scales, rows, cols, g)
@@ -375,40 +369,30 @@ def test_batched_gemv_row_groups(cuda, fmt, batch, rows, cols):
 
 
 @pytest.mark.parametrize("fmt", [1, 2, 3, 4, 5, 6, 7])
-@pytest.mark.parametrize("cfg", [3, 6])
 @pytest.mark.parametrize("rows,cols", [(70, 2048), (33, 640)])
 @pytest.mark.parametrize("flags", [0, 1])
-def test_four_vector_full_k(cuda, monkeypatch, fmt, cfg, rows, cols, flags):
-    # 4 vectors on a full-K plan of K <= 2048 (8x2x1, 4x4x1) take the kernel
-    # that holds the 4 vectors' tables side by side and sums in the
-    # workgroup: the oracle for each vector, and the batched kernel's values
-    # (LMX_NO_QUAD=1) to the same bar; 640 leaves the upper slices idle
-    monkeypatch.setenv("LMX_FULLK", str(cfg))
-    planes, scales, g = synth.make_weights(fmt, rows, cols, seed=cfg * 31 + fmt, group=128)
+def test_four_vector_full_k(cuda, fmt, rows, cols, flags):
+    # 4 vectors in one launch that sums the whole K in the workgroup: the oracle
+    # for each vector, and the split form (the same vectors in a batch of 8) to
+    # the same bar
+    planes, scales, g = synth.make_weights(fmt, rows, cols, seed=31 + fmt, group=128)
     xs = np.stack([synth.make_activations(cols, seed=3000 + s, outliers=True) for s in range(4)])
     w = L.Weight.from_planes(fmt, planes, scales, rows, cols, g)
-    assert w.kernel_config()[0] == cfg
     y = w.gemv(dev(xs.ravel()), flags=flags).cpu().numpy().reshape(4, rows)
-    monkeypatch.setenv("LMX_NO_QUAD", "1")
-    yb = w.gemv(dev(xs.ravel()), flags=flags).cpu().numpy().reshape(4, rows)
+    yb = w.gemv(dev(np.concatenate([xs, xs]).ravel()), flags=flags).cpu().numpy().reshape(8, rows)
     for b in range(4):
         ref = oracle_planes_gemv(fmt, planes, scales, rows, cols, g, xs[b], flags)
         assert rel_max_err(y[b], ref) < TOL, f"vector {b}"
-        assert rel_max_err(y[b], yb[b]) < TOL, f"vector {b}"
+        assert rel_max_err(y[b], yb[b]) < TOL and np.array_equal(yb[b], yb[b + 4]), f"vector {b}"
 
 
-@pytest.mark.parametrize("qps", ["0", "1"])
 @pytest.mark.parametrize("rows,cols", [(70, 2048), (2048, 1536), (1536, 1536), (33, 640)])
-def test_four_vector_plane_split(cuda, monkeypatch, qps, rows, cols):
-    # 4 unrotated 4-bit vectors on the 4x4x1 plan: the four-vector kernel
-    # with a chunk's planes split over two lanes (where twice its workgroups
-    # still make one round; LMX_QPS=0 keeps one lane per row and chunk),
-    # against the oracle for each vector
-    monkeypatch.setenv("LMX_QPS", qps)
+def test_four_vector_int4(cuda, rows, cols):
+    # 4 unrotated 4-bit vectors of a decoder's small linears, against the oracle
+    # for each vector
     planes, scales, g = synth.make_weights(L.FMT_INT4, rows, cols, seed=rows + 5 * cols, group=128)
     xs = np.stack([synth.make_activations(cols, seed=4000 + s, outliers=True) for s in range(4)])
     w = L.Weight.from_planes(L.FMT_INT4, planes, scales, rows, cols, g)
-    assert w.kernel_config()[0] == 6
     y = w.gemv(dev(xs.ravel()), flags=L.ROTATE_NONE).cpu().numpy().reshape(4, rows)
     for b in range(4):
         ref = oracle_planes_gemv(L.FMT_INT4, planes, scales, rows, cols, g, xs[b], L.ROTATE_NONE)
@@ -418,14 +402,13 @@ def test_four_vector_plane_split(cuda, monkeypatch, qps, rows, cols):
 
 @pytest.mark.parametrize("fmt", [L.FMT_INT4, L.FMT_TERNARY])
 def test_four_vector_linear_bias(cuda, fmt):
-    # lmx_linear on exactly 4 vectors of a 4 x 4 x 1 plan: the four-vector
-    # kernel's bias epilogue (ternary: the FWHT-256 lut_linear applies)
+    # lmx_linear on exactly 4 vectors: the one-launch kernel's bias epilogue
+    # (ternary: the FWHT-256 lut_linear applies)
     rows, cols = 2048, 1536
     planes, scales, g = synth.make_weights(fmt, rows, cols, seed=90 + fmt, group=128)
     xs = np.stack([synth.make_activations(cols, seed=900 + s, outliers=True) for s in range(4)])
     bias = np.random.default_rng(91).standard_normal(rows).astype(np.float32)
     w = L.Weight.from_planes(fmt, planes, scales, rows, cols, g)
-    assert w.kernel_config()[0] == 6
     y = w.linear(dev(xs.ravel()), bias=dev(bias)).cpu().numpy().reshape(4, rows)
     rot = L.ROTATE_FWHT256 if fmt == L.FMT_TERNARY else L.ROTATE_NONE
     for b in range(4):

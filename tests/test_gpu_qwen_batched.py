@@ -6,16 +6,12 @@ Qwen-2.5-1.5B-width decoder of 2 layers (hidden 1536, GQA 12/2 at head_dim
 4 and 16 against one oracle decode step per sequence (Model::forward,
 src/model.cpp:47-453) and the oracle's greedy pick.
 
-The kernel plans are those of the bench's config-5 rows (same matrices, same
-batch, same cache capacity; only the layer count differs):
-  * down 1536 x 8960: 35 k-slices of 256, so the batched reduction keeps 48
-    split loads in flight (batched_reduce_kernel<48>, batch 4 in the
-    four-vector step) or the fused norm reduction sums 35 splits
-    (batched_reduce_norm_kernel, batch 16);
-  * gate|up 17920 x 1536 with SiLU(gate)*up written by its reduction
-    (batched_reduce_pair_kernel, batch 16) or by the four-vector plan;
-  * the 151936 x 1536 head on the batched kernel (3564 workgroups at batch 16)
-    with the batched greedy pick over 151936 columns (argmax_rows_kernel).
+The kernels are those of the benchmark's Qwen rows (same matrices, same batch,
+same cache capacity; only the layer count differs): batch 4 in one launch a
+linear (digit_gemv_kernel, several rounds of 256-chunks per wave at K 8960),
+batch 16 on split vectors (digit_rows_kernel for qkv, o and down,
+digit_tile_kernel for gate|up and the head), SiLU(gate)*up written by gate|up's launch, the
+greedy pick over 151936 columns by argmax_rows_kernel.
 """
 from dataclasses import replace
 

@@ -2,9 +2,9 @@
 caller-held device tiles and scales, with its scratch (split-K partials,
 ticket counters, x staging) in the library's static per-GPU array.  Its
 output must equal lmx_gemv's on a handle built from the same planes (same
-kernels and plan; bit-identical below batch 4, where lmx_gemv runs one
-vector at a time too; within TOL at batch 5, where lmx_gemv batches), call
-after call, the second call smaller than the first.
+kernels and plan; bit-identical up to batch 4, which both take in one launch;
+within TOL at batch 5, where lmx_gemv splits the vectors), call after call, the
+second call smaller than the first.
 
 The first test of this file makes the process's first call (the one that
 zeroes the array) on one stream and the next call on another stream."""
