@@ -179,7 +179,11 @@ __global__ __launch_bounds__(256) void digit_split_chunks_kernel(const float *__
   const bool wide = (wide_chunks(lm, e) >> dl.c) & 1;
   const size_t qc = size_t(v >> 2) * size_t(Kp / kChunk) + size_t(2 * c2 + dl.c);
   store_digits(d, qc, v & 3, dl, o, e, wide);
-  if ((lane & 31) == 0) d.mult[qc * 4 + (v & 3)] = chunk_mult(mb, e, wide);
+  if ((lane & 31) == 0) {
+    d.mult[qc * 4 + (v & 3)] = chunk_mult(mb, e, wide);
+    if (v == d.count - 1)   // the last quad's other vectors, so that theirs are no 0
+      for (int n = (v & 3) + 1; n < 4; ++n) d.mult[qc * 4 + n] = 1.0f;
+  }
 }
 
 }  // namespace

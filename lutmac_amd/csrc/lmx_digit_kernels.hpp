@@ -443,7 +443,7 @@ __global__ __launch_bounds__(1024) void digit_rows_kernel(GemvArgs a, DigitVecto
         f[b][q][m] = reinterpret_cast<const v4i *>(d.digits + size_t(qq) * qbytes + size_t(ch) * kQuadChunk + m * 1024)[lane];
     }
   };
-  uint64_t any_wide = 0;   // lanes with a multiplier of 0 among the wave's chunks
+  uint64_t any_wide = 0;   // lanes with a multiplier of 0 among the wave's chunks (in scalar registers)
   float acc[RT][NQ];
 #pragma unroll
   for (int t = 0; t < RT; ++t)
