@@ -132,7 +132,8 @@ def gemv_bench(L, synth, torch, fmt, n, steps, warmup, graph=True, rotate_in_ker
     gbps = B / (ms * 1e-3) / 1e9
     out = {"format": L.FORMAT_NAMES[fmt], "rows": n, "cols": cols, "group": g,
            "rotation": "FWHT-256 in the kernel" if rotate_in_kernel else "input pre-rotated (FWHT-256), kernel unrotated",
-           "kernel_plan": dict(zip(("fullk", "kslice", "staged"), ws[0].kernel_config())),
+           # the plan of the lookup-table kernels, which most 4- and 8-bit calls do not run
+           "lookup_plan": dict(zip(("fullk", "kslice", "staged"), ws[0].kernel_config())),
            "algorithmic_bytes": B, "us_per_gemv": round(ms * 1e3, 3), "GB_per_s": round(gbps, 1),
            "launch": "hip_graph" if ms_graph is not None else "stream",
            "replays_us_per_gemv": [round(r * 1e3, 3) for r in reps],

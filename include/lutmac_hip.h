@@ -132,7 +132,9 @@ int lmx_weight_create(const lmx_planes_desc *desc, lmx_weight **out);
 int lmx_weight_from_blocks(int format, const void *blocks, size_t num_blocks,
                            size_t rows, size_t cols, lmx_weight **out);
 int lmx_weight_destroy(lmx_weight *w);
-/* Format, shape and device bytes (planes + scales) of a handle. */
+/* Format, shape and device bytes (planes + scales) of a handle.  A 4- or 8-bit
+ * handle holds its codes a second time, laid out for the matrix cores, which
+ * the count leaves out as it does the scratch. */
 int lmx_weight_info(const lmx_weight *w, int *format, size_t *rows,
                     size_t *cols, size_t *device_bytes);
 /* Lookup-table plan chosen for a handle at creation (calls on the digit
@@ -140,8 +142,8 @@ int lmx_weight_info(const lmx_weight *w, int *format, size_t *rows,
  * (0 = split-K kernel, 1..6 = LMX_FULLK values), split-K k-slice, and
  * whether the full-K kernel stages its weight loads.  Diagnostic only; the
  * environment variables LMX_FULLK, LMX_KSLICE, LMX_WAVES, LMX_STAGED and
- * LMX_REDUCE, read when a handle is created, override the plan.  No
- * reference counterpart (the reference has one CPU kernel per format). */
+ * LMX_REDUCE, read when a handle is created, override the plan, and any of them
+ * sends 4- and 8-bit vectors to it.  No reference counterpart (the reference has one CPU kernel per format). */
 int lmx_weight_kernel_config(const lmx_weight *w, int *fullk, int *kslice,
                              int *staged);
 /* Copy the device tile layout back to the host (bit-exact repack check). */
@@ -153,9 +155,20 @@ int lmx_weight_read_tiles(const lmx_weight *w, uint8_t *tiles, size_t bytes);
  * kernel zero-extends to the padded width).  The rows of a batch share
  * one pass over the weights, up to 4 in one launch, more through scratch
  * allocated with the handle (no call allocates, so calls can be captured
- * into a HIP graph).  A vector of 4- or 8-bit weights, or of any batch, with
- * an element that is not finite gives NaN in all of its outputs.  Replaces the raw per-format
- * dispatchers lut_gemv / lut_gemv_binary / int2_gemv / int3_gemv /
+ * into a HIP graph).
+ *
+ * Sums are fp32.  One vector of a 1-3 bit format, and of 4 bits on a lookup plan
+ * that fills its k-slices, adds table entries of x itself.  Batches and the other
+ * 4- and 8-bit vectors hold x (rotated, if it is) to 2^-31 of a power of two at or
+ * above the largest of its 128 columns, in batches of many vectors of the whole
+ * vector: an absolute error, below what fp32 sums of typical elements round off.
+ * Columns among which more than a quarter of the groups {k, k + 8, k + 16, k + 24}
+ * lie below 2^-8 of that power are multiplied in fp32 as they are instead (the
+ * calls are then up to 3 times slower, 4 where every vector of a large batch is
+ * so).  In these calls a vector with an element that is not finite gives NaN in
+ * all of its outputs.
+ *
+ * Replaces the raw per-format dispatchers lut_gemv / lut_gemv_binary / int2_gemv / int3_gemv /
  * int4_gemv / int8_gemv (lut_gemm.hpp:172-408). */
 int lmx_gemv(const lmx_weight *w, const float *x, float *y, size_t batch,
              unsigned flags, void *stream);
@@ -190,8 +203,9 @@ int lmx_extract_indices(const uint8_t *sign_plane, const uint8_t *zero_plane,
  * until the process ends: a fixed 64 KiB of split-K ticket counters (one per
  * 64-row block), then the staging copy of x (Kp*4 B), then the split-K
  * partials ((Kp/kslice)*Npad*4 B) or the digits of up to 4 vectors; shapes
- * whose staging and partials need more return LMX_ERR_INVALID_ARGUMENT.  The first call on a device looks the array up,
- * zeroes it with a kernel on `stream` and waits for that kernel before it
+ * whose staging and partials need more return LMX_ERR_INVALID_ARGUMENT.  4- and
+ * 8-bit codes are read from the tiles, there being no copy of them.  The first call
+ * on a device looks the array up, zeroes it with a kernel on `stream` and waits for that kernel before it
  * returns or launches anything else, so make it outside graph capture; every
  * later call, on any stream or thread, then finds the counters zeroed.  Calls
  * on one GPU share the array: calls that overlap in time on one GPU race, so
