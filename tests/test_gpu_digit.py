@@ -268,3 +268,20 @@ def test_digit_far_channel(cuda, fmt, spike, rows, cols, batch):
     fp32 = np.linalg.norm(y - x.astype(np.float64) @ W.T) / np.linalg.norm(x.astype(np.float64) @ W.T)
     assert fp32 < 3e-7, fp32
     w.close()
+
+
+# Activations below the smallest power the fixed point can be relative to (2^-97)
+# are multiplied in fp32: all of them (2^-112), or those of one chunk.
+@pytest.mark.parametrize("rows,cols,batch", [(96, 512, 1), (96, 512, 3), (96, 512, 6), (16380, 512, 70)])
+def test_digit_tiny(cuda, rows, cols, batch):
+    planes, scales, g, w = make(L.FMT_INT4, rows, cols, seed=5)
+    x = (vectors(batch, cols, seed=9) * np.float32(2.0 ** -112)).astype(np.float32)
+    y = w.gemv(torch.from_numpy(x).cuda()).cpu().numpy().reshape(batch, rows)
+    ref = x.astype(np.float64) @ synth.dequant_f64(L.FMT_INT4, planes, scales, rows, cols, g).T
+    # sums of `cols` terms, and 2^-149 for each product and sum that may be subnormal
+    mag = np.abs(x).astype(np.float64) @ np.abs(synth.dequant_f64(L.FMT_INT4, planes, scales, rows, cols, g)).T
+    assert (np.abs(y - ref) <= (cols // 128 + 52) * EPS * mag + 2 * cols * 2.0 ** -149).all()
+    x[:, 128:256] = vectors(batch, cols, seed=10)[:, :128]
+    y = w.gemv(torch.from_numpy(x).cuda()).cpu().numpy().reshape(batch, rows)
+    check(L.FMT_INT4, planes, scales, rows, cols, g, x, y, rotate=False)
+    w.close()

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import lutmac_amd as L
+import oracle
 from conftest import rel_max_err
 from lutmac_amd import decode as D
 
@@ -125,3 +126,50 @@ def test_prompt_passes_side_by_side(cuda):
             assert np.array_equal(wt, gt) and np.array_equal(wl.view(np.uint32), gl.view(np.uint32))
     b.close()
     a.close()
+
+
+# Norm weights that put one channel far above the rest, where the linears have
+# code 8 (weight 0): the chunk is multiplied in fp32 by the kernels that norm as
+# they split, one launch (1 and 3 sequences, the SiLU pair too), split vectors (6)
+# and a pass in the tile form (300 positions of gate|up's 1024 rows).
+def far_model(max_seq):
+    cfg = D.small_config(n_layers=3, max_seq=max_seq, vocab=515)
+    model = D.SyntheticModel(cfg, seed=8, group=128, random_norms=True)
+
+    def zero(entry, k):
+        planes = entry[0]
+        bit = 1 << (7 - k % 8)
+        planes[:3, :, k // 8] &= 255 - bit
+        planes[3, :, k // 8] |= bit
+
+    for layer in model.layers:
+        for norm, w, k in (("in_norm", "qkv", 5), ("post_norm", "gate_up", 200)):
+            layer[norm][k] = 1e6
+            zero(layer[w], k)
+    model.final_norm[77] = 1e6
+    zero(model.head, 77)
+    return model
+
+
+@pytest.mark.parametrize("batch", [1, 3, 6])
+def test_far_norm_channel_steps(cuda, batch):
+    model = far_model(16)
+    vocab = model.cfg.vocab
+    toks = np.random.default_rng(batch).integers(0, vocab, (batch, 8)).astype(np.int32)
+    dec = D.Decoder(model, batch=batch)
+    dec.reset(toks if batch > 1 else toks[0])
+    refs = [oracle.OracleDecoder(model) for _ in range(batch)]
+    lg = torch.empty(batch * vocab, device="cuda")
+    for pos in range(8):
+        dec.step(lg)
+        got = lg.cpu().numpy().reshape(batch, vocab)
+        for b in range(batch):
+            assert rel_max_err(got[b], refs[b].step(toks[b, pos], pos)) < DECODE_TOL, (pos, b)
+    dec.close()
+
+
+def test_far_norm_channel_pass(cuda):
+    model = far_model(304)
+    prompt = np.random.default_rng(5).integers(0, model.cfg.vocab, (1, 300)).astype(np.int32)
+    passes, steps = both(model, 1, prompt)
+    assert rel_max_err(passes[0], steps[0]) < DECODE_TOL
