@@ -162,7 +162,7 @@ int lmx_weight_read_tiles(const lmx_weight *w, uint8_t *tiles, size_t bytes);
  * 4- and 8-bit vectors hold x (rotated, if it is) to 2^-31 of a power of two at or
  * above the largest of its 128 columns, in batches of many vectors of the whole
  * vector: an absolute error, below what fp32 sums of typical elements round off.
- * Columns among which more than a quarter of the groups {k, k + 8, k + 16, k + 24}
+ * Columns among which more than half of the groups {k, k + 8, k + 16, k + 24}
  * lie below 2^-8 of that power are multiplied in fp32 as they are instead (the
  * calls are then up to 3 times slower, 4 where every vector of a large batch is
  * so).  In these calls a vector with an element that is not finite gives NaN in

@@ -31,7 +31,7 @@ __device__ __forceinline__ void store_digits(const DigitVectors &d, size_t qc, i
 // Digits of many vectors, one workgroup per vector (tile form):
 // dig[quad][chunk][step][lane][16 B].  Relative to the vector's largest, which
 // saves the products a multiplier per chunk, unless its values lie too far apart
-// (wide_chunks); then (d.exp kFarVector) relative to each chunk's.  Bound by the
+// (far_chunks); then (d.exp kFarVector) relative to each chunk's.  Bound by the
 // latency of the row's read and its maximum; up to K = 8192 the row stays in
 // registers between the passes (512 vectors of 2048: 4.4 us, once a call, where
 // every row block of the products would make them again).
@@ -96,11 +96,11 @@ __global__ __launch_bounds__(512) void digit_split_kernel(const float *__restric
   bool far = false;
 #pragma unroll
   for (int j = 0; j < KEEP; ++j)
-    if (wave + j * NW < pairs) far |= wide_chunks(lane_max_bits(keep[j]), ev) != 0;
+    if (wave + j * NW < pairs) far |= far_chunks(lane_max_bits(keep[j]), ev);
   for (int c2 = wave + KEEP * NW; c2 < pairs; c2 += NW) {
     float o[4];
     values(c2, o);
-    far |= wide_chunks(lane_max_bits(o), ev) != 0;
+    far |= far_chunks(lane_max_bits(o), ev);
   }
   if (lane == 0) wd[wave] = far;
   __syncthreads();

@@ -312,25 +312,37 @@ __device__ __forceinline__ uint32_t chunk_max_bits(uint32_t lane_max) {
   return max(uint32_t(r[0]), uint32_t(r[1]));
 }
 
-// Which of a wave's two 128-chunks are wide (bits 0 and 1): more than a quarter
-// of the lanes with a nonzero value have their largest of four below 2^-8 of the
-// power of two that the fixed point is relative to (exponent e).  Rounding leaves
-// each value off by about 2^-32 of that power; up to there (70 % of Gaussian
-// values below it) that is at most 2^-23.7 of a typical value, what fp32 sums of
-// the values round off too (1.0e-7 to 1.3e-7 of an output), even for a row
-// without weight for the largest.  Wave-uniform, as is maybe_wide: whether one may be, `zeros` of
-// the lanes being known to be zero, without a branch.
+// Which of a wave's two 128-chunks are wide (bits 0 and 1): more than half of the
+// lanes with a nonzero value have their largest of four below 2^-8 of the power
+// of two that the fixed point is relative to (exponent e).  Rounding leaves each
+// value off by about 2^-32 of that power; up to there (84 % of Gaussian values
+// below it) that is at most 2^-23.5 of a typical value, what fp32 sums of the
+// values round off too (1.0e-7 to 1.3e-7 of an output), even for a row without
+// weight for the largest.  Wave-uniform, as is maybe_wide: whether one
+// may be, the last `zeros` lanes being known to be zero, without a branch.
 __device__ __forceinline__ uint64_t small_lanes(uint32_t lane_max, int e) {
   return __builtin_amdgcn_ballot_w64(lane_max < uint32_t(e - 7) << 23);
 }
 __device__ __forceinline__ bool maybe_wide(uint32_t lane_max, int e, int zeros) {
-  return __builtin_popcountll(small_lanes(lane_max, e)) - zeros > (zeros ? 0 : 8);
+  const int lanes = kWave - zeros;   // in the chunk that has fewer of them
+  return 2 * (__builtin_popcountll(small_lanes(lane_max, e)) - zeros) > (lanes > 32 ? lanes - 32 : lanes);
 }
 __device__ __forceinline__ unsigned wide_chunks(uint32_t lane_max, int e) {
   const uint64_t nonzero = __builtin_amdgcn_ballot_w64(lane_max != 0), small = small_lanes(lane_max, e) & nonzero;
-  const bool lo = 4 * __builtin_popcount(uint32_t(small)) > __builtin_popcount(uint32_t(nonzero));
-  const bool hi = 4 * __builtin_popcount(uint32_t(small >> 32)) > __builtin_popcount(uint32_t(nonzero >> 32));
+  const bool lo = 2 * __builtin_popcount(uint32_t(small)) > __builtin_popcount(uint32_t(nonzero));
+  const bool hi = 2 * __builtin_popcount(uint32_t(small >> 32)) > __builtin_popcount(uint32_t(nonzero >> 32));
   return unsigned(lo) | unsigned(hi) << 1;
+}
+
+// Whether one of the two is wide at the exponent of the whole vector, where a
+// chunk with few values may have them all far below a largest that lies elsewhere
+// and is no outlier: more than 16 of its lanes, or all that are not zero, or wide
+// by itself.
+__device__ __forceinline__ bool far_chunks(uint32_t lane_max, int e) {
+  const uint64_t nonzero = __builtin_amdgcn_ballot_w64(lane_max != 0), small = small_lanes(lane_max, e) & nonzero;
+  const uint32_t z0 = uint32_t(nonzero), z1 = uint32_t(nonzero >> 32), s0 = uint32_t(small), s1 = uint32_t(small >> 32);
+  if (__builtin_popcount(s0) > 16 || __builtin_popcount(s1) > 16 || (z0 && s0 == z0) || (z1 && s1 == z1)) return true;
+  return nonzero != ~uint64_t(0) && wide_chunks(lane_max, split_exponent(chunk_max_bits(lane_max)));
 }
 
 // The multiplier of a chunk's digits.

@@ -285,3 +285,24 @@ def test_digit_tiny(cuda, rows, cols, batch):
     y = w.gemv(torch.from_numpy(x).cuda()).cpu().numpy().reshape(batch, rows)
     check(L.FMT_INT4, planes, scales, rows, cols, g, x, y, rotate=False)
     w.close()
+
+
+# A last chunk of few columns: 8 beside outliers elsewhere, which make no vector
+# far, and 8 of which one is far above the others.
+@pytest.mark.parametrize("rows,cols,batch", [(70, 1032, 1), (70, 1032, 3), (70, 1032, 9), (16380, 520, 70), (16380, 8, 70),
+                                             (70, 8, 2), (70, 8, 1), (70, 8, 7)])
+def test_digit_short_last_chunk(cuda, rows, cols, batch):
+    planes, scales, g = synth.make_weights(L.FMT_INT4, rows, cols, seed=6, group=128)
+    zero_columns(L.FMT_INT4, planes, [cols - 3])
+    w = L.Weight.from_planes(L.FMT_INT4, planes, scales, rows, cols, g)
+    W = synth.dequant_f64(L.FMT_INT4, planes, scales, rows, cols, g)
+    x = vectors(batch, cols, seed=11)
+    y = w.gemv(torch.from_numpy(x).cuda()).cpu().numpy().reshape(batch, rows)
+    check(L.FMT_INT4, planes, scales, rows, cols, g, x, y, rotate=False)
+    x[:, cols - 3] = 1e10
+    y = w.gemv(torch.from_numpy(x).cuda()).cpu().numpy().reshape(batch, rows)
+    rest = np.abs(np.delete(x, cols - 3, axis=1)).max()
+    mag = np.abs(x).astype(np.float64) @ np.abs(W).T
+    bound = (cols // 128 + 53) * EPS * mag + 2.0 ** -31 * 2.0 ** 8 * rest * np.abs(W).sum(axis=1)
+    assert (np.abs(y - x.astype(np.float64) @ W.T) <= bound).all()
+    w.close()
