@@ -269,17 +269,17 @@ __device__ __forceinline__ v4i chunk_product(const uint32_t (&wb)[8], const v4i 
 // float 4 (t % 4) + B of step t / 4.  Seldom run: it takes as few registers as it
 // can, so that the kernels keep the waves they have without it.
 __device__ __forceinline__ float raw_sum(const uint32_t (&wb)[8], const char *lo, const char *hi) {
-  float s = 0.0f;
+  float s0 = 0.0f, s1 = 0.0f;   // two sums of 16: half the rounding of one of 32
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
     const float4 x = *reinterpret_cast<const float4 *>((t < 4 ? lo : hi) + (t & 3) * 16);
-    s = fmaf(float(int(wb[t] << 24) >> 24), x.x, s);
-    s = fmaf(float(int(wb[t] << 16) >> 24), x.y, s);
-    s = fmaf(float(int(wb[t] << 8) >> 24), x.z, s);
-    s = fmaf(float(int(wb[t]) >> 24), x.w, s);
+    s0 = fmaf(float(int(wb[t] << 24) >> 24), x.x, s0);
+    s1 = fmaf(float(int(wb[t] << 16) >> 24), x.y, s1);
+    s0 = fmaf(float(int(wb[t] << 8) >> 24), x.z, s0);
+    s1 = fmaf(float(int(wb[t]) >> 24), x.w, s1);
     __builtin_amdgcn_sched_barrier(0);
   }
-  return s;
+  return s0 + s1;
 }
 
 // Lane roles while digits are made, a 256-chunk per wave: lane = chunk c (1
