@@ -284,28 +284,16 @@ int stage_if_needed(const lmx_weight *w, GemvArgs &a, void *stream) {
 
 }  // namespace
 
-// Whether one vector of this weight runs on the digit kernels.  8 bits always.
-// 4 bits unless its lookup-table plan has small workgroups and a chunk for
-// three in four of their k-slices: that plan's tables and lookups then take one
-// step per wave, and little of the launch goes by before its planes arrive (us,
-// tables / digits: 256 x 2048 2.78 / 2.99, 2048 x 1536 3.03 / 3.21, 3072 x 1792
-// 3.37 / 3.49, 2048 x 8192 4.76 / 5.14, 256 x 6144 3.81 / 3.98; 2048 x 1024 2.98
-// / 2.93, 4096 x 2048 3.57 / 3.52, 2048 x 4096 4.29 / 3.92, 2048 x 8960 6.50 /
-// 6.02).  The same rule without a handle, so both give the same bits.
-static bool one_vector_on_digits(const lmx_weight *w) {
-  if (!w->digit || !code_copy_bytes(w->format, 1, kRotChunk)) return false;
-  if (w->format != LMX_FMT_INT4) return true;
-  const size_t chunks = w->Kp / kChunk;
-  if (w->fullk == kFullK_4x4x1) return chunks < 12 || w->Npad > 3072;
-  return w->fullk != kFullK_16x4x1 || chunks < 48;
-}
-
 // y = W x of `batch` vectors on the digit kernels: up to 4 in one launch,
 // more through digits split into the handle's scratch.  One vector of a 1-3
 // bit format stays on the lookup tables, whose planes are half to an eighth of
 // the bytes while the digits cost the same (8192 x 8192, us: ternary 6.5
 // against 8.2, RRQ-2 7.1 / 9.5, binary 5.3 / 7.1; 4-bit 9.7 / 8.0, 8-bit
-// 17.9 / 15.7).  *done = the vectors covered; `all`: every one, the single
+// 17.9 / 15.7).  4-bit vectors take the digits also where the tables, on a plan
+// with a chunk for every k-slice, end a launch 4 to 9 % sooner (graph replays, us,
+// tables / digits: 512 x 2048 2.78 / 2.99, 2048 x 1536 3.03 / 3.21, 2048 x 8192
+// 4.76 / 5.14; by eager launches both take the host's 5): their outputs are off
+// by half as much (6e-8 of the result against 1.2e-7).  *done = the vectors covered; `all`: every one, the single
 // vectors of those formats too (a.xmode and a.epi have no other form there).
 int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size_t batch, void *stream, size_t *done,
                  bool all, void *scratch, size_t scratch_bytes) {
@@ -338,7 +326,7 @@ int digit_linear(const lmx_weight *w, GemvArgs a, const float *x, float *y, size
         return st;
     } else {
       // one by one on the lookup tables
-      if (!all && (left == 1 ? !one_vector_on_digits(w) : !copies && w->Kp > 4096)) return LMX_OK;
+      if (!all && (left == 1 ? !copies || !w->digit : !copies && w->Kp > 4096)) return LMX_OK;
       if ((st = launch_digit_gemv(w->format, a, int(n), stream))) return st;
     }
     *done += n;

@@ -168,23 +168,6 @@ def test_digit_graph(cuda, rows, cols, batch):
     w.close()
 
 
-# One 4-bit vector of a lookup plan whose small workgroups have a chunk for three
-# in four k-slices runs that plan, one of any other the digit kernels: the bits
-# of a handle made for the lookup tables, and not.
-@pytest.mark.parametrize("rows,cols,tables", [(2048, 1536, True), (3072, 2048, True), (70, 6144, True),
-                                              (2048, 1280, False), (3136, 2048, False), (70, 5888, False)])
-def test_one_vector_route(cuda, monkeypatch, rows, cols, tables):
-    planes, scales, g, w = make(L.FMT_INT4, rows, cols, seed=rows + cols)
-    monkeypatch.setenv("LMX_DIGIT", "0")
-    lut = L.Weight.from_planes(L.FMT_INT4, planes, scales, rows, cols, g)
-    x = torch.from_numpy(vectors(1, cols, seed=1)).cuda()
-    a, b = w.gemv(x), lut.gemv(x)
-    assert torch.equal(a, b) == tables
-    check(L.FMT_INT4, planes, scales, rows, cols, g, x.cpu().numpy(), a.cpu().numpy()[None], rotate=False)
-    w.close()
-    lut.close()
-
-
 # The digits' products with codes read from the planes (no handle, so no code
 # copy; 8 bits: one vector of a handle too): the handle's bits, for one and two
 # row tiles, one and more 256-chunks per wave, the last of them alone.
