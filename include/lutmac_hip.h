@@ -157,19 +157,19 @@ int lmx_weight_read_tiles(const lmx_weight *w, uint8_t *tiles, size_t bytes);
  * allocated with the handle (no call allocates, so calls can be captured
  * into a HIP graph).
  *
- * Sums are fp32.  One vector of a 1-3 bit format, and of 4 bits on a lookup plan
- * that fills its k-slices, adds table entries of x itself.  Batches and the other
- * 4- and 8-bit vectors hold x (rotated, if it is) to 2^-31 of a power of two at or
- * above the largest of its 128 columns, in batches of many vectors of the whole
- * vector: an absolute error, below what fp32 sums of typical elements round off.
+ * Sums are fp32.  One vector of a 1-3 bit format adds table entries of x itself.
+ * Batches and 4- and 8-bit vectors hold x (rotated, if it is) to 2^-31 of a power
+ * of two at or above the largest of its 128 columns, in batches of many vectors
+ * of the whole vector: an absolute error, below what fp32 sums of typical
+ * elements round off.
  * Columns among which more than half of the groups {k, k + 8, k + 16, k + 24}
  * lie below 2^-8 of that power are multiplied in fp32 as they are instead (the
  * calls are then up to 3 times slower, 4 where every vector of a large batch is
  * so).  In these calls a vector with an element that is not finite gives NaN in
  * all of its outputs.
  *
- * Replaces the raw per-format dispatchers lut_gemv / lut_gemv_binary / int2_gemv / int3_gemv /
- * int4_gemv / int8_gemv (lut_gemm.hpp:172-408). */
+ * Replaces the raw per-format dispatchers lut_gemv / lut_gemv_binary /
+ * int2_gemv / int3_gemv / int4_gemv / int8_gemv (lut_gemm.hpp:172-408). */
 int lmx_gemv(const lmx_weight *w, const float *x, float *y, size_t batch,
              unsigned flags, void *stream);
 /* lut_linear (lut_gemm.hpp:419-420, lut_gemm_scalar.cpp:68-180): rotation
